@@ -194,6 +194,31 @@ __device__ double d_eta_scale(const CkParams &prm, int model, double l_turb, dou
     return prm.eta_dpp_cap / eta;
 }
 
+// The state-independent part of d_eta_scale: the turbulent energy q t (erg)
+// that the CR energy is compared with, 0 where the scale is 1 whatever the
+// state; the scale is then d_eta_scale_qt.
+__device__ double d_eta_qt(const CkParams &prm, int model, double l_turb, double dv, double cs, double beta,
+                           double mass, double t_acc_direct)
+{
+#pragma clang fp contract(off)
+    if (!(prm.eta_dpp_cap > 0.0) || !isfinite(prm.eta_dpp_cap)) return 0.0;
+    if (!(mass > 0.0) || !(l_turb > 0.0) || !(dv > 0.0)) return 0.0;
+    const double t = d_tacc_for_cap(prm, model, l_turb, dv, cs, beta, t_acc_direct);
+    if (!(t > 0.0) || !isfinite(t)) return 0.0;
+    const double q = 0.5 * mass * K_MSUN * dv * dv * dv / (l_turb * K_MPC);
+    if (!(q > 0.0) || !isfinite(q)) return 0.0;
+    return q * t * K_GYR;
+}
+
+__device__ __forceinline__ double d_eta_scale_qt(double cap, double qt, double ecr)
+{
+#pragma clang fp contract(off)
+    if (!(qt > 0.0) || !(ecr > 0.0) || !isfinite(ecr)) return 1.0;
+    const double eta = ecr / qt;
+    if (!(eta > cap) || !isfinite(eta)) return 1.0;
+    return cap / eta;
+}
+
 // Chang-Cooper face weights W+ = B(-w), W- = B(w) (Chang_Cooper.c:22-40).
 // For |w| >= 0.1 the reference's two exponentials reduce exactly to one:
 // one argument is exactly 0 and the other exactly -|w|.
@@ -290,19 +315,17 @@ __device__ __forceinline__ void d_cc_row(int kind, double dt, double x, double d
     }
 }
 
-// tracer_fp_choose_coeff_interp_segments (tracer_fp_setup.c:73-95)
+// tracer_fp_choose_coeff_interp_segments (tracer_fp_setup.c:73-95): 1, doubled
+// while twice as many stays within max_seg and nsub / min_steps, so the
+// largest power of two (up to 2^30) within both; at most nsub since
+// min_steps >= 1.
 __device__ __host__ __forceinline__ int d_choose_segments(int nsub, int allow, int min_steps, int max_seg)
 {
-    int segments = 1;
     if (!allow || nsub <= 1) return 1;
     if (min_steps <= 0) return 1;
-    if (max_seg < 1) max_seg = 1;
-    const int max_allowed = nsub / min_steps;
-    if (max_allowed < 1) return 1;
-    while (segments <= 1073741823 && segments * 2 <= max_seg && segments * 2 <= max_allowed) segments *= 2;
-    if (segments > nsub) segments = nsub;
-    if (segments < 1) segments = 1;
-    return segments;
+    const int most = nsub / min_steps < max_seg ? nsub / min_steps : max_seg;
+    if (most < 2) return 1;
+    return 1 << (31 - __builtin_clz((unsigned)most));
 }
 
 // ---------------------------------------------------------------------------
@@ -426,6 +449,14 @@ __device__ __forceinline__ double d_lerp(double cur, double nxt, double alpha)
 // source lies outside its group reads a neighbouring group's (finite) value,
 // or 0, and every caller discards it or multiplies it by a zero coefficient.
 // ---------------------------------------------------------------------------
+// LDS written by lanes of the wave before it is read by others of the wave
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 template <int CTRL>
 __device__ __forceinline__ double dpp64(double v)
 {
@@ -580,8 +611,8 @@ __device__ __forceinline__ double d_div_normal(double a, double b)
 __device__ __forceinline__ void pm_mul(double &m00, double &m01, double &m10, double &m11, double o00, double o01,
                                        double o10, double o11)
 {
-    const double n00 = m00 * o00 + m01 * o10, n01 = m00 * o01 + m01 * o11;
-    const double n10 = m10 * o00 + m11 * o10, n11 = m10 * o01 + m11 * o11;
+    const double n00 = fma(m00, o00, m01 * o10), n01 = fma(m00, o01, m01 * o11);
+    const double n10 = fma(m10, o00, m11 * o10), n11 = fma(m10, o01, m11 * o11);
     m00 = n00; m01 = n01; m10 = n10; m11 = n11;
 }
 __device__ __forceinline__ void pm_renorm(double &m00, double &m01, double &m10, double &m11)
@@ -592,20 +623,29 @@ __device__ __forceinline__ void pm_renorm(double &m00, double &m01, double &m10,
         m00 = ldexp(m00, -e); m01 = ldexp(m01, -e); m10 = ldexp(m10, -e); m11 = ldexp(m11, -e);
     }
 }
+// (second column of m) <- m o (column o)
+__device__ __forceinline__ void pm_apply(double m00, double &m01, double m10, double &m11, double o01, double o11)
+{
+    const double n01 = fma(m00, o01, m01 * o11), n11 = fma(m10, o01, m11 * o11);
+    m01 = n01;
+    m11 = n11;
+}
 // In-row Hillis-Steele levels of the pivot-map scan (shift 1, 2, 4, 8 by DPP;
 // a source lane outside the row, or outside a group narrower than a row,
-// contributes nothing).
+// contributes nothing).  The last level of a group within one row forms only
+// the second column.
 template <int G, int ST>
 __device__ __forceinline__ void pm_row_scan(int gl, int rl, double &m00, double &m01, double &m10, double &m11)
 {
     constexpr int LV = LogG<G>::v < 4 ? LogG<G>::v : 4;
     if constexpr (ST < LV) {
         constexpr int s = 1 << ST;
-        const double o00 = row_up<s>(m00), o01 = row_up<s>(m01);
-        const double o10 = row_up<s>(m10), o11 = row_up<s>(m11);
-        if ((G >= 16) ? (rl >= s) : (gl >= s)) {
-            pm_mul(m00, m01, m10, m11, o00, o01, o10, o11);
-            pm_renorm(m00, m01, m10, m11);
+        const double o01 = row_up<s>(m01), o11 = row_up<s>(m11);
+        if constexpr (G <= 16 && ST == LV - 1) {
+            if ((G >= 16) ? (rl >= s) : (gl >= s)) pm_apply(m00, m01, m10, m11, o01, o11);
+        } else {
+            const double o00 = row_up<s>(m00), o10 = row_up<s>(m10);
+            if ((G >= 16) ? (rl >= s) : (gl >= s)) pm_mul(m00, m01, m10, m11, o00, o01, o10, o11);
         }
         pm_row_scan<G, ST + 1>(gl, rl, m00, m01, m10, m11);
     }
@@ -615,69 +655,83 @@ __device__ __forceinline__ void pm_row_scan(int gl, int rl, double &m00, double 
 // fp_thomas_solve_ws (fp_shared_core.c:226-257): denom_i = b_i + a_i cprime_{i-1},
 // cprime_i = -c_i / denom_i, pivot guard |denom| <= 1e-300.  The pivot
 // entering each lane comes from a scan of 2x2 projective maps across the
-// group's lanes (renormalised by powers of two, so exact up to rounding of
-// the products); inside the lane the reference recurrence is applied.
+// group's lanes, exact up to rounding of the products; inside the lane the
+// reference recurrence is applied.
+//
+// Row k maps (u, v), cprime = u / v, to (-c_k v, a_k u + b_k v); both columns
+// of the product over the lane's rows therefore follow the three-term
+// recurrence v_k = b_k v_{k-1} - a_k c_{k-1} v_{k-2} (5 operations a row for
+// both), and the product's first row is -c_{R-1} times the recurrence one row
+// back.  The entries are renormalised by a power of two every eight rows
+// (rows' coefficient sums up to 1e38 stay in range) and after the lane's last
+// row; the up to six products across lanes then stay within 2^63 of the
+// renormalised entries and shrink by at most a few powers of R per lane, so
+// they need no further scaling.
 template <int R, int G, bool NOSRC = false>
-__device__ __forceinline__ void factorize(int gl, int n, const double (&sv)[R], Factor<R, G> &F, int &bad)
+__device__ __forceinline__ void factorize(int gl, const double (&sv)[R], Factor<R, G> &F, int &bad)
 {
-    double m00 = 1.0, m01 = 0.0, m10 = 0.0, m11 = 1.0;
+    double m00, m01, m10, m11;
+    {
+        // (p, q): the recurrence at the row before and at this row, of the
+        // columns that start from (u, v) = (1, 0) and (0, 1)
+        double p0 = 0.0, q0 = F.al[0], p1 = 1.0, q1 = F.iv[0];
 #pragma unroll
-    for (int k = 0; k < R; ++k) {
-        const double a = F.al[k], b = F.iv[k], c = F.g[k];
-        const double n00 = -c * m10, n01 = -c * m11;
-        const double n10 = a * m00 + b * m10, n11 = a * m01 + b * m11;
-        m00 = n00; m01 = n01; m10 = n10; m11 = n11;
-        // renormalised every second row: two rows grow the entries by at most
-        // the product of two rows' coefficient sums, far inside the range
-        if ((k & 1) || k == R - 1) pm_renorm(m00, m01, m10, m11);
+        for (int k = 1; k < R; ++k) {
+            const double ac = F.al[k] * F.g[k - 1], b = F.iv[k];
+            const double n0 = fma(b, q0, -(ac * p0)), n1 = fma(b, q1, -(ac * p1));
+            p0 = q0;
+            p1 = q1;
+            q0 = n0;
+            q1 = n1;
+            if ((k & 7) == 7 && k < R - 1) pm_renorm(p0, p1, q0, q1);
+        }
+        const double c = F.g[R - 1];
+        m00 = (R > 1 ? -c * p0 : 0.0);
+        m01 = -c * p1;
+        m10 = q0;
+        m11 = q1;
+        pm_renorm(m00, m01, m10, m11);
     }
     // inclusive prefix over the group's lanes, P_l = M_l ... M_0: Hillis-Steele
     // levels inside 16-lane rows (DPP), then the rows of a wider group take the
-    // full prefix at the last lane of the row before (readlane)
+    // full prefix at the last lane of the row before.  Only the second column
+    // (the image of cprime = 0) is needed in the end.
     const int rl = (int)(threadIdx.x & 15);
     pm_row_scan<G, 0>(gl, rl, m00, m01, m10, m11);
-    if constexpr (G > 16) {
+    if constexpr (G == 32) {
+        // rows (0, 1) and (2, 3) form groups: odd rows continue lane 15 / 47
+        const double c01 = bcast15(m01), c11 = bcast15(m11);
+        if (threadIdx.x & 16) pm_apply(m00, m01, m10, m11, c01, c11);
+    } else if constexpr (G == 64) {
+        // one group per wave: carries through rows 0, 1, 2
         const int row = (int)((threadIdx.x & 63) >> 4);
-        double c00, c01, c10, c11;  // full prefix entering this lane's row
-        if constexpr (G == 32) {
-            // rows (0, 1) and (2, 3) form groups: odd rows take lane 15 / 47
-            const double a00 = rdlane64(m00, 15), a01 = rdlane64(m01, 15);
-            const double a10 = rdlane64(m10, 15), a11 = rdlane64(m11, 15);
-            const double b00 = rdlane64(m00, 47), b01 = rdlane64(m01, 47);
-            const double b10 = rdlane64(m10, 47), b11 = rdlane64(m11, 47);
-            const bool hi = row >= 2;
-            c00 = hi ? b00 : a00; c01 = hi ? b01 : a01; c10 = hi ? b10 : a10; c11 = hi ? b11 : a11;
-        } else {
-            // one group per wave: carries through rows 0, 1, 2
-            double f00 = rdlane64(m00, 15), f01 = rdlane64(m01, 15);
-            double f10 = rdlane64(m10, 15), f11 = rdlane64(m11, 15);  // full prefix at lane 15
-            c00 = f00; c01 = f01; c10 = f10; c11 = f11;
+        double f01 = rdlane64(m01, 15), f11 = rdlane64(m11, 15);
+        double c01 = f01, c11 = f11;
 #pragma unroll
-            for (int r = 1; r < 3; ++r) {
-                double u00 = rdlane64(m00, 16 * r + 15), u01 = rdlane64(m01, 16 * r + 15);
-                double u10 = rdlane64(m10, 16 * r + 15), u11 = rdlane64(m11, 16 * r + 15);
-                pm_mul(u00, u01, u10, u11, f00, f01, f10, f11);
-                pm_renorm(u00, u01, u10, u11);
-                f00 = u00; f01 = u01; f10 = u10; f11 = u11;
-                if (row == r + 1) { c00 = f00; c01 = f01; c10 = f10; c11 = f11; }
+        for (int r = 1; r < 3; ++r) {
+            const double u00 = rdlane64(m00, 16 * r + 15), u10 = rdlane64(m10, 16 * r + 15);
+            double u01 = rdlane64(m01, 16 * r + 15), u11 = rdlane64(m11, 16 * r + 15);
+            pm_apply(u00, u01, u10, u11, f01, f11);
+            f01 = u01;
+            f11 = u11;
+            if (row == r + 1) {
+                c01 = f01;
+                c11 = f11;
             }
         }
-        if (row & (G / 16 - 1)) {
-            pm_mul(m00, m01, m10, m11, c00, c01, c10, c11);
-            pm_renorm(m00, m01, m10, m11);
-        }
+        if (row) pm_apply(m00, m01, m10, m11, c01, c11);
     }
     const double uin = wave_up1(m01), vin = wave_up1(m11);
-    double cprev = (gl == 0) ? 0.0 : uin / vin;
-    const int base = gl * R;
+    double cprev = (gl == 0) ? 0.0 : d_div_normal(uin, vin);
+    bool ok = true;
     double A = 1.0, Bq = 1.0;
 #pragma unroll
     for (int k = 0; k < R; ++k) {
         const double a = F.al[k], b = F.iv[k], c = F.g[k];
-        const double den = b + a * cprev;
-        if (!(fabs(den) > 1.0e-300)) bad |= ERR_PIVOT;
+        const double den = fma(a, cprev, b);
+        ok = ok && fabs(den) > 1.0e-300;
         const double inv = d_div_normal(1.0, den);
-        const double cp = (base + k == n - 1) ? 0.0 : -c * inv;
+        const double cp = -c * inv;  // the system's last row has c = 0
         F.iv[k] = inv;
         // the group's first row has no predecessor: its multiplier is 0, so
         // the value a substep shifts in from the lane before (another
@@ -689,6 +743,7 @@ __device__ __forceinline__ void factorize(int gl, int n, const double (&sv)[R], 
         Bq *= F.g[k];
         cprev = cp;
     }
+    if (!ok) bad |= ERR_PIVOT;
     // Scan multipliers of the substep solve.  Hillis-Steele levels run
     // inside 16-lane rows (DPP); a group spanning several rows completes the
     // scan with per-row carries (see apply_solve).
@@ -868,14 +923,18 @@ __device__ __forceinline__ SpGridT<T> sp_grid(const CkGrid &g, bool elec, const 
 }
 
 // Face between rows j and j+1 (cc_prepare_face_weight + cc_eval_face_weights,
-// Chang_Cooper.c:22-66): w = (B/C)_face * h, W+ = B(-w), W- = B(w); both zero
-// when |C_j| <= 1e-200.  Fh = C_face / h.  The Bernoulli pair is formed from
-// one exponential h2 = exp(-|w|/2):
+// Chang_Cooper.c:22-66): w = (B/C)_face * h, W+ = B(-w), W- = B(w), both zero
+// when |C_j| <= 1e-200; Fh = C_face / h, Fp = Fh W+, Fm = Fh W-; bm the mean
+// advection.
+// The Bernoulli pair is formed from one exponential h2 = exp(-|w|/2):
 //   |w| <  0.1: W_big = 1 / (h2 * den), den = 1 + w^2/24 + w^4/1920
 //   |w| >= 0.1: W_big = |w| / (1 - h2^2)
 //   W_small = W_big * h2^2; W+ = W_big for w > 0 (else W_small).
+// The rounding of the rows' couplings sets how well the scheme conserves
+// particle number over thousands of substeps, so the products keep the order
+// of the reference's rows and are not contracted.
 struct Face {
-    double bm, Fh, wp, wm, w;
+    double bm, Fh, wp, wm, Fp, Fm, w;
 };
 
 // FP32 coefficients (T = float): the face averages, diffusion flux factor
@@ -886,27 +945,26 @@ __device__ __forceinline__ Face d_face2(T Bl, T Br, T Cl, T Cr, T h, T inv_h)
 {
 #pragma clang fp contract(off)
     Face f;
-    double wv;
+    double w;
     bool live;
     if constexpr (sizeof(T) == sizeof(double)) {
         f.bm = 0.5 * (Bl + Br);
         const double cm = 0.5 * (Cl + Cr);
         f.Fh = cm * inv_h;
         live = fabs(Cl) > 1.0e-200;
-        wv = live ? d_div_normal(f.bm, cm) * h : 0.0;
+        w = live ? d_div_normal(f.bm, cm) * h : 0.0;
     } else {
         const float bm = 0.5f * (Bl + Br);
         const float cm = 0.5f * (Cl + Cr);
         f.bm = (double)bm;
         f.Fh = (double)(cm * inv_h);
         live = fabs((double)Cl) > 1.0e-200;
-        wv = live ? (double)(bm * __builtin_amdgcn_rcpf(cm) * h) : 0.0;
+        w = live ? (double)(bm * __builtin_amdgcn_rcpf(cm) * h) : 0.0;
     }
     f.wp = 0.0;
     f.wm = 0.0;
-    f.w = 0.0;
+    f.w = w;
     if (live) {
-        const double w = wv;
         const double aw = fabs(w);
         const double h2 = d_exp_nonpos(-0.5 * aw);
         const double E = h2 * h2;
@@ -917,51 +975,32 @@ __device__ __forceinline__ Face d_face2(T Bl, T Br, T Cl, T Cr, T h, T inv_h)
         const double sm = big * E;
         f.wp = (w > 0.0) ? big : sm;
         f.wm = (w > 0.0) ? sm : big;
-        f.w = w;
     }
+    f.Fp = f.Fh * f.wp;
+    f.Fm = f.Fh * f.wm;
     return f;
 }
 
 // Row j of the Chang-Cooper system (fp_shared_core.c:660-704 ->
-// Chang_Cooper.c:68-184), A = 1, from its two faces.  kind: 0 interior, 1 left
-// boundary, 2 right boundary.  Output as positive coupling magnitudes
-// b x_j - a x_{j-1} - c x_{j+1}.
-__device__ __forceinline__ void d_cc_row2(int kind, double t1, double C, double dtT, const Face &fl,
+// Chang_Cooper.c:68-184), A = 1, from its two faces, as positive coupling
+// magnitudes b x_j - a x_{j-1} - c x_{j+1}.  The system's first (last) row has
+// an all-zero left (right) face, which turns the interior form into the
+// boundary form; only the last row without diffusion differs (`last`): its a
+// takes the weight delta of its left face, nonzero when that face carries
+// weights (Cl: the C of the row before).
+__device__ __forceinline__ void d_cc_row2(bool last, double t1, double C, double dtT, const Face &fl,
                                           const Face &fr, double Cl, double &a, double &b, double &c)
 {
 #pragma clang fp contract(off)
-    const bool cz = !(fabs(C) > 1.0e-200);
-    if (kind == 0) {
-        if (!cz) {
-            a = t1 * fl.Fh * fl.wm;
-            b = 1.0 + t1 * (fl.Fh * fl.wp + fr.Fh * fr.wm) + dtT;
-            c = t1 * fr.Fh * fr.wp;
-        } else {
-            a = 0.0;
-            b = 1.0 + t1 * fl.bm + dtT;
-            c = t1 * fr.bm;
-        }
-    } else if (kind == 1) {
-        a = 0.0;
-        if (!cz) {
-            b = 1.0 + t1 * (fr.Fh * fr.wm) + dtT;
-            c = t1 * fr.Fh * fr.wp;
-        } else {
-            b = 1.0 + dtT;
-            c = t1 * fr.bm;
-        }
+    if (fabs(C) > 1.0e-200) {
+        a = t1 * fl.Fh * fl.wm;
+        b = 1.0 + t1 * (fl.Fp + fr.Fm) + dtT;
+        c = t1 * fr.Fh * fr.wp;
     } else {
-        c = 0.0;
-        if (!cz) {
-            a = t1 * fl.Fh * fl.wm;
-            b = 1.0 + t1 * (fl.Fh * fl.wp) + dtT;
-        } else {
-            // delta of the left face (Chang_Cooper.c:143-184): nonzero only
-            // when that face carries weights
-            const double delta = (fabs(Cl) > 1.0e-200) ? d_face_delta(fl.w) : 0.0;
-            a = -delta * fl.bm * t1;
-            b = 1.0 + t1 * fl.bm + dtT;
-        }
+        a = 0.0;
+        if (last && fabs(Cl) > 1.0e-200) a = -d_face_delta(fl.w) * fl.bm * t1;
+        b = 1.0 + t1 * fl.bm + dtT;
+        c = t1 * fr.bm;
     }
 }
 
@@ -971,7 +1010,6 @@ struct RunCoef {
     double dt;
     double dfac;     // inv_on * scale (model) or scale / 4e5 (floor)
     bool model;      // filled form (p^2 inv exp(-E/Epmax) exp(-1/p)) vs floor p^2/4e5
-    double inv_epmax;
     double dtT_fac;  // dt * 0.5 c n_gas Gyr (protons), 0 for electrons
 };
 
@@ -1006,9 +1044,12 @@ __device__ __forceinline__ T wave_up1_t(T v)
 
 // Builds the rows of the lane into F (al = a, iv = b, g = c) and factorises.
 // The rows' coefficients (B, C and the face inputs) are of type T; the
-// face weights, the rows a, b, c and the factorisation are FP64.
+// face weights, the rows a, b, c and the factorisation are FP64.  Each lane
+// evaluates the right faces of its own rows; its first row takes its left
+// face from the lane before, when that lane is done (eight lane moves instead
+// of a face, 1 of R + 1).
 template <bool ELEC, int R, int G, typename T, bool NOSRC = false>
-__device__ __forceinline__ void build_factor(int gl, int n, const SpGridT<T> &sg, const RunCoef &rc,
+__device__ __forceinline__ void build_factor(int gl, const SpGridT<T> &sg, const RunCoef &rc,
                                              const T *radp, const SrcRows &src, Factor<R, G> &F, int &bad)
 {
 #pragma clang fp contract(off)
@@ -1017,80 +1058,140 @@ __device__ __forceinline__ void build_factor(int gl, int n, const SpGridT<T> &sg
     T B0, C0, BL, CL;
     row_BC<ELEC, T>(sg, rc, base, radp[o], B0, C0);
     row_BC<ELEC, T>(sg, rc, base + R - 1, radp[o + R - 1], BL, CL);
-    // neighbour lanes' edge rows (DPP across the wave; a group's edge lanes
-    // read the next group's values and do not use them)
+    // the next lane's first row (DPP across the wave; a group's last lane
+    // reads the next group's values and does not use them)
     const T Bn = wave_dn1_t(B0), Cn = wave_dn1_t(C0);
-    const T Bp = wave_up1_t(BL), Cp = wave_up1_t(CL);
-    Face fl = {0.0, 0.0, 0.0, 0.0, 0.0};
-    if (gl > 0) fl = d_face2<T>(Bp, B0, Cp, C0, sg.h[sg.ix(base - 1)], sg.inv_h[sg.ix(base - 1)]);
-    double Cl = (double)Cp;
+    const bool glast = gl == G - 1;
+    const Face none = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    Face fl = none, f0 = none;
+    double t10 = 0.0, dtT0 = 0.0, Cl = 0.0;
     T Bk = B0, Ck = C0;
 #pragma unroll
     for (int k = 0; k < R; ++k) {
         const int j = base + k;
-        const bool last = (j == n - 1);
         T Br, Cr;
         if (k == R - 1) { Br = Bn; Cr = Cn; }
         else if (k == R - 2) { Br = BL; Cr = CL; }
         else row_BC<ELEC, T>(sg, rc, j + 1, radp[o + k + 1], Br, Cr);
-        Face fr = {0.0, 0.0, 0.0, 0.0, 0.0};
-        if (!last) fr = d_face2<T>(Bk, Br, Ck, Cr, sg.h[sg.ix(j)], sg.inv_h[sg.ix(j)]);
-        const int kind = (j == 0) ? 1 : (last ? 2 : 0);
+        Face fr = none;
+        if (k < R - 1 || !glast) fr = d_face2<T>(Bk, Br, Ck, Cr, sg.h[sg.ix(j)], sg.inv_h[sg.ix(j)]);
         const double t1 = rc.dt * (double)sg.inv_dx[sg.ix(j)];
         double dtT = 0.0;
         if constexpr (!ELEC) dtT = (double)((T)rc.dtT_fac * sg.sig[sg.ix(j)]);
-        double a, b, c;
-        d_cc_row2(kind, t1, (double)Ck, dtT, fl, fr, Cl, a, b, c);
-        F.al[k] = a;
-        F.iv[k] = b;
-        F.g[k] = c;
+        if (k == 0) {
+            f0 = fr;
+            t10 = t1;
+            dtT0 = dtT;
+        } else {
+            d_cc_row2(k == R - 1 && glast, t1, (double)Ck, dtT, fl, fr, Cl, F.al[k], F.iv[k], F.g[k]);
+        }
         fl = fr;
         Cl = (double)Ck;
         Bk = Br;
         Ck = Cr;
     }
+    // fl: the lane's last right face, the left face of the next lane's first row
+    Face fp = none;
+    fp.bm = wave_up1(fl.bm);
+    fp.Fh = wave_up1(fl.Fh);
+    fp.wm = wave_up1(fl.wm);
+    fp.Fp = wave_up1(fl.Fp);
+    if (gl == 0) fp = none;
+    d_cc_row2(false, t10, (double)C0, dtT0, fp, f0, 0.0, F.al[0], F.iv[0], F.g[0]);
     // the run's sources after the rows (absent rows point at the grid's zero
     // row: no branches), so they hold no registers during the row build;
     // their loads overlap the factorisation's pivot scan
     double sv[R];
 #pragma unroll
     for (int k = 0; k < R; ++k) sv[k] = NOSRC ? 0.0 : src.scale * (src.inj[o + k] * src.ka * src.kb + src.q[o + k]);
-    factorize<R, G, NOSRC>(gl, n, sv, F, bad);
+    factorize<R, G, NOSRC>(gl, sv, F, bad);
 }
 
 // ---------------------------------------------------------------------------
 // Fused persistent kernel
 // ---------------------------------------------------------------------------
-struct SegScalars {
-    double n_gas, kbt, bfield, divv, lturb, dv, cs, beta;
-};
+// Per-segment scalars.  Everything a segment needs beyond the tracer's state
+// (interpolated backgrounds, D_pp prefactor, loss-rate coefficients) depends
+// on the segment index only, so the group's lanes evaluate one segment each,
+// SC segments at a time, and leave the values in LDS, slot SV_* of segment
+// (iseg mod SC).  Evaluated by every lane for each segment in turn (with the
+// segment bounds by 64-bit divisions, now shifts) this was about 1,100 of the
+// 2,800 vector instructions outside the substep loop of a segment at n = 256,
+// 8 rows per lane.  With the leaner pivot scan (factorize): 10,000 tracers of
+// both species x 256 bins, ASA, two snapshots, electron pass 1330 -> 1047 us
+// (4.04e8 -> 3.14e8 vector instructions), proton pass 1362 -> 1170 us.
+enum { SV_DFAC, SV_MODEL, SV_QT, SV_ADIA,       // D_pp factor, filled form (1) or floor (0), eta-cap energy, adiabatic rate
+       SV_NGAS,                                  // n_gas
+       SV_SYNCH, SV_COUL, SV_LNING, SV_NE,       // electrons: synchrotron and Coulomb factors, ln(1 / n_gas)
+       SV_KBT = SV_SYNCH, SV_IKBT, SV_NP,        // protons alone: kT, 1 / kT
+       SV_EP_KBT = SV_NE, SV_EP_IKBT, SV_NEP };  // both species: after the electron slots
+__host__ __device__ constexpr int fused_nsv(int MODE) { return MODE == 1 ? SV_NEP : MODE == 2 ? SV_NP : SV_NE; }
+
+template <int MODE>
+__device__ void seg_scalars(const CkSlot &S, const double *s_bg, int iseg, int sh, int nsub, double dt, bool dis,
+                            double mass, double *sv)
+{
+#pragma clang fp contract(off)
+    constexpr bool PROT = (MODE == 1 || MODE == 2);
+    constexpr bool ELEC = (MODE != 2);
+    const CkParams &prm = S.prm;
+    const int fb = (int)(((long long)iseg * nsub) >> sh), fe = (int)(((long long)(iseg + 1) * nsub) >> sh);
+    // alpha is 0 (the current snapshot's value) without interpolation
+    const double alpha = sh ? ldexp((double)iseg + 0.5, -sh) : 0.0;
+    double v[CK_NBG];
+#pragma unroll
+    for (int f = 0; f < CK_NBG; ++f) v[f] = d_lerp(s_bg[f], s_bg[CK_NBG + f], alpha);
+    const double n_gas = v[CK_BG_NGAS], lturb = v[CK_BG_LTURB], dv = v[CK_BG_DV], cs = v[CK_BG_CS];
+    const double beta = v[CK_BG_BETA];
+    double tacc_d = prm.t_acc_direct_gyr;
+    if (prm.dpp_model == 4) {
+        const double tmid = S.elapsed + ((double)fb + 0.5 * (double)(fe - fb)) * dt;
+        const bool direct_on = isfinite(prm.t_acc_direct_gyr) && prm.t_acc_direct_gyr > 0.0 && isfinite(prm.t_off_gyr) &&
+                               prm.t_off_gyr > 0.0 && isfinite(prm.t_acc_off_gyr) && prm.t_acc_off_gyr > 0.0;
+        if (direct_on && tmid < prm.t_off_gyr) tacc_d = prm.t_acc_off_gyr;
+    }
+    double inv_on = 0.0;
+    const bool mode_on = d_dpp_model(prm, prm.dpp_model, lturb, dv, cs, beta, tacc_d, &inv_on) != 0;
+    sv[SV_DFAC] = mode_on ? inv_on : 1.0 / (4.0 * 1.0e+5);
+    sv[SV_MODEL] = mode_on ? 1.0 : 0.0;
+    sv[SV_QT] = (prm.dpp_model != 3 && prm.eta_dpp_cap > 0.0)
+                    ? d_eta_qt(prm, prm.dpp_model, lturb, dv, cs, beta, mass, tacc_d)
+                    : 0.0;
+    sv[SV_ADIA] = 1.0 / 3.0 * (dis ? 0.0 : v[CK_BG_DIVV]);
+    sv[SV_NGAS] = n_gas;
+    if (ELEC) {
+        // (prepare_cre_losses_1d, fp_shared_core.c:780-842); ln(p / n_gas) as
+        // ln p (table) + ln(1 / n_gas)
+        const double b_micro = v[CK_BG_B] * 1.0e+6;
+        const double b_ratio = b_micro / 3.2;
+        sv[SV_SYNCH] = 4.8e-4 * b_ratio * b_ratio * 9.11e-28 * 3.0e+10 * 3.1536e+16;
+        sv[SV_COUL] = 3.05e-29 * n_gas * K_C * K_GYR / (K_ME * K_GEV);
+        sv[SV_LNING] = log(1.0 / n_gas);
+    }
+    if (PROT) {
+        sv[ELEC ? (int)SV_EP_KBT : (int)SV_KBT] = v[CK_BG_KBT];
+        sv[ELEC ? (int)SV_EP_IKBT : (int)SV_IKBT] = 1.0 / v[CK_BG_KBT];
+    }
+}
 
 // Electron loss rates of the lane's rows for one segment
 // (prepare_cre_losses_1d, fp_shared_core.c:780-842).
 template <int R, typename T>
-__device__ __forceinline__ void seg_radp_e(const SpGridT<T> &sg, const CkSlot &S, int base, int nseg, double alpha,
-                                           const SegScalars &q, T *radp)
+__device__ __forceinline__ void seg_radp_e(const SpGridT<T> &sg, const double *ric_c, const double *ric_n, int base,
+                                           double alpha, const double *sv, T *radp)
 {
 #pragma clang fp contract(off)
-    {
-        const double b_micro = q.bfield * 1.0e+6;
-        const double b_ratio = b_micro / 3.2;
-        const T synch_coeff = (T)(4.8e-4 * b_ratio * b_ratio * 9.11e-28 * 3.0e+10 * 3.1536e+16);
-        const T coul_coeff = (T)(3.05e-29 * q.n_gas * K_C * K_GYR / (K_ME * K_GEV));
-        const T adia = (T)(1.0 / 3.0 * q.divv);
-        // ln(p / n_gas) as ln p (table) + ln(1 / n_gas), one log per segment
-        const T lning = (T)log(1.0 / q.n_gas);
+    const T synch = (T)sv[SV_SYNCH], coul_coeff = (T)sv[SV_COUL], lning = (T)sv[SV_LNING], adia = (T)sv[SV_ADIA];
 #pragma unroll
-        for (int k = 0; k < R; ++k) {
-            const int j = base + k;
-            const T pe = sg.x[sg.ix(j)];
-            const T pe2 = sg.p2[sg.ix(j)];
-            // both rows loaded unconditionally (ric_n is always a valid row)
-            // alpha is 0 without interpolation; ric_n is always a valid row
-            const T ric = (T)d_lerp(S.ric_c[j], S.ric_n[j], alpha);
-            const T coul = coul_coeff * ((T)1.0 + (sg.lnp[sg.ix(j)] + lning) * (T)(1.0 / 74.8)) * sg.ib2[sg.ix(j)];
-            radp[k] = synch_coeff * pe2 + ric + coul + adia * pe;
-        }
+    for (int k = 0; k < R; ++k) {
+        const int j = base + k;
+        const T pe = sg.x[sg.ix(j)];
+        const T pe2 = sg.p2[sg.ix(j)];
+        // both rows loaded unconditionally (ric_n is always a valid row); alpha
+        // is 0 (exactly the current row) without interpolation, below 1 with it
+        const T ric = (T)(ric_c[j] + alpha * (ric_n[j] - ric_c[j]));
+        const T coul = coul_coeff * ((T)1.0 + (sg.lnp[sg.ix(j)] + lning) * (T)(1.0 / 74.8)) * sg.ib2[sg.ix(j)];
+        radp[k] = synch * pe2 + ric + coul + adia * pe;
     }
 }
 
@@ -1103,28 +1204,22 @@ __device__ __forceinline__ void seg_radp_e(const SpGridT<T> &sg, const CkSlot &S
 // ceil(rows / G) times.  s_tr holds N + N / R doubles (row j at j + j / R:
 // one pad slot per block of R rows against LDS bank conflicts on the reads).
 template <int N, int R, int G, typename T>
-__device__ __forceinline__ void seg_radp_p(const SpGridT<T> &sg, int gl, const SegScalars &q, T *s_tr)
+__device__ __forceinline__ void seg_radp_p(const SpGridT<T> &sg, int gl, double n_gas, double kbt, double ikbt,
+                                           double adia, T *s_tr)
 {
 #pragma clang fp contract(off)
 #pragma unroll
     for (int m = 0; m < R; ++m) {
         const int j = m * G + gl;
         const int i = sg.ix(j);
-        if constexpr (sizeof(T) == sizeof(double)) {
-            const double adia = 1.0 / 3.0 * q.divv;
-            const double ikbt = 1.0 / q.kbt;
-            s_tr[j + j / R] =
-                d_b_coulomb_p_tab(q.n_gas, q.kbt, ikbt, sg.Ep[i], sg.i2mk[i], sg.ib2[i]) + adia * sg.x[i];
-        } else {
-            const float adia = (float)(1.0 / 3.0 * q.divv);
-            s_tr[j + j / R] = d_b_coulomb_p_tabf((float)q.n_gas, (float)q.kbt, (float)(1.0 / q.kbt), sg.Ep[i],
-                                                 sg.i2mk[i], sg.ib2[i]) +
-                              adia * sg.x[i];
-        }
+        if constexpr (sizeof(T) == sizeof(double))
+            s_tr[j + j / R] = d_b_coulomb_p_tab(n_gas, kbt, ikbt, sg.Ep[i], sg.i2mk[i], sg.ib2[i]) + adia * sg.x[i];
+        else
+            s_tr[j + j / R] = d_b_coulomb_p_tabf((float)n_gas, (float)kbt, (float)ikbt, sg.Ep[i], sg.i2mk[i],
+                                                 sg.ib2[i]) +
+                              (float)adia * sg.x[i];
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_sync();
 }
 
 // The lane's R spectrum values move to LDS (own slots, stride R + 1) while a
@@ -1169,7 +1264,7 @@ __device__ __forceinline__ void species_segment(int gl, const SpGridT<T> &sg, in
         rc.dfac = on ? dfac_on : dfac_off;
         if (s0 > 0) park_rows<R>(xpark, x);
         Factor<R, G> F;
-        build_factor<ELEC, R, G, T, NOSRC>(gl, N, sg, rc, radp, src, F, bad);
+        build_factor<ELEC, R, G, T, NOSRC>(gl, sg, rc, radp, src, F, bad);
         unpark_rows<R>(xpark, x);
         // substeps two per loop trip (one loop branch per pair)
         int s = s0;
@@ -1198,10 +1293,12 @@ enum { CK_MODE_E = 0,      // electron_only: protons are exactly zero
 
 // LDS doubles per lane group of the fused kernel: loss rates (padded), the
 // parked spectrum (PK), in mode EP the contraction's protons / electron
-// sources, and the tracer's backgrounds at two snapshots.
-__host__ __device__ constexpr int fused_lds_doubles(int N, int R, int MODE, bool PK)
+// sources, the tracer's backgrounds at two snapshots, and the scalars of SC
+// segments.
+__host__ __device__ constexpr int fused_lds_doubles(int N, int R, int MODE, bool PK, int SC)
 {
-    return N + N / R + 1 + (PK ? (N / R) * (R + 1) : 0) + (MODE == CK_MODE_EP ? N : 0) + 2 * CK_NBG;
+    return N + N / R + 1 + (PK ? (N / R) * (R + 1) : 0) + (MODE == CK_MODE_EP ? N : 0) + 2 * CK_NBG +
+           SC * fused_nsv(MODE);
 }
 
 // Grid tables copied to LDS per block (electron set, proton set or both).
@@ -1212,29 +1309,41 @@ __host__ __device__ constexpr int fused_grid_tables(int MODE)
 
 // Whether the blocks that the register budget lets share a CU (OCC waves per
 // SIMD, WPB waves per block) fit its 160 KiB of LDS with the grid tables (LG,
-// TB bytes per entry: 8 for FP64 coefficients, 4 for FP32) and the parked
-// spectra (PK).
+// TB bytes per entry: 8 for FP64 coefficients, 4 for FP32), the parked
+// spectra (PK) and the scalars of SC segments per group.
 __host__ __device__ constexpr bool fused_lds_fits(int N, int R, int WPB, int MODE, int OCC, bool LG, bool PK,
-                                                  int TB = 8)
+                                                  int TB, int SC)
 {
-    return ((size_t)8 * WPB * (64 / (N / R)) * fused_lds_doubles(N, R, MODE, PK) +
+    return ((size_t)8 * WPB * (64 / (N / R)) * fused_lds_doubles(N, R, MODE, PK, SC) +
             (LG ? (size_t)TB * fused_grid_tables(MODE) * (N + N / R + 1) : 0)) *
                (OCC * 4 / WPB > 0 ? OCC * 4 / WPB : 1) <=
            (size_t)160 * 1024;
 }
 // LDS use of an instance: the grid tables take precedence over parking (the
-// tables cut the build's load latency, parking its register pressure).
+// tables cut the build's load latency, parking its register pressure), and
+// both over more than one segment's scalars at a time.
 // FP32-coefficient instances exist only where their float tables fit.
 __host__ __device__ constexpr bool fused_use_lg(int N, int R, int WPB, int MODE, int OCC, int TB = 8)
 {
-    return fused_lds_fits(N, R, WPB, MODE, OCC, true, false, TB);
+    return fused_lds_fits(N, R, WPB, MODE, OCC, true, false, TB, 1);
 }
 __host__ __device__ constexpr bool fused_use_pk(int N, int R, int WPB, int MODE, int OCC, int TB = 8)
 {
-    return fused_lds_fits(N, R, WPB, MODE, OCC, fused_use_lg(N, R, WPB, MODE, OCC, TB), true, TB);
+    return fused_lds_fits(N, R, WPB, MODE, OCC, fused_use_lg(N, R, WPB, MODE, OCC, TB), true, TB, 1);
+}
+// Segments whose scalars are evaluated at a time: the largest power of two up
+// to 16 (the default most of a snapshot) and the group's lanes that fits.
+__host__ __device__ constexpr int fused_sc(int N, int R, int WPB, int MODE, int OCC, int TB = 8)
+{
+    int sc = 16;
+    while (sc > N / R) sc /= 2;
+    while (sc > 1 && !fused_lds_fits(N, R, WPB, MODE, OCC, fused_use_lg(N, R, WPB, MODE, OCC, TB),
+                                     fused_use_pk(N, R, WPB, MODE, OCC, TB), TB, sc))
+        sc /= 2;
+    return sc;
 }
 
-template <int N, int R, int MODE, bool PK, typename T>
+template <int N, int R, int MODE, bool PK, int SC, typename T>
 __device__ __forceinline__ void snapshot_update(const CkGrid &g, const SpGridT<T> &sge, const SpGridT<T> &sgp,
                                                 const CkSlot &S, int t, int gl, double *s_grp, double (&xe)[R],
                                                 double (&xp)[R], int &bad)
@@ -1253,8 +1362,10 @@ __device__ __forceinline__ void snapshot_update(const CkGrid &g, const SpGridT<T
     const CkParams &prm = S.prm;
     const int nsub = S.nsub[t];
     const int non = S.n_on[t];
+    // a power of two: nseg = 2^sh
     const int nseg =
         d_choose_segments(nsub, S.allow_interp, prm.coeff_interp_min_steps, prm.coeff_interp_max_segments);
+    const int sh = 31 - __builtin_clz((unsigned)nseg);
     const int on_start = (nsub - non) / 2;
     const int on_end = on_start + non;
     const double dt = S.dt_snap / (double)nsub;
@@ -1273,48 +1384,32 @@ __device__ __forceinline__ void snapshot_update(const CkGrid &g, const SpGridT<T
     // the tracer's backgrounds at this snapshot and the next, one round trip
     // for the group, then read from LDS by every segment
     for (int i = gl; i < 2 * CK_NBG; i += G) s_bg[i] = (i < CK_NBG ? S.bgc[i] : S.bgn[i - CK_NBG])[t];
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_sync();
+    double *const s_sv = s_bg + 2 * CK_NBG;
+    const double *const ric_c = S.ric_c, *const ric_n = S.ric_n;
+    const bool capped = prm.dpp_model != 3 && prm.eta_dpp_cap > 0.0;
 
     for (int iseg = 0; iseg < nseg; ++iseg) {
-        const int fb = (int)(((long long)iseg * nsub) / nseg);
-        const int fe = (int)(((long long)(iseg + 1) * nsub) / nseg);
+        if ((iseg & (SC - 1)) == 0) {
+            // the scalars of the next SC segments, one per lane
+            if (gl < SC && iseg + gl < nseg)
+                seg_scalars<MODE>(S, s_bg, iseg + gl, sh, nsub, dt, dis, mass, s_sv + gl * fused_nsv(MODE));
+            wave_sync();
+        }
+        const double *const sv = s_sv + (iseg & (SC - 1)) * fused_nsv(MODE);
+        const int fb = (int)(((long long)iseg * nsub) >> sh);
+        const int fe = (int)(((long long)(iseg + 1) * nsub) >> sh);
         const int steps = fe - fb;
         if (steps <= 0) continue;
-        const double alpha = (nseg > 1) ? ((double)iseg + 0.5) / (double)nseg : 0.0;
-        SegScalars q;
-        {
-            // alpha is 0 (the current snapshot's value) without interpolation
-            double v[CK_NBG];
-#pragma unroll
-            for (int f = 0; f < CK_NBG; ++f) v[f] = d_lerp(s_bg[f], s_bg[CK_NBG + f], alpha);
-            q.n_gas = v[CK_BG_NGAS];
-            q.kbt = v[CK_BG_KBT];
-            q.bfield = v[CK_BG_B];
-            q.divv = dis ? 0.0 : v[CK_BG_DIVV];
-            q.lturb = v[CK_BG_LTURB];
-            q.dv = v[CK_BG_DV];
-            q.cs = v[CK_BG_CS];
-            q.beta = v[CK_BG_BETA];
-        }
+        const double alpha = sh ? ldexp((double)iseg + 0.5, -sh) : 0.0;
         int sob = (on_start > fb) ? on_start : fb;
         int soe = (on_end < fe) ? on_end : fe;
         if (soe < sob) soe = sob;
         const bool windowed = (soe - sob) < steps;
         const int ls = sob - fb, le = ls + (soe - sob);
-        double tacc_d = prm.t_acc_direct_gyr;
-        {
-            const double tmid = S.elapsed + ((double)fb + 0.5 * (double)steps) * dt;
-            const bool direct_on = prm.dpp_model == 4 && isfinite(prm.t_acc_direct_gyr) &&
-                                   prm.t_acc_direct_gyr > 0.0 && isfinite(prm.t_off_gyr) && prm.t_off_gyr > 0.0 &&
-                                   isfinite(prm.t_acc_off_gyr) && prm.t_acc_off_gyr > 0.0;
-            if (direct_on && tmid < prm.t_off_gyr) tacc_d = prm.t_acc_off_gyr;
-        }
-        double inv_on = 0.0;
-        const bool mode_on = d_dpp_model(prm, prm.dpp_model, q.lturb, q.dv, q.cs, q.beta, tacc_d, &inv_on) != 0;
+        const bool mode_on = sv[SV_MODEL] != 0.0;
         double scale = 1.0;
-        if (prm.dpp_model != 3 && prm.eta_dpp_cap > 0.0) {
+        if (capped) {
             double part = 0.0;
 #pragma unroll
             for (int k = 0; k < R; ++k) {
@@ -1325,17 +1420,16 @@ __device__ __forceinline__ void snapshot_update(const CkGrid &g, const SpGridT<T
                 if (we_ > 0.0 && isfinite(xe[k])) part += we_ * xe[k] * g.edp[j];
             }
             const double ecr = g_sum<G>(part);
-            scale = d_eta_scale(prm, prm.dpp_model, q.lturb, q.dv, q.cs, q.beta, mass, tacc_d, ecr);
+            scale = d_eta_scale_qt(prm.eta_dpp_cap, sv[SV_QT], ecr);
         }
         RunCoef rc;
         rc.dt = dt;
         rc.model = false;
         rc.dfac = 0.0;
-        rc.inv_epmax = 1.0 / prm.epmax;
         rc.dtT_fac = 0.0;
         // D prefactors: on-window uses the model form times the eta scale (or
         // the floor times the scale), outside the floor p^2/4e5
-        const double dfac_on = mode_on ? inv_on * scale : (1.0 / (4.0 * 1.0e+5)) * scale;
+        const double dfac_on = sv[SV_DFAC] * scale;
         const double dfac_off = 1.0 / (4.0 * 1.0e+5);
 
         if (PROT) {
@@ -1350,9 +1444,10 @@ __device__ __forceinline__ void snapshot_update(const CkGrid &g, const SpGridT<T
                 for (int k = 0; k < R; ++k) rec[k] = xp[k];
             }
             park_rows<R>(own_x, xp);
-            seg_radp_p<N, R, G, T>(sgp, gl, q, s_rad);
+            seg_radp_p<N, R, G, T>(sgp, gl, sv[SV_NGAS], sv[ELEC ? (int)SV_EP_KBT : (int)SV_KBT],
+                                   sv[ELEC ? (int)SV_EP_IKBT : (int)SV_IKBT], sv[SV_ADIA], s_rad);
             RunCoef rp = rc;
-            rp.dtT_fac = dt * (0.5 * K_C * q.n_gas) * K_GYR;
+            rp.dtT_fac = dt * (0.5 * K_C * sv[SV_NGAS]) * K_GYR;
             const SrcRows sp = {S.qpi ? S.qpi + roff : g.zeros + base, g.zeros + base, 0.0, 0.0, dt};
             species_segment<false, N, R, G, T>(gl, sgp, steps, windowed, ls, le, rp, dfac_on, dfac_off, mode_on, own_rad,
                                             sp, own_x, xp, bad);
@@ -1366,9 +1461,7 @@ __device__ __forceinline__ void snapshot_update(const CkGrid &g, const SpGridT<T
                 double acc[R];
 #pragma unroll
                 for (int k = 0; k < R; ++k) acc[k] = 0.0;
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                wave_sync();
                 for (int jp = S.jp0; jp < N; ++jp) {
                     const double nn = s_row[jp];
                     const double *wrow = S.fqe_t + (size_t)jp * N + base;
@@ -1377,16 +1470,14 @@ __device__ __forceinline__ void snapshot_update(const CkGrid &g, const SpGridT<T
                 }
                 // every lane of the group has read the protons before the
                 // sources overwrite them
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                wave_sync();
 #pragma unroll
-                for (int k = 0; k < R; ++k) src[k] = acc[k] * K_GYR * q.n_gas + src[k];
+                for (int k = 0; k < R; ++k) src[k] = acc[k] * K_GYR * sv[SV_NGAS] + src[k];
             }
 #pragma unroll
             for (int k = 0; k < R; ++k) own_src[k] = dt * src[k];
             park_rows<R>(own_x, xe);
-            seg_radp_e<R, T>(sge, S, base, nseg, alpha, q, (T *)s_grp + gl * (R + 1));
+            seg_radp_e<R, T>(sge, ric_c, ric_n, base, alpha, sv, (T *)s_grp + gl * (R + 1));
             const SrcRows se = {own_src, g.zeros + base, 0.0, 0.0, 1.0};
             species_segment<true, N, R, G, T>(gl, sge, steps, windowed, ls, le, rc, dfac_on, dfac_off, mode_on, own_rad,
                                            se, own_x, xe, bad);
@@ -1397,15 +1488,15 @@ __device__ __forceinline__ void snapshot_update(const CkGrid &g, const SpGridT<T
             const double *inj =
                 (MODE == CK_MODE_E_SEC) ? S.seg_inje + (size_t)(row0 + iseg) * N + base : g.zeros + base;
             park_rows<R>(own_x, xe);
-            seg_radp_e<R, T>(sge, S, base, nseg, alpha, q, (T *)s_grp + gl * (R + 1));
-            const SrcRows se = {S.qepri ? S.qepri + roff : g.zeros + base, inj, K_GYR, q.n_gas, dt};
+            seg_radp_e<R, T>(sge, ric_c, ric_n, base, alpha, sv, (T *)s_grp + gl * (R + 1));
+            const SrcRows se = {S.qepri ? S.qepri + roff : g.zeros + base, inj, K_GYR, sv[SV_NGAS], dt};
             species_segment<true, N, R, G, T, MODE == CK_MODE_E_NOSRC>(gl, sge, steps, windowed, ls, le, rc, dfac_on,
                                                                       dfac_off, mode_on, own_rad, se, own_x, xe, bad);
         }
     }
 }
 
-template <int N, int R, int WPB, int MODE, bool LG, bool PK, typename T>
+template <int N, int R, int WPB, int MODE, bool LG, bool PK, int SC, typename T>
 __device__ __forceinline__ void k_fused_body(const CkGrid &g, const CkSlot *__restrict__ slots,
                                              const CkTask *__restrict__ tasks, int ntasks,
                                              int *__restrict__ counter, int *__restrict__ err)
@@ -1414,7 +1505,7 @@ __device__ __forceinline__ void k_fused_body(const CkGrid &g, const CkSlot *__re
     constexpr bool ELEC = (MODE != CK_MODE_P_REC);
     constexpr int G = N / R;
     constexpr int GPW = 64 / G;
-    __shared__ double s_lds[WPB][GPW][fused_lds_doubles(N, R, MODE, PK)];
+    __shared__ double s_lds[WPB][GPW][fused_lds_doubles(N, R, MODE, PK, SC)];
     constexpr int NP = N + N / R + 1;
     constexpr int PS = LogG<R>::v;
     static_assert(LG || sizeof(T) == sizeof(double), "FP32-coefficient instances need their tables in LDS");
@@ -1469,7 +1560,7 @@ __device__ __forceinline__ void k_fused_body(const CkGrid &g, const CkSlot *__re
             // a task advances one tracer over nslot consecutive snapshots
             for (int sl = task.slot; sl < task.slot + task.nslot; ++sl) {
                 const CkSlot &S = slots[sl];
-                snapshot_update<N, R, MODE, PK, T>(g, sge, sgp, S, t, gl, s_grp, xe, xp, bad);
+                snapshot_update<N, R, MODE, PK, SC, T>(g, sge, sgp, S, t, gl, s_grp, xe, xp, bad);
                 if (ELEC && S.out_e && !idle) {
 #pragma unroll
                     for (int k = 0; k < R; ++k) S.out_e[roff + k] = xe[k];
@@ -1503,5 +1594,5 @@ __global__ __launch_bounds__(WPB * 64) __attribute__((amdgpu_waves_per_eu(OCC, 8
 {
     constexpr int TB = (int)sizeof(T);
     k_fused_body<N, R, WPB, MODE, fused_use_lg(N, R, WPB, MODE, OCC, TB), fused_use_pk(N, R, WPB, MODE, OCC, TB),
-                 T>(g, slots, tasks, ntasks, counter, err);
+                 fused_sc(N, R, WPB, MODE, OCC, TB), T>(g, slots, tasks, ntasks, counter, err);
 }

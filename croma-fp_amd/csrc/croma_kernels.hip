@@ -53,10 +53,11 @@ extern "C" int ck_fused_supported(int n, int r)
 }
 
 // Host-side check of one fused instance's LDS use.  Per lane group the
-// slice of fused_lds_doubles(N, R, MODE, PK) doubles holds, in this order,
+// slice of fused_lds_doubles(N, R, MODE, PK, SC) doubles holds, in this order,
 // the segment's loss rates (row j at j + j / R; a lane reads its own rows
 // at gl (R + 1) + k), the parked spectrum (PK; rows at gl (R + 1) + k), the
-// EP rows (MODE 1; row j at j) and the 2 CK_NBG backgrounds.  info[0..5]:
+// EP rows (MODE 1; row j at j), the 2 CK_NBG backgrounds and the scalars of SC
+// segments.  info[0..5]:
 // largest index of each region's accesses (rates, own rates, parked, EP,
 // backgrounds) and the slice size; info[6] the bytes a CU holds for the
 // blocks its register budget admits.  Returns 0 when every index lies in the
@@ -67,7 +68,8 @@ extern "C" int ck_fused_lds_check(int n, int r, int occ, int mode, int tb, long 
     const int WPB = 4, G = n / r;
     const bool LG = fused_use_lg(n, r, WPB, mode, occ, tb);
     const bool PK = fused_use_pk(n, r, WPB, mode, occ, tb);
-    const long D = fused_lds_doubles(n, r, mode, PK);
+    const int SC = fused_sc(n, r, WPB, mode, occ, tb);
+    const long D = fused_lds_doubles(n, r, mode, PK, SC);
     const long nrates = n + n / r + 1;
     const long rates_max = (long)(n - 1) + (n - 1) / r;
     const long own_rates_max = (long)(G - 1) * (r + 1) + r - 1;
@@ -76,6 +78,7 @@ extern "C" int ck_fused_lds_check(int n, int r, int occ, int mode, int tb, long 
     const long row_base = pk_base + (PK ? (long)G * (r + 1) : 0);
     const long ep_max = (mode == CK_MODE_EP) ? row_base + n - 1 : -1;
     const long bg_max = row_base + (mode == CK_MODE_EP ? n : 0) + 2 * CK_NBG - 1;
+    const long sv_max = bg_max + (long)SC * fused_nsv(mode);
     const long blocks = (occ * 4 / WPB > 0) ? occ * 4 / WPB : 1;
     const long bytes = (8L * WPB * (64 / G) * D + (LG ? (long)tb * fused_grid_tables(mode) * nrates : 0)) * blocks;
     if (info) {
@@ -88,7 +91,7 @@ extern "C" int ck_fused_lds_check(int n, int r, int occ, int mode, int tb, long 
         info[6] = bytes;
     }
     const bool ok = rates_max < nrates && own_rates_max < nrates && parked_max < row_base && ep_max < D &&
-                    bg_max < D && bytes <= 160L * 1024 && (LG || tb == 8);
+                    bg_max < D && sv_max < D && SC >= 1 && SC <= G && bytes <= 160L * 1024 && (LG || tb == 8);
     return ok ? 0 : 1;
 }
 
