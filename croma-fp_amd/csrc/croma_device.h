@@ -651,12 +651,33 @@ __device__ __forceinline__ void pm_row_scan(int gl, int rl, double &m00, double 
     }
 }
 
-// Thomas LU of the rows held in F (on entry al = a, iv = b, g = c), as in
-// fp_thomas_solve_ws (fp_shared_core.c:226-257): denom_i = b_i + a_i cprime_{i-1},
-// cprime_i = -c_i / denom_i, pivot guard |denom| <= 1e-300.  The pivot
-// entering each lane comes from a scan of 2x2 projective maps across the
-// group's lanes, exact up to rounding of the products; inside the lane the
-// reference recurrence is applied.
+// Scan multipliers of a lane group from the lanes' products A (of al) and Bq
+// (of g).
+template <int R, int G>
+__device__ __forceinline__ void group_coeffs(int gl, double A, double Bq, Factor<R, G> &F)
+{
+    scan_coeffs<G, 0>(gl, (int)(threadIdx.x & 15), A, Bq, F);
+    // two-row groups: the carry multiplier is used in rows 1 and 3 only
+    F.PA = (G == 32 && !((threadIdx.x >> 4) & 1)) ? 0.0 : A;
+    F.PQ = Bq;
+    if constexpr (G == 32) {
+        const int row = (int)((threadIdx.x & 63) >> 4);
+        F.PQ0 = (row == 0) ? Bq : 0.0;
+        F.PQ2 = (row == 2) ? Bq : 0.0;
+    }
+    if constexpr (G == 64) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            F.Tf[r] = rdlane64(A, 16 * r + 15);
+            F.Tb[r] = rdlane64(Bq, 16 * r);
+        }
+    }
+}
+
+// cprime entering each lane (0 at the group's first) of the Thomas recurrence
+// denom_i = b_i + a_i cprime_{i-1}, cprime_i = -c_i / denom_i over the group's
+// rows, from a scan of 2x2 projective maps across the lanes, exact up to
+// rounding of the products.
 //
 // Row k maps (u, v), cprime = u / v, to (-c_k v, a_k u + b_k v); both columns
 // of the product over the lane's rows therefore follow the three-term
@@ -667,27 +688,26 @@ __device__ __forceinline__ void pm_row_scan(int gl, int rl, double &m00, double 
 // row; the up to six products across lanes then stay within 2^63 of the
 // renormalised entries and shrink by at most a few powers of R per lane, so
 // they need no further scaling.
-template <int R, int G, bool NOSRC = false>
-__device__ __forceinline__ void factorize(int gl, const double (&sv)[R], Factor<R, G> &F, int &bad)
+template <int R, int G>
+__device__ __forceinline__ double pivot_in(int gl, const double (&a)[R], const double (&b)[R], const double (&c)[R])
 {
     double m00, m01, m10, m11;
     {
         // (p, q): the recurrence at the row before and at this row, of the
         // columns that start from (u, v) = (1, 0) and (0, 1)
-        double p0 = 0.0, q0 = F.al[0], p1 = 1.0, q1 = F.iv[0];
+        double p0 = 0.0, q0 = a[0], p1 = 1.0, q1 = b[0];
 #pragma unroll
         for (int k = 1; k < R; ++k) {
-            const double ac = F.al[k] * F.g[k - 1], b = F.iv[k];
-            const double n0 = fma(b, q0, -(ac * p0)), n1 = fma(b, q1, -(ac * p1));
+            const double ac = a[k] * c[k - 1];
+            const double n0 = fma(b[k], q0, -(ac * p0)), n1 = fma(b[k], q1, -(ac * p1));
             p0 = q0;
             p1 = q1;
             q0 = n0;
             q1 = n1;
             if ((k & 7) == 7 && k < R - 1) pm_renorm(p0, p1, q0, q1);
         }
-        const double c = F.g[R - 1];
-        m00 = (R > 1 ? -c * p0 : 0.0);
-        m01 = -c * p1;
+        m00 = -c[R - 1] * p0;
+        m01 = -c[R - 1] * p1;
         m10 = q0;
         m11 = q1;
         pm_renorm(m00, m01, m10, m11);
@@ -722,7 +742,17 @@ __device__ __forceinline__ void factorize(int gl, const double (&sv)[R], Factor<
         if (row) pm_apply(m00, m01, m10, m11, c01, c11);
     }
     const double uin = wave_up1(m01), vin = wave_up1(m11);
-    double cprev = (gl == 0) ? 0.0 : d_div_normal(uin, vin);
+    return (gl == 0) ? 0.0 : d_div_normal(uin, vin);
+}
+
+// Thomas LU of the rows held in F (on entry al = a, iv = b, g = c), as in
+// fp_thomas_solve_ws (fp_shared_core.c:226-257), pivot guard |denom| <=
+// 1e-300: the cprime entering each lane comes from pivot_in; inside the lane
+// the reference recurrence is applied.
+template <int R, int G, bool NOSRC = false>
+__device__ __forceinline__ void factorize(int gl, const double (&sv)[R], Factor<R, G> &F, int &bad)
+{
+    double cprev = pivot_in<R, G>(gl, F.al, F.iv, F.g);
     bool ok = true;
     double A = 1.0, Bq = 1.0;
 #pragma unroll
@@ -744,25 +774,7 @@ __device__ __forceinline__ void factorize(int gl, const double (&sv)[R], Factor<
         cprev = cp;
     }
     if (!ok) bad |= ERR_PIVOT;
-    // Scan multipliers of the substep solve.  Hillis-Steele levels run
-    // inside 16-lane rows (DPP); a group spanning several rows completes the
-    // scan with per-row carries (see apply_solve).
-    scan_coeffs<G, 0>(gl, rl, A, Bq, F);
-    // two-row groups: the carry multiplier is used in rows 1 and 3 only
-    F.PA = (G == 32 && !((threadIdx.x >> 4) & 1)) ? 0.0 : A;
-    F.PQ = Bq;
-    if constexpr (G == 32) {
-        const int row = (int)((threadIdx.x & 63) >> 4);
-        F.PQ0 = (row == 0) ? Bq : 0.0;
-        F.PQ2 = (row == 2) ? Bq : 0.0;
-    }
-    if constexpr (G == 64) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            F.Tf[r] = rdlane64(A, 16 * r + 15);
-            F.Tb[r] = rdlane64(Bq, 16 * r);
-        }
-    }
+    group_coeffs(gl, A, Bq, F);
 }
 
 // In-row Hillis-Steele levels of the forward (prefix) and backward (suffix)
@@ -785,21 +797,13 @@ __device__ __forceinline__ void scan_bwd(const double *Qb, double &B)
     }
 }
 
-// One implicit substep: x <- M^{-1} (x + src) for the group, in place.
-// NOSRC: a run without sources (src = 0; vs is not formed).
-template <int R, int G, bool NOSRC = false>
-__device__ __forceinline__ void apply_solve(int gl, const Factor<R, G> &F, double (&x)[R])
+// Inclusive prefix (suffix) of the lanes' affine maps: L_l (M_l), the value of
+// the lane's last (first) row from a zero value entering it, becomes the true
+// one.  Hillis-Steele levels run inside 16-lane rows (DPP); a group spanning
+// several rows completes the scan with per-row carries.
+template <int R, int G>
+__device__ __forceinline__ double group_prefix(const Factor<R, G> &F, double L)
 {
-    double t[R];
-    // the lane-local prefixes start from the first row itself (al * 0 + t is
-    // t exactly for the finite multipliers of a factorised run)
-    t[0] = NOSRC ? F.iv[0] * x[0] : fma(F.iv[0], x[0], F.vs[0]);
-    double L = t[0];
-#pragma unroll
-    for (int k = 1; k < R; ++k) {
-        t[k] = NOSRC ? F.iv[k] * x[k] : fma(F.iv[k], x[k], F.vs[k]);
-        L = fma(F.al[k], L, t[k]);
-    }
     scan_fwd<G, 0, Factor<R, G>::LV>(F.Af, L);
     if constexpr (G == 32) {
         // rows 1 and 3 continue the groups begun in rows 0 and 2: they take
@@ -818,16 +822,11 @@ __device__ __forceinline__ void apply_solve(int gl, const Factor<R, G> &F, doubl
         const double C = (row == 1) ? C1 : (row == 2) ? C2 : (row == 3) ? C3 : 0.0;
         L = fma(F.PA, C, L);
     }
-    // the first lane of the group multiplies the shifted-in value by al[0] = 0
-    double d = wave_up1(L);
-#pragma unroll
-    for (int k = 0; k < R; ++k) {
-        d = fma(F.al[k], d, t[k]);
-        t[k] = d;
-    }
-    double M = t[R - 1];
-#pragma unroll
-    for (int k = R - 2; k >= 0; --k) M = fma(F.g[k], M, t[k]);
+    return L;
+}
+template <int R, int G>
+__device__ __forceinline__ double group_suffix(const Factor<R, G> &F, double M)
+{
     scan_bwd<G, 0, Factor<R, G>::LV>(F.Qb, M);
     if constexpr (G == 32) {
         // rows 0 and 2 take the value at the first lane of the row after:
@@ -844,6 +843,36 @@ __device__ __forceinline__ void apply_solve(int gl, const Factor<R, G> &F, doubl
         const double D = (row == 0) ? D0 : (row == 1) ? D1 : (row == 2) ? D2 : 0.0;
         M = fma(F.PQ, D, M);
     }
+    return M;
+}
+
+// One implicit substep: x <- M^{-1} (x + src) for the group, in place.
+// NOSRC: a run without sources (src = 0; vs is not formed).
+template <int R, int G, bool NOSRC = false>
+__device__ __forceinline__ void apply_solve(int gl, const Factor<R, G> &F, double (&x)[R])
+{
+    double t[R];
+    // the lane-local prefixes start from the first row itself (al * 0 + t is
+    // t exactly for the finite multipliers of a factorised run)
+    t[0] = NOSRC ? F.iv[0] * x[0] : fma(F.iv[0], x[0], F.vs[0]);
+    double L = t[0];
+#pragma unroll
+    for (int k = 1; k < R; ++k) {
+        t[k] = NOSRC ? F.iv[k] * x[k] : fma(F.iv[k], x[k], F.vs[k]);
+        L = fma(F.al[k], L, t[k]);
+    }
+    L = group_prefix(F, L);
+    // the first lane of the group multiplies the shifted-in value by al[0] = 0
+    double d = wave_up1(L);
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        d = fma(F.al[k], d, t[k]);
+        t[k] = d;
+    }
+    double M = t[R - 1];
+#pragma unroll
+    for (int k = R - 2; k >= 0; --k) M = fma(F.g[k], M, t[k]);
+    M = group_suffix(F, M);
     // the group's last row has g = 0 (the system's last row), so the value
     // shifted in from the lane after drops out without a select
     double xn = wave_dn1(M);

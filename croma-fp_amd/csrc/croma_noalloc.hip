@@ -2,13 +2,13 @@
 // allocate device memory (code under HIP graph capture, serving loops,
 // harnesses that forbid hipMalloc).
 //
-// It runs the kernel of croma_hip_solve_cc_batch (k_solve_cc_batch: x <-
+// It runs the kernels of croma_hip_solve_cc_batch (ck_solve_cc_batch: x <-
 // dt Q + x, then the Thomas sweep of fp_shared_core.c:226-257 per system) on
-// caller-owned device arrays.  The kernel's only scratch -- the modified
-// upper diagonal c' of every system and the pivot-failure word -- lives in
-// the file-scope device array `scratch` below: one copy per GPU, held until
-// the process ends, whose address is looked up once per device with
-// hipGetSymbolAddress.  Nothing here calls hipMalloc, hipFree or an
+// caller-owned device arrays.  Their only scratch -- the pivot-failure word
+// and, for systems longer than the lane-group kernel takes, the modified
+// upper diagonal c' -- lives in the file-scope device array `scratch` below:
+// one copy per GPU, held until the process ends, whose address is looked up
+// once per device with hipGetSymbolAddress.  Nothing here calls hipMalloc, hipFree or an
 // allocating library routine.
 //
 // Layout of `scratch`: bytes [0, 256) hold the pivot-failure word (cleared by
