@@ -506,39 +506,159 @@ __device__ __forceinline__ double wave_dn1(double v) { return dpp64<0x130>(v); }
 // held in registers.  One implicit substep is x <- M^{-1} (x + src):
 //   forward   d_i = al_i d_{i-1} + iv_i x_i + vs_i
 //   backward  x_i = d_i + g_i x_{i+1}
-// with the lane-level affine scans over the group (Af, Qb: products of al
-// resp. g over lane ranges, zero where the source lane is outside the group).
+// with the lane-level affine scans over the group (products of al resp. g
+// over lane ranges as multipliers, zero where the source lane does not count).
+//
+// The scan of a 16-lane row: a Hillis-Steele level is two 32-bit DPP moves
+// and an FMA per double; v_fmac_f64 takes row_newbcast (one lane of the row to
+// all) as its DPP form, one instruction.  So only the first levels are
+// Hillis-Steele, inside blocks of HS lanes, and the blocks' last (first) lanes
+// are broadcast: HS = 4, three broadcasts in sequence, each completing the next
+// block (9 instructions a direction against 12 for four levels, one
+// multiplier); or HS = 2, seven broadcasts that do not wait for each other
+// (11 instructions, seven multipliers, a third less latency), for up to 4 rows
+// per lane, where the chain through the scans is what a substep waits for.
+// With this, the overlap below and the wave priorities of k_fused_body: 256
+// electrons x 64 bins, 10 snapshots, 2.72 -> 2.51 ms (a launch waits for its
+// longest chain); 10,000 of both species x 256 bins 17.6 -> 16.9 ms; 65,536 x
+// 512 bins 153.7 -> 152.1 ms (8% fewer vector instructions, but the FP64
+// operations, which stay, hold the clock at 2.13 GHz).
 template <int R, int G>
 struct Factor {
-    static constexpr int LV = LogG<G>::v < 4 ? LogG<G>::v : 4;  // scan levels inside a 16-lane row
+    static constexpr bool ROW = G >= 16;           // the group covers whole 16-lane rows
+    static constexpr int HS = !ROW ? G : (R <= 4 ? 2 : 4);
+    static constexpr int LV = LogG<HS>::v;         // Hillis-Steele levels
+    static constexpr int NB = !ROW ? 0 : (HS == 2 ? 7 : 1);  // broadcast multipliers
+    // up to 8 rows per lane the local back substitution runs on the local
+    // forward values, beside the forward scan, and the carry's response K is
+    // added (apply_solve)
+    static constexpr bool OVERLAP = R <= 8;
     double al[R];   // a_i / denom_i
     double iv[R];   // 1 / denom_i
     double vs[R];   // src_i / denom_i
     double g[R];    // c_i / denom_i (= -cprime_i of the reference)
-    double Af[LV + 1];  // forward scan multipliers, zero where the source lane is outside the row / group
+    double Af[LV + 1];  // forward scan multipliers, zero where the source lane is outside the block
     double Qb[LV + 1];  // backward scan multipliers
+    double Ta[NB + 1], Tq[NB + 1];  // broadcast multipliers
+    double K;           // OVERLAP: response of the lane's local first-row value to the entering carry
     double PA, PQ;      // groups wider than a row: in-row inclusive products (prefix of A, suffix of Q)
     double PQ0, PQ2;    // two-row groups: PQ in rows 0 / 2 only (0 elsewhere)
     double Tf[4], Tb[4];  // and (one group per wave) the row totals of those products
 };
 
-// Multipliers of the in-row scan levels (and the running in-row products).
-template <int G, int ST, int R>
-__device__ __forceinline__ void scan_coeffs(int gl, int rl, double &A, double &Bq, Factor<R, G> &F)
+// lane K of each 16-lane row, in every lane of the row
+template <int K>
+__device__ __forceinline__ double row_bcast(double v)
 {
-    if constexpr (ST < Factor<R, G>::LV) {
+    const long r = __builtin_amdgcn_update_dpp(0L, (long)__double_as_longlong(v), 0x150 + K, 0xF, 0xF, true);
+    return __longlong_as_double(r);
+}
+
+// The broadcast steps.  A DPP operand must be two wait states old; the
+// compiler does not look into inline asm for that, so the blocks wait before
+// their first DPP read and, since their result goes into a DPP move next,
+// after their last write.
+__device__ __forceinline__ double bcast_prefix4(double L, double m)
+{
+    asm("s_nop 1\n\t"
+        "v_fmac_f64_dpp %0, %0, %1 row_newbcast:3 row_mask:0xf bank_mask:0x2\n\t"
+        "s_nop 1\n\t"
+        "v_fmac_f64_dpp %0, %0, %1 row_newbcast:7 row_mask:0xf bank_mask:0x4\n\t"
+        "s_nop 1\n\t"
+        "v_fmac_f64_dpp %0, %0, %1 row_newbcast:11 row_mask:0xf bank_mask:0x8\n\t"
+        "s_nop 1"
+        : "+v"(L)
+        : "v"(m));
+    return L;
+}
+__device__ __forceinline__ double bcast_suffix4(double M, double m)
+{
+    asm("s_nop 1\n\t"
+        "v_fmac_f64_dpp %0, %0, %1 row_newbcast:12 row_mask:0xf bank_mask:0x4\n\t"
+        "s_nop 1\n\t"
+        "v_fmac_f64_dpp %0, %0, %1 row_newbcast:8 row_mask:0xf bank_mask:0x2\n\t"
+        "s_nop 1\n\t"
+        "v_fmac_f64_dpp %0, %0, %1 row_newbcast:4 row_mask:0xf bank_mask:0x1\n\t"
+        "s_nop 1"
+        : "+v"(M)
+        : "v"(m));
+    return M;
+}
+__device__ __forceinline__ double bcast_prefix2(double L, const double *m)
+{
+    double r;
+    asm("v_mov_b64 %0, %1\n\t"
+        "s_nop 0\n\t"
+        "v_fmac_f64_dpp %0, %1, %2 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %0, %1, %3 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %0, %1, %4 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %0, %1, %5 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %0, %1, %6 row_newbcast:9 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %0, %1, %7 row_newbcast:11 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %0, %1, %8 row_newbcast:13 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1"
+        : "=&v"(r)
+        : "v"(L), "v"(m[0]), "v"(m[1]), "v"(m[2]), "v"(m[3]), "v"(m[4]), "v"(m[5]), "v"(m[6]));
+    return r;
+}
+__device__ __forceinline__ double bcast_suffix2(double M, const double *m)
+{
+    double r;
+    asm("v_mov_b64 %0, %1\n\t"
+        "s_nop 0\n\t"
+        "v_fmac_f64_dpp %0, %1, %2 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %0, %1, %3 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %0, %1, %4 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %0, %1, %5 row_newbcast:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %0, %1, %6 row_newbcast:10 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %0, %1, %7 row_newbcast:12 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %0, %1, %8 row_newbcast:14 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1"
+        : "=&v"(r)
+        : "v"(M), "v"(m[0]), "v"(m[1]), "v"(m[2]), "v"(m[3]), "v"(m[4]), "v"(m[5]), "v"(m[6]));
+    return r;
+}
+
+// Multipliers of the Hillis-Steele levels inside blocks of HS lanes (and the
+// running products over the block).
+template <int HS, int ST, int R, int G>
+__device__ __forceinline__ void scan_coeffs(int bl, double &A, double &Bq, Factor<R, G> &F)
+{
+    if constexpr ((1 << ST) < HS) {
         constexpr int s = 1 << ST;
         const double Ao = row_up<s>(A);
         const double Bo = row_dn<s>(Bq);
-        // a source lane outside the row (or, for groups narrower than a row,
-        // outside the group) contributes nothing
-        const bool okf = (G >= 16) ? (rl >= s) : (gl >= s);
-        const bool okb = (G >= 16) ? (rl + s <= 15) : (gl + s < G);
+        const bool okf = bl >= s, okb = bl + s < HS;
         F.Af[ST] = okf ? A : 0.0;
         F.Qb[ST] = okb ? Bq : 0.0;
         if (okf) A = A * Ao;
         if (okb) Bq = Bq * Bo;
-        scan_coeffs<G, ST + 1, R>(gl, rl, A, Bq, F);
+        scan_coeffs<HS, ST + 1, R, G>(bl, A, Bq, F);
+    }
+}
+
+// Multipliers of the seven pair broadcasts: the product over the lanes after
+// the broadcast lane 2J + 1 up to this one (prefix), from this one up to the
+// lane before lane 2J (suffix); 0 where the broadcast does not count.  On
+// exit acc is the product over the row up to (from) this lane.
+template <int J>
+__device__ __forceinline__ void pair_prefix_coeffs(int pr, double A2, double &acc, double *T)
+{
+    if constexpr (J >= 0) {
+        T[J] = (pr > J) ? acc : 0.0;
+        const double e = row_bcast<2 * J + 1>(A2);
+        if (pr > J) acc *= e;
+        pair_prefix_coeffs<J - 1>(pr, A2, acc, T);
+    }
+}
+template <int J>
+__device__ __forceinline__ void pair_suffix_coeffs(int pr, double Q2, double &acc, double *T)
+{
+    if constexpr (J <= 7) {
+        T[J - 1] = (pr < J) ? acc : 0.0;
+        const double e = row_bcast<2 * J>(Q2);
+        if (pr < J) acc *= e;
+        pair_suffix_coeffs<J + 1>(pr, Q2, acc, T);
     }
 }
 
@@ -656,7 +776,27 @@ __device__ __forceinline__ void pm_row_scan(int gl, int rl, double &m00, double 
 template <int R, int G>
 __device__ __forceinline__ void group_coeffs(int gl, double A, double Bq, Factor<R, G> &F)
 {
-    scan_coeffs<G, 0>(gl, (int)(threadIdx.x & 15), A, Bq, F);
+    using FT = Factor<R, G>;
+    const int rl = (int)(threadIdx.x & 15);
+    scan_coeffs<FT::HS, 0, R, G>(FT::ROW ? (rl & (FT::HS - 1)) : gl, A, Bq, F);
+    if constexpr (FT::ROW && FT::HS == 4) {
+        F.Ta[0] = A;
+        F.Tq[0] = Bq;
+        if constexpr (G > 16) {
+            const double a3 = row_bcast<3>(A), a7 = row_bcast<7>(A), a11 = row_bcast<11>(A);
+            const double q4 = row_bcast<4>(Bq), q8 = row_bcast<8>(Bq), q12 = row_bcast<12>(Bq);
+            if (rl >= 4) A *= a3;
+            if (rl >= 8) A *= a7;
+            if (rl >= 12) A *= a11;
+            if (rl < 12) Bq *= q12;
+            if (rl < 8) Bq *= q8;
+            if (rl < 4) Bq *= q4;
+        }
+    } else if constexpr (FT::ROW) {
+        const double A2 = A, Q2 = Bq;
+        pair_prefix_coeffs<6>(rl >> 1, A2, A, F.Ta);
+        pair_suffix_coeffs<1>(rl >> 1, Q2, Bq, F.Tq);
+    }
     // two-row groups: the carry multiplier is used in rows 1 and 3 only
     F.PA = (G == 32 && !((threadIdx.x >> 4) & 1)) ? 0.0 : A;
     F.PQ = Bq;
@@ -754,7 +894,7 @@ __device__ __forceinline__ void factorize(int gl, const double (&sv)[R], Factor<
 {
     double cprev = pivot_in<R, G>(gl, F.al, F.iv, F.g);
     bool ok = true;
-    double A = 1.0, Bq = 1.0;
+    double A = 1.0, Bq = 1.0, K = 0.0;
 #pragma unroll
     for (int k = 0; k < R; ++k) {
         const double a = F.al[k], b = F.iv[k], c = F.g[k];
@@ -770,9 +910,11 @@ __device__ __forceinline__ void factorize(int gl, const double (&sv)[R], Factor<
         if constexpr (!NOSRC) F.vs[k] = inv * sv[k];
         F.g[k] = -cp;
         A *= F.al[k];
+        if constexpr (Factor<R, G>::OVERLAP) K = fma(Bq, A, K);
         Bq *= F.g[k];
         cprev = cp;
     }
+    F.K = K;
     if (!ok) bad |= ERR_PIVOT;
     group_coeffs(gl, A, Bq, F);
 }
@@ -804,7 +946,10 @@ __device__ __forceinline__ void scan_bwd(const double *Qb, double &B)
 template <int R, int G>
 __device__ __forceinline__ double group_prefix(const Factor<R, G> &F, double L)
 {
-    scan_fwd<G, 0, Factor<R, G>::LV>(F.Af, L);
+    using FT = Factor<R, G>;
+    scan_fwd<G, 0, FT::LV>(F.Af, L);
+    if constexpr (FT::ROW && FT::HS == 4) L = bcast_prefix4(L, F.Ta[0]);
+    else if constexpr (FT::ROW) L = bcast_prefix2(L, F.Ta);
     if constexpr (G == 32) {
         // rows 1 and 3 continue the groups begun in rows 0 and 2: they take
         // the inclusive value at the last lane of the row before (PA is 0 in
@@ -827,7 +972,10 @@ __device__ __forceinline__ double group_prefix(const Factor<R, G> &F, double L)
 template <int R, int G>
 __device__ __forceinline__ double group_suffix(const Factor<R, G> &F, double M)
 {
-    scan_bwd<G, 0, Factor<R, G>::LV>(F.Qb, M);
+    using FT = Factor<R, G>;
+    scan_bwd<G, 0, FT::LV>(F.Qb, M);
+    if constexpr (FT::ROW && FT::HS == 4) M = bcast_suffix4(M, F.Tq[0]);
+    else if constexpr (FT::ROW) M = bcast_suffix2(M, F.Tq);
     if constexpr (G == 32) {
         // rows 0 and 2 take the value at the first lane of the row after:
         // the wave-uniform values at lanes 16 and 48 times multipliers that
@@ -848,6 +996,13 @@ __device__ __forceinline__ double group_suffix(const Factor<R, G> &F, double M)
 
 // One implicit substep: x <- M^{-1} (x + src) for the group, in place.
 // NOSRC: a run without sources (src = 0; vs is not formed).
+// Each lane reduces its rows to the affine map from the value entering it, a
+// scan across the lanes gives those values, and the rows' recurrences run
+// from them; forward, then backward: five operations a row and two scans.
+// OVERLAP: the lane's back substitution reduces the local forward values
+// (no carry yet), which does not wait for the forward scan; the entering
+// carry c then adds K c to it.  The reduction fills the scan's wait states,
+// and the rows' forward recurrences those of the backward scan.
 template <int R, int G, bool NOSRC = false>
 __device__ __forceinline__ void apply_solve(int gl, const Factor<R, G> &F, double (&x)[R])
 {
@@ -855,24 +1010,42 @@ __device__ __forceinline__ void apply_solve(int gl, const Factor<R, G> &F, doubl
     // the lane-local prefixes start from the first row itself (al * 0 + t is
     // t exactly for the finite multipliers of a factorised run)
     t[0] = NOSRC ? F.iv[0] * x[0] : fma(F.iv[0], x[0], F.vs[0]);
-    double L = t[0];
+    double L = t[0], M = 0.0;
+    if constexpr (Factor<R, G>::OVERLAP) {
+        double l[R];
+        l[0] = L;
 #pragma unroll
-    for (int k = 1; k < R; ++k) {
-        t[k] = NOSRC ? F.iv[k] * x[k] : fma(F.iv[k], x[k], F.vs[k]);
-        L = fma(F.al[k], L, t[k]);
+        for (int k = 1; k < R; ++k) {
+            t[k] = NOSRC ? F.iv[k] * x[k] : fma(F.iv[k], x[k], F.vs[k]);
+            L = fma(F.al[k], L, t[k]);
+            l[k] = L;
+        }
+        M = L;
+#pragma unroll
+        for (int k = R - 2; k >= 0; --k) M = fma(F.g[k], M, l[k]);
+    } else {
+#pragma unroll
+        for (int k = 1; k < R; ++k) {
+            t[k] = NOSRC ? F.iv[k] * x[k] : fma(F.iv[k], x[k], F.vs[k]);
+            L = fma(F.al[k], L, t[k]);
+        }
     }
     L = group_prefix(F, L);
     // the first lane of the group multiplies the shifted-in value by al[0] = 0
+    // (K, too, has it as a factor)
     double d = wave_up1(L);
+    if constexpr (Factor<R, G>::OVERLAP) M = group_suffix(F, fma(F.K, d, M));
 #pragma unroll
     for (int k = 0; k < R; ++k) {
         d = fma(F.al[k], d, t[k]);
         t[k] = d;
     }
-    double M = t[R - 1];
+    if constexpr (!Factor<R, G>::OVERLAP) {
+        M = t[R - 1];
 #pragma unroll
-    for (int k = R - 2; k >= 0; --k) M = fma(F.g[k], M, t[k]);
-    M = group_suffix(F, M);
+        for (int k = R - 2; k >= 0; --k) M = fma(F.g[k], M, t[k]);
+        M = group_suffix(F, M);
+    }
     // the group's last row has g = 0 (the system's last row), so the value
     // shifted in from the lane after drops out without a select
     double xn = wave_dn1(M);
@@ -1575,6 +1748,12 @@ __device__ __forceinline__ void k_fused_body(const CkGrid &g, const CkSlot *__re
         // zero, so every lane must hold finite values of a real tracer, not
         // registers that were never written in this launch
         const bool idle = tid >= ntasks;
+        // the costliest tasks (taken first) issue ahead of the wave they share
+        // a SIMD with: the launch ends with the longest of them
+        if (tbase < ntasks / 8) __builtin_amdgcn_s_setprio(3);
+        else if (tbase < ntasks / 4) __builtin_amdgcn_s_setprio(2);
+        else if (tbase < ntasks / 2) __builtin_amdgcn_s_setprio(1);
+        else __builtin_amdgcn_s_setprio(0);
         {
             const CkTask task = tasks[idle ? tbase : tid];
             const CkSlot &S0 = slots[task.slot];
