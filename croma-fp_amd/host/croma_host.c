@@ -156,7 +156,8 @@ struct CromaHipContext {
     void *stream_e; /* split windows: the electron pass, beside the next window's proton pass */
     int *d_counter;
     int *d_err;
-    CromaHipTile tile[2]; /* [protons] */
+    CromaHipTile tile[2]; /* [protons]; used once set (set_tile, autotuners), else by size (run_tile) */
+    int tile_set[2];
     pthread_mutex_t ic_lock;
     struct {
         int valid;
@@ -186,7 +187,7 @@ struct CromaHipContext {
     int pws_cap;
     /* window launches replayed as hipGraphs */
     int use_graphs;
-    int pipeline; /* split windows: electron pass beside the next proton pass */
+    int pipeline; /* split windows: electron pass beside the next proton pass; -1: by size */
     /* batch runs estimate nsub and order the queue on the device */
     int nsub_device;
     /* coefficient evaluation in FP32 (losses, D_pp, B, C, face inputs) feeding
@@ -303,6 +304,60 @@ static void default_tiles(CromaHipContext *c)
     c->tile[1].secondary_gemm = 1;
 }
 
+/* Whether every fused launch mode a tile runs has an FP32-coefficient
+ * instance (electrons: mode 0; two species: the split passes 2 and 3, or the
+ * in-kernel contraction 1, which the eta cap also selects). */
+static int tile_f32_ok(const CromaHipContext *c, int protons, int r, int w, int g)
+{
+    const int n = c->g.n;
+    if (!protons) return ck_fused_f32_supported(n, r, w, 0);
+    if (!g || c->prm.eta_dpp_cap > 0.0) return ck_fused_f32_supported(n, r, w, 1);
+    return ck_fused_f32_supported(n, r, w, 2) && ck_fused_f32_supported(n, r, w, 3);
+}
+
+/* Rows (tracers x bins) up to which a launch waits for its costliest tracers
+ * rather than for the sum of the work, and the two passes of split windows
+ * run beside each other with gain. */
+#define CH_ROWS_LATENCY (1L << 20)
+#define CH_ROWS_MIDDLE (6L << 20)
+#define CH_ROWS_PIPE (3L << 20)
+
+/* The tile of a run of `run` snapshots of ntr tracers: the one set, or by
+ * size.  Small launches end with their costliest tracers' substep chain, so
+ * they take the fewest rows per lane that the scan's latency allows, one wave
+ * per SIMD, and (electrons, in-kernel secondaries: one launch per window) all
+ * the run's snapshots in one window, whose tasks wait for that chain once
+ * instead of once per snapshot.  Large ones take the rows per lane with the
+ * fewest instructions per row.  Measured, best against the default by n alone
+ * in us (four to ten snapshots): e 256 x 64 1781 / 2358, 1,024 x 128 2776 /
+ * 4083, 6,000 x 128 4104 / 5469, 16,000 x 128 2520 / 2860, 32,000 x 128 3245 /
+ * 4619, 32,000 x 256 5770 / 6744, 60,000 x 64 3126 / 4183; both species,
+ * split 2,000 x 256 5373 / 6599 (pipelined 3932), 300 x 512 7243 / 8300
+ * (pipelined 5305). */
+static CromaHipTile run_tile(const CromaHipContext *c, int protons, long ntr, int run)
+{
+    const int n = c->g.n, p = protons ? 1 : 0;
+    const long rows = ntr * (long)n;
+    const int split = p && c->tile[1].secondary_gemm && !(c->prm.dpp_model != 3 && c->prm.eta_dpp_cap > 0.0);
+    CromaHipTile t = c->tile[p];
+    if (c->tile_set[p]) return t;
+    if (!p) {
+        if (n == 64) t.rows_per_lane = rows <= CH_ROWS_LATENCY ? 4 : 8;
+        else if (n <= 256) t.rows_per_lane = (n == 128 && rows <= CH_ROWS_LATENCY) ? 4 : rows <= CH_ROWS_MIDDLE ? 8 : 16;
+        t.waves_per_simd = (n <= 128 && rows <= CH_ROWS_LATENCY) ? 1 : 2;
+    } else if (split) {
+        t.rows_per_lane = n <= 128 ? 4 : n == 256 ? 8 : 16;
+        t.waves_per_simd = (n == 512 || (n <= 128 && rows <= CH_ROWS_LATENCY)) ? 1 : 2;
+    } else {
+        t.rows_per_lane = n == 64 ? 2 : n <= 256 ? 4 : 8;
+        t.waves_per_simd = 2;
+    }
+    if (c->coeff_fp32 && !tile_f32_ok(c, p, t.rows_per_lane, t.waves_per_simd, t.secondary_gemm)) t = c->tile[p];
+    /* a window's schedule buffers are bounded by 16 snapshots of 65,536 tracers */
+    if (!split && ntr <= 65536) t.chain = run < 16 ? run : 16;
+    return t;
+}
+
 static int tile_ok(int n, const CromaHipTile *t)
 {
     return ck_fused_supported(n, t->rows_per_lane) && t->waves_per_simd >= 1 && t->waves_per_simd <= 2 &&
@@ -357,7 +412,7 @@ CromaHipContext *croma_hip_context_create(const CromaHipGridSpec *gs, const Crom
     }
     default_tiles(c);
     c->use_graphs = 1;
-    c->pipeline = 0;
+    c->pipeline = -1;
     c->nsub_device = 1;
     return c;
 }
@@ -429,8 +484,8 @@ int croma_hip_context_set_tile(CromaHipContext *c, int protons, const CromaHipTi
 {
     if (!c || !t || protons < -1 || protons > 1) return CROMA_HIP_EINVAL;
     if (!tile_ok(c->g.n, t)) return CROMA_HIP_EUNSUPPORTED;
-    if (protons != 1) c->tile[0] = *t;
-    if (protons != 0) c->tile[1] = *t;
+    if (protons != 1) c->tile[0] = *t, c->tile_set[0] = 1;
+    if (protons != 0) c->tile[1] = *t, c->tile_set[1] = 1;
     return 0;
 }
 
@@ -534,30 +589,46 @@ int croma_hip_ic_cooling_rows_device(CromaHipContext *c, int nz, const double *z
     return rc;
 }
 
-/* IC cooling rate at the first and last electron bins at z (cached). */
-void ch_ctx_ic_ends(CromaHipContext *c, double z, double ends[2])
+static int ic_ends_find(CromaHipContext *c, double z, double ends[2])
 {
-    int k, bins[2];
-    pthread_mutex_lock(&c->ic_lock);
+    int k;
     for (k = 0; k < CH_IC_ENDS; k++)
         if (c->ic_end[k].valid && c->ic_end[k].z == z) {
-            ends[0] = c->ic_end[k].v[0];
-            ends[1] = c->ic_end[k].v[1];
-            pthread_mutex_unlock(&c->ic_lock);
-            return;
+            if (ends) memcpy(ends, c->ic_end[k].v, sizeof(c->ic_end[k].v));
+            return 1;
         }
-    pthread_mutex_unlock(&c->ic_lock);
-    bins[0] = 0;
-    bins[1] = c->g.n - 1;
-    ch_ic_cooling_bins(&c->g, z, 2, bins, ends);
-    pthread_mutex_lock(&c->ic_lock);
-    k = c->ic_end_next;
-    c->ic_end_next = (k + 1) % CH_IC_ENDS;
-    c->ic_end[k].z = z;
-    c->ic_end[k].v[0] = ends[0];
-    c->ic_end[k].v[1] = ends[1];
-    c->ic_end[k].valid = 1;
-    pthread_mutex_unlock(&c->ic_lock);
+    return 0;
+}
+
+/* IC cooling rates at the first and last electron bins at nz redshifts,
+ * ends[2 q], ends[2 q + 1] (cached).  Those not cached yet are evaluated side
+ * by side on the host threads: one takes half a millisecond, and a run's
+ * first pass needs one per snapshot before its first window is launched. */
+void ch_ctx_ic_ends(CromaHipContext *c, int nz, const double *z, double *ends)
+{
+    double zn[CH_IC_ENDS], v[2 * CH_IC_ENDS];
+    int q, k, first = 0;
+    while (first < nz) {
+        int m = 0, last;
+        pthread_mutex_lock(&c->ic_lock);
+        for (last = first; last < nz && m < CH_IC_ENDS; last++)
+            if (!ic_ends_find(c, z[last], ends + 2 * last)) zn[m++] = z[last];
+        pthread_mutex_unlock(&c->ic_lock);
+        if (m) ch_ic_cooling_ends(&c->g, m, zn, v);
+        pthread_mutex_lock(&c->ic_lock);
+        for (k = 0; k < m; k++) {
+            for (q = first; q < last; q++)
+                if (z[q] == zn[k]) memcpy(ends + 2 * q, v + 2 * k, 2 * sizeof(double));
+            if (ic_ends_find(c, zn[k], 0)) continue;
+            q = c->ic_end_next;
+            c->ic_end_next = (q + 1) % CH_IC_ENDS;
+            c->ic_end[q].z = zn[k];
+            memcpy(c->ic_end[q].v, v + 2 * k, sizeof(c->ic_end[q].v));
+            c->ic_end[q].valid = 1;
+        }
+        pthread_mutex_unlock(&c->ic_lock);
+        first = last;
+    }
 }
 
 int croma_hip_ic_cooling_row(const CromaHipContext *cc, double z, double *row, double *m1, double *p1)
@@ -707,7 +778,7 @@ const ChGrid *ch_ctx_grid(const CromaHipContext *c) { return &c->g; }
 const CkGrid *ch_ctx_dgrid(const CromaHipContext *c) { return &c->dgrid; }
 const CkParams *ch_ctx_prm(const CromaHipContext *c) { return &c->prm; }
 int ch_ctx_cu_count(const CromaHipContext *c) { return c->cu_count; }
-CromaHipTile ch_ctx_tile(const CromaHipContext *c, int protons) { return c->tile[protons ? 1 : 0]; }
+CromaHipTile ch_ctx_tile(const CromaHipContext *c, int protons, long ntr) { return run_tile(c, protons, ntr, 1); }
 const double *ch_ctx_d_fqe(const CromaHipContext *c) { return c->d_fqe; }
 /* np_min of the secondary weights on the device (after the weights and beta_p) */
 const int *ch_ctx_d_npmin(const CromaHipContext *c) { return c->d_fqe ? (const int *)(c->d_fqe + (size_t)c->g.n * c->g.n + c->g.n) : 0; }
@@ -818,6 +889,8 @@ static void graph_reset(CromaHipContext *c, ChGraph *g)
  * sets alternate so the host prepares window w+1 while the GPU runs w. */
 typedef struct {
     int cap;          /* snapshots the buffers hold */
+    int host;         /* the pinned schedule buffers exist */
+    void *d_mem, *h_mem;
     int *d_nsub, *d_non;
     CkTask *d_tasks;
     CkSlot *d_slot;
@@ -850,6 +923,8 @@ struct CromaHipBatch {
     double *h_bg;  /* host copy for nsub */
     double *d_src; /* optional [nsnap_res][2][ntr*n] per-snapshot sources */
     unsigned char *src_set;
+    CromaHipTile tile; /* of the run under way */
+    int pipe;          /* split windows of the run under way are pipelined */
     WinBuf win[2];
     double *d_segrec, *d_seginje; /* split launches: [segrows_cap][n] */
     long segrows_cap;
@@ -873,58 +948,61 @@ static void win_free(CromaHipContext *c, WinBuf *w)
     graph_reset(c, &w->graph);
     graph_reset(c, &w->graph_g);
     graph_reset(c, &w->graph_e);
-    ck_free(w->d_nsub);
-    ck_free(w->d_non);
-    ck_free(w->d_tasks);
-    ck_free(w->d_slot);
-    ck_free(w->d_segoff);
-    ck_free(w->d_key);
-    ck_free(w->d_segloc);
-    ck_free(w->d_blk);
-    ck_free(w->d_hist);
-    ck_host_free(w->h_segoff);
-    ck_host_free(w->h_nsub);
-    ck_host_free(w->h_non);
-    ck_host_free(w->h_tasks);
-    ck_host_free(w->h_slot);
+    ck_free(w->d_mem);
+    ck_host_free(w->h_mem);
     ck_event_destroy(w->ev_up);
     ck_event_destroy(w->ev_g);
     ck_event_destroy(w->ev_e);
     memset(w, 0, sizeof(*w));
 }
 
-static int win_reserve(CromaHipContext *c, WinBuf *w, int cap, int ntr)
+/* Buffers of a window of cap snapshots, one device and one pinned allocation;
+ * host: also the pinned schedule (nsub, tasks, segment rows) of windows that
+ * are ordered on the host. */
+static int win_reserve(CromaHipContext *c, WinBuf *w, int cap, int ntr, int host)
 {
-    if (w->cap >= cap) return 0;
+#define WIN_UP(x) (((size_t)(x) + 255) & ~(size_t)255)
+    const size_t sched = WIN_UP((size_t)cap * ntr * sizeof(int)), tasks = WIN_UP((size_t)ntr * sizeof(CkTask));
+    const size_t slots = WIN_UP((size_t)cap * sizeof(CkSlot)), each = WIN_UP((size_t)ntr * sizeof(int));
+    const size_t blk = WIN_UP(((size_t)ntr / 256 + 2) * sizeof(int)), hist = WIN_UP(CK_NSUB_HIST * sizeof(int));
+    char *p;
+    if (w->cap >= cap && w->host >= host) return 0;
     if (w->ev_up) ck_event_sync(w->ev_up);
     ck_stream_sync(c->stream);
     if (c->stream_e) ck_stream_sync(c->stream_e);
+    if (w->host > host) host = w->host;
     win_free(c, w);
-    w->d_nsub = (int *)ck_malloc((size_t)cap * ntr * sizeof(int));
-    w->d_non = (int *)ck_malloc((size_t)cap * ntr * sizeof(int));
-    w->d_tasks = (CkTask *)ck_malloc((size_t)ntr * sizeof(CkTask));
-    w->d_slot = (CkSlot *)ck_malloc((size_t)cap * sizeof(CkSlot));
-    w->h_nsub = (int *)ck_host_alloc((size_t)cap * ntr * sizeof(int));
-    w->h_non = (int *)ck_host_alloc((size_t)cap * ntr * sizeof(int));
-    w->h_tasks = (CkTask *)ck_host_alloc((size_t)ntr * sizeof(CkTask));
-    w->h_slot = (CkSlot *)ck_host_alloc((size_t)cap * sizeof(CkSlot));
-    w->d_segoff = (int *)ck_malloc((size_t)cap * ntr * sizeof(int));
-    w->h_segoff = (int *)ck_host_alloc((size_t)cap * ntr * sizeof(int));
-    w->d_key = (int *)ck_malloc((size_t)ntr * sizeof(int));
-    w->d_segloc = (int *)ck_malloc((size_t)ntr * sizeof(int));
-    w->d_blk = (int *)ck_malloc(((size_t)ntr / 256 + 2) * sizeof(int));
-    w->d_hist = (int *)ck_malloc((size_t)CK_NSUB_HIST * sizeof(int));
+    w->d_mem = ck_malloc(3 * sched + tasks + slots + 2 * each + blk + hist);
+    w->h_mem = ck_host_alloc(slots + (host ? 3 * sched + tasks : 0));
     w->ev_up = ck_event_create();
     w->ev_g = ck_event_create();
     w->ev_e = ck_event_create();
-    if (!w->d_nsub || !w->d_non || !w->d_tasks || !w->d_slot || !w->h_nsub || !w->h_non ||
-        !w->h_tasks || !w->h_slot || !w->ev_up || !w->ev_g || !w->ev_e || !w->d_segoff || !w->h_segoff ||
-        !w->d_key || !w->d_segloc || !w->d_blk || !w->d_hist) {
+    if (!w->d_mem || !w->h_mem || !w->ev_up || !w->ev_g || !w->ev_e) {
         win_free(c, w);
         return dev_fail("window buffers");
     }
+    p = (char *)w->d_mem;
+    w->d_nsub = (int *)p;
+    w->d_non = (int *)(p += sched);
+    w->d_segoff = (int *)(p += sched);
+    w->d_tasks = (CkTask *)(p += sched);
+    w->d_slot = (CkSlot *)(p += tasks);
+    w->d_key = (int *)(p += slots);
+    w->d_segloc = (int *)(p += each);
+    w->d_blk = (int *)(p += each);
+    w->d_hist = (int *)(p += blk);
+    p = (char *)w->h_mem;
+    w->h_slot = (CkSlot *)p;
+    if (host) {
+        w->h_nsub = (int *)(p += slots);
+        w->h_non = (int *)(p += sched);
+        w->h_segoff = (int *)(p += sched);
+        w->h_tasks = (CkTask *)(p += sched);
+    }
     w->cap = cap;
+    w->host = host;
     return 0;
+#undef WIN_UP
 }
 
 void croma_hip_batch_destroy(CromaHipBatch *b)
@@ -995,7 +1073,7 @@ CromaHipBatch *croma_hip_batch_create(CromaHipContext *c, int ntr, int species, 
         !b->ev_a || !b->ev_b || !b->d_cells)
         goto fail;
     for (k = 0; k < 2; k++)
-        if (win_reserve(c, &b->win[k], 1, ntr)) goto fail;
+        if (win_reserve(c, &b->win[k], run_tile(c, b->protons, ntr, nsnap_res).chain, ntr, 0)) goto fail;
     if (b->protons && ch_ctx_fqe(c) != 0) goto fail;
     return b;
 fail:
@@ -1164,7 +1242,7 @@ static int prepare_window(CromaHipBatch *b, WinBuf *w, int s_first, int count, i
         const int al = (s + 1 < nsnap_total) ? 1 : 0;
         const int sn = (s + 1 < b->nsnap_res && al) ? s + 1 : s;
         const double *hb = b->h_bg + (size_t)s * CK_NBG * ntr;
-        int *nsub = w->h_nsub + (size_t)q * ntr, *non = w->h_non + (size_t)q * ntr;
+        int *nsub = dev_nsub ? 0 : w->h_nsub + (size_t)q * ntr, *non = dev_nsub ? 0 : w->h_non + (size_t)q * ntr;
         CkSlot *S = &w->h_slot[q];
         double ends[2];
         if (al && s + 1 >= b->nsnap_res) {
@@ -1174,7 +1252,7 @@ static int prepare_window(CromaHipBatch *b, WinBuf *w, int s_first, int count, i
         }
         allow_v[q] = al;
         t0 = ch_now_s();
-        ch_ctx_ic_ends(c, z[s], ends);
+        ch_ctx_ic_ends(c, 1, z + s, ends);
         ps->ic_ms += 1e3 * (ch_now_s() - t0);
         if (!dev_nsub) {
             t0 = ch_now_s();
@@ -1218,12 +1296,13 @@ static int prepare_window(CromaHipBatch *b, WinBuf *w, int s_first, int count, i
         S->ric_lo = ends[0];
         S->ric_hi = ends[1];
         if (split) {
-            int *off = w->h_segoff + (size_t)q * ntr;
-            if (!dev_nsub)
+            if (!dev_nsub) {
+                int *off = w->h_segoff + (size_t)q * ntr;
                 for (i = 0; i < ntr; i++) {
                     off[i] = (int)w->segrows;
                     w->segrows += ch_choose_segments(&c->prm, nsub[i], al);
                 }
+            }
             S->seg_off = w->d_segoff + (size_t)q * ntr;
             S->seg_rec = b->d_segrec;
             S->seg_inje = b->d_seginje;
@@ -1307,10 +1386,9 @@ static int upload_window(CromaHipBatch *b, WinBuf *w)
  * waves), or half of it when it runs beside the other species' pass of the
  * neighbouring window; the two passes then take their tasks from separate
  * queue counters. */
-static int launch_mode(CromaHipContext *c, int protons, int mode, const CkSlot *d_slot, const CkTask *d_tasks,
-                       int ntasks, int shared, int *counter, void *stream)
+static int launch_mode(CromaHipContext *c, const CromaHipTile *t, int mode, const CkSlot *d_slot,
+                       const CkTask *d_tasks, int ntasks, int shared, int *counter, void *stream)
 {
-    const CromaHipTile *t = &c->tile[protons ? 1 : 0];
     const int nfull = c->cu_count * t->waves_per_simd;
     const int nblocks = shared ? (nfull + 1) / 2 : nfull;
     if (c->coeff_fp32 && !ck_fused_f32_supported(c->g.n, t->rows_per_lane, t->waves_per_simd, mode)) {
@@ -1328,10 +1406,10 @@ static int launch_mode(CromaHipContext *c, int protons, int mode, const CkSlot *
 
 /* nosrc: an electron_only launch whose slots have no source rows (the
  * instance without source terms; the same results) */
-static int launch_tasks(CromaHipContext *c, int protons, int nosrc, const CkSlot *d_slot, const CkTask *d_tasks,
-                        int ntasks)
+static int launch_tasks(CromaHipContext *c, const CromaHipTile *t, int protons, int nosrc, const CkSlot *d_slot,
+                        const CkTask *d_tasks, int ntasks)
 {
-    return launch_mode(c, protons, protons ? 1 : (nosrc ? CK_LAUNCH_NOSRC : 0), d_slot, d_tasks, ntasks, 0,
+    return launch_mode(c, t, protons ? 1 : (nosrc ? CK_LAUNCH_NOSRC : 0), d_slot, d_tasks, ntasks, 0,
                        c->d_counter, c->stream);
 }
 
@@ -1361,9 +1439,9 @@ static int launch_gemm(CromaHipBatch *b, WinBuf *w)
 static int launch_split(CromaHipBatch *b, WinBuf *w)
 {
     CromaHipContext *c = b->ctx;
-    int rc = launch_mode(c, 1, 2, w->d_slot, w->d_tasks, b->ntr, 0, c->d_counter, c->stream);
+    int rc = launch_mode(c, &b->tile, 2, w->d_slot, w->d_tasks, b->ntr, 0, c->d_counter, c->stream);
     if (!rc) rc = launch_gemm(b, w);
-    if (!rc) rc = launch_mode(c, 1, 3, w->d_slot, w->d_tasks, b->ntr, 0, c->d_counter, c->stream);
+    if (!rc) rc = launch_mode(c, &b->tile, 3, w->d_slot, w->d_tasks, b->ntr, 0, c->d_counter, c->stream);
     return rc;
 }
 
@@ -1383,9 +1461,10 @@ static int issue_window(void *arg)
     if (w->dev_nsub && ck_nsub_order(c->dgrid, w->d_slot, w->count, b->ntr, b->protons, w->split, w->d_tasks,
                                      w->d_key, w->d_segloc, w->d_blk, w->d_hist, b->d_cells, c->stream))
         return dev_fail("device nsub");
-    if (wi->pipe) return launch_mode(c, 1, 2, w->d_slot, w->d_tasks, b->ntr, wi->shared, c->d_counter, c->stream);
+    if (wi->pipe)
+        return launch_mode(c, &b->tile, 2, w->d_slot, w->d_tasks, b->ntr, wi->shared, c->d_counter, c->stream);
     if (w->split) return launch_split(b, w);
-    return launch_tasks(c, b->protons, w->nosrc, w->d_slot, w->d_tasks, b->ntr);
+    return launch_tasks(c, &b->tile, b->protons, w->nosrc, w->d_slot, w->d_tasks, b->ntr);
 }
 
 static int issue_gemm(void *arg)
@@ -1398,15 +1477,15 @@ static int issue_epass(void *arg)
 {
     WinIssue *wi = (WinIssue *)arg;
     CromaHipContext *c = wi->b->ctx;
-    return launch_mode(c, 1, 3, wi->w->d_slot, wi->w->d_tasks, wi->b->ntr, wi->shared, c->d_counter + CH_CTR_E,
+    return launch_mode(c, &wi->b->tile, 3, wi->w->d_slot, wi->w->d_tasks, wi->b->ntr, wi->shared, c->d_counter + CH_CTR_E,
                        c->stream_e);
 }
 
 static int launch_window(CromaHipBatch *b, WinBuf *w, WinBuf *prev, int last, GraphStats *gs)
 {
     CromaHipContext *c = b->ctx;
-    const CromaHipTile *t = &c->tile[b->protons ? 1 : 0];
-    const int pipe = w->split && c->pipeline;
+    const CromaHipTile *t = &b->tile;
+    const int pipe = w->split && b->pipe;
     WinIssue wi;
     long key[CH_GKEY];
     int rc;
@@ -1676,6 +1755,31 @@ int croma_hip_batch_sync(CromaHipBatch *b)
     return 0;
 }
 
+/* Segment rows of a window of wsz snapshots (split launches). */
+static int reserve_segrows(CromaHipBatch *b, int wsz)
+{
+    CromaHipContext *c = b->ctx;
+    const long segmax = c->prm.coeff_interp_max_segments > 1 ? c->prm.coeff_interp_max_segments : 1;
+    long need = (long)wsz * b->ntr * segmax, q = 256;
+    while (q < need / 64) q <<= 1;
+    need = (need + q - 1) / q * q;
+    if (need > b->segrows_cap) {
+        const size_t cnt = (size_t)need * c->g.n;
+        ck_stream_sync(c->stream);
+        ck_free(b->d_segrec);
+        ck_free(b->d_seginje);
+        b->d_segrec = (double *)ck_malloc(cnt * sizeof(double));
+        b->d_seginje = (double *)ck_malloc(cnt * sizeof(double));
+        b->segrows_cap = (b->d_segrec && b->d_seginje) ? need : 0;
+        if (!b->segrows_cap) return dev_fail("segment rows");
+        /* rows past a window's segment count enter the rounded GEMM: keep them finite */
+        if (ck_fill_f64(b->d_segrec, 0.0, cnt, c->stream) || ck_fill_f64(b->d_seginje, 0.0, cnt, c->stream))
+            return dev_fail("segment rows");
+    }
+    b->seg_quantum = q;
+    return 0;
+}
+
 int croma_hip_batch_run(CromaHipBatch *b, int s0, int s1, int nsnap_total, const double *z, const double *dt_snap,
                         double elapsed, int path, CromaHipTimes *times)
 {
@@ -1691,36 +1795,19 @@ int croma_hip_batch_run(CromaHipBatch *b, int s0, int s1, int nsnap_total, const
         return CROMA_HIP_EINVAL;
     if (s1 == s0) return 0;
     c = b->ctx;
-    wsz = (path == CROMA_HIP_PATH_FUSED) ? c->tile[b->protons ? 1 : 0].chain : 1;
+    b->tile = run_tile(c, b->protons, b->ntr, s1 - s0);
+    b->pipe = c->pipeline < 0 ? (long)b->ntr * c->g.n <= CH_ROWS_PIPE : c->pipeline;
+    wsz = (path == CROMA_HIP_PATH_FUSED) ? b->tile.chain : 1;
     if (wsz > s1 - s0) wsz = s1 - s0;
     /* the split launches need the species decoupled within a segment: no eta cap */
-    split = path == CROMA_HIP_PATH_FUSED && b->protons && c->tile[1].secondary_gemm &&
+    split = path == CROMA_HIP_PATH_FUSED && b->protons && b->tile.secondary_gemm &&
             !(c->prm.dpp_model != 3 && c->prm.eta_dpp_cap > 0.0);
     /* the plain path keeps the reference's host-side buckets */
     dev_nsub = path == CROMA_HIP_PATH_FUSED && c->nsub_device;
-    if (split) {
-        const long segmax = c->prm.coeff_interp_max_segments > 1 ? c->prm.coeff_interp_max_segments : 1;
-        long need = (long)wsz * b->ntr * segmax, q = 256;
-        while (q < need / 64) q <<= 1;
-        need = (need + q - 1) / q * q;
-        if (need > b->segrows_cap) {
-            const size_t cnt = (size_t)need * c->g.n;
-            ck_stream_sync(c->stream);
-            ck_free(b->d_segrec);
-            ck_free(b->d_seginje);
-            b->d_segrec = (double *)ck_malloc(cnt * sizeof(double));
-            b->d_seginje = (double *)ck_malloc(cnt * sizeof(double));
-            b->segrows_cap = (b->d_segrec && b->d_seginje) ? need : 0;
-            if (!b->segrows_cap) return dev_fail("segment rows");
-            /* rows past a window's segment count enter the rounded GEMM: keep them finite */
-            if (ck_fill_f64(b->d_segrec, 0.0, cnt, c->stream) || ck_fill_f64(b->d_seginje, 0.0, cnt, c->stream))
-                return dev_fail("segment rows");
-        }
-        b->seg_quantum = q;
-    }
+    if (split && (rc = reserve_segrows(b, wsz)) != 0) return rc;
     nwin = (s1 - s0 + wsz - 1) / wsz;
     for (k = 0; k < 2; k++)
-        if ((rc = win_reserve(c, &b->win[k], wsz, b->ntr)) != 0) return rc;
+        if ((rc = win_reserve(c, &b->win[k], wsz, b->ntr, !dev_nsub)) != 0) return rc;
     if (path == CROMA_HIP_PATH_FUSED && b->ev_k_cap < 2 * nwin) {
         int need = 2 * nwin, j;
         void **ne = (void **)realloc(b->ev_k, (size_t)need * sizeof(void *));
@@ -1741,6 +1828,14 @@ int croma_hip_batch_run(CromaHipBatch *b, int s0, int s1, int nsnap_total, const
     if (ck_event_record(b->ev_a, c->stream)) return dev_fail("event");
     if (dev_nsub && ck_fill_i32((int *)b->d_cells, 0, 2, c->stream)) return dev_fail("cell counter");
     if ((rc = run_ic_rows(b, s0, s1, nsnap_total, z)) != 0) return rc;
+    /* the first window's, and in its shadow the others': a run's redshifts at once */
+    if (s1 - s0 > 1 && dev_nsub) {
+        double *ends = (double *)malloc((size_t)(s1 - s0) * 2 * sizeof(double));
+        const double t0 = ch_now_s();
+        if (ends) ch_ctx_ic_ends(c, s1 - s0 < CH_IC_ENDS / 2 ? s1 - s0 : CH_IC_ENDS / 2, z + s0, ends);
+        free(ends);
+        ps.ic_ms += 1e3 * (ch_now_s() - t0);
+    }
     rc = prepare_window(b, &b->win[0], s0, (s1 - s0 < wsz) ? s1 - s0 : wsz, nsnap_total, z, dt_snap, el, split,
                         dev_nsub, &ps);
     if (rc) return rc;
@@ -1801,12 +1896,44 @@ typedef struct {
     int protons, ntr;
     const CkSlot *d_slot;
     const CkTask *d_tasks;
+    /* split: proton pass, contraction of the rows counted at d_rows, electron pass */
+    const double *d_fqe;
+    const int *d_npmin, *d_rows;
 } XIssue;
 
 static int issue_tasks(void *arg)
 {
     XIssue *x = (XIssue *)arg;
-    return launch_tasks(x->c, x->protons, 0, x->d_slot, x->d_tasks, x->ntr);
+    CromaHipContext *c = x->c;
+    CromaHipBatch *b = c->xb;
+    int rc;
+    if (!x->d_rows) return launch_tasks(c, &b->tile, x->protons, 0, x->d_slot, x->d_tasks, x->ntr);
+    rc = launch_mode(c, &b->tile, 2, x->d_slot, x->d_tasks, x->ntr, 0, c->d_counter, c->stream);
+    if (!rc && ck_sec_contract(c->g.n, x->d_fqe, x->d_npmin, b->d_segrec, b->d_seginje, b->segrows_cap, x->d_rows,
+                               8 * c->cu_count, c->stream))
+        rc = dev_fail("secondary contraction");
+    if (!rc) rc = launch_mode(c, &b->tile, 3, x->d_slot, x->d_tasks, x->ntr, 0, c->d_counter, c->stream);
+    return rc;
+}
+
+/* First contributing proton row of every electron bin (at least jp0), as the
+ * contraction's launch wants it; returns 0 when the caller's weights have
+ * entries below jp0 in the rows the contraction would read (it starts at a
+ * multiple of 16), which the in-kernel sum leaves out. */
+static int snapshot_npmin(int n, int jp0, const double *fqe, int *first)
+{
+    int jp, je, open = n;
+    for (jp = jp0 & ~15; jp < jp0; jp++)
+        for (je = 0; je < n; je++)
+            if (fqe[(size_t)jp * n + je] != 0.0) return 0;
+    for (je = 0; je < n; je++) first[je] = n;
+    for (jp = jp0; jp < n && open; jp++)
+        for (je = 0; je < n; je++)
+            if (first[je] == n && fqe[(size_t)jp * n + je] != 0.0) {
+                first[je] = jp;
+                open--;
+            }
+    return 1;
 }
 
 /* ------------------------------------------------------------------ */
@@ -1837,6 +1964,7 @@ int croma_hip_execute_snapshot(
     double *d_ric = 0, *d_fqe = 0;
     CkParams prm;
     double ric2[2 * CH_NMAX]; /* staging of the caller's rows; read by the async upload before the final sync */
+    int npm[CH_NMAX + 1], *d_npm = 0, split = 0; /* first proton rows, and the segment row count */
     (void)z_curr;
     (void)z_next;
     if (!c || ntr <= 0 || !nsubsteps || !n_onsteps || !base_nsteps || !fp_cadence_steps || !rad_ic_zero ||
@@ -1882,6 +2010,7 @@ int croma_hip_execute_snapshot(
                                          2)))
         return CROMA_HIP_ENOMEM;
     b = c->xb;
+    if ((rc = win_reserve(c, &b->win[0], 1, ntr, 1)) != 0) return rc;
     rc = croma_hip_batch_set_state(b, protons ? crp : 0, cre, protons ? qpi : 0, qepri, mass, dis);
     if (!rc) rc = croma_hip_batch_set_background(b, 0, cur);
     if (!rc) rc = croma_hip_batch_set_background(b, 1, nxt);
@@ -1890,7 +2019,8 @@ int croma_hip_execute_snapshot(
     /* caller-provided schedule, IC rows and secondary weights */
     {
         const size_t need = (size_t)ntr * (2 * sizeof(int) + sizeof(CkTask)) + sizeof(CkSlot) +
-                            2 * (size_t)n * sizeof(double) + (size_t)n * n * sizeof(double) + 8192;
+                            2 * (size_t)n * sizeof(double) + (size_t)n * n * sizeof(double) +
+                            ((size_t)n + 1) * sizeof(int) + 8192;
         if (need > c->x_ws_bytes) {
             ck_stream_sync(c->stream);
             ck_graph_destroy(c->x_graph.exec);
@@ -1918,6 +2048,8 @@ int croma_hip_execute_snapshot(
         d_ric = (double *)p;
         p += ((2 * (size_t)n * sizeof(double)) + 255) & ~(size_t)255;
         d_fqe = (double *)p;
+        p += (((size_t)n * n * sizeof(double)) + 255) & ~(size_t)255;
+        d_npm = (int *)p;
     }
     {
         WinBuf *w = &b->win[0];
@@ -1958,7 +2090,27 @@ int croma_hip_execute_snapshot(
         S->dt_snap = dt_snap;
         S->elapsed = elapsed;
         S->prm = prm;
-        if (ck_h2d(d_nsub, w->h_nsub, (size_t)ntr * sizeof(int), c->stream) ||
+        /* two species without the eta cap: the split launch (a third to a half
+         * of the in-kernel contraction's time), when its instances exist */
+        b->tile = run_tile(c, protons, ntr, 1);
+        if (protons && b->tile.secondary_gemm && !(prm.dpp_model != 3 && prm.eta_dpp_cap > 0.0) &&
+            (!c->coeff_fp32 || tile_f32_ok(c, 1, b->tile.rows_per_lane, b->tile.waves_per_simd, 1)) &&
+            snapshot_npmin(n, jp0, fqe_flat, npm)) {
+            long segrows = 0;
+            if ((rc = reserve_segrows(b, 1)) != 0) goto done;
+            for (i = 0; i < ntr; i++) {
+                w->h_segoff[i] = (int)segrows;
+                segrows += ch_choose_segments(&prm, nsubsteps[i], allow);
+            }
+            npm[n] = (int)segrows;
+            S->seg_off = w->d_segoff;
+            S->seg_rec = b->d_segrec;
+            S->seg_inje = b->d_seginje;
+            split = 1;
+        }
+        if ((split && (ck_h2d(w->d_segoff, w->h_segoff, (size_t)ntr * sizeof(int), c->stream) ||
+                       ck_h2d(d_npm, npm, ((size_t)n + 1) * sizeof(int), c->stream))) ||
+            ck_h2d(d_nsub, w->h_nsub, (size_t)ntr * sizeof(int), c->stream) ||
             ck_h2d(d_non, w->h_non, (size_t)ntr * sizeof(int), c->stream) ||
             ck_h2d(d_tasks, w->h_tasks, (size_t)ntr * sizeof(CkTask), c->stream) ||
             ck_h2d(d_slot, S, sizeof(CkSlot), c->stream) ||
@@ -1968,22 +2120,27 @@ int croma_hip_execute_snapshot(
             goto done;
         }
         {
-            const CromaHipTile *t = &c->tile[protons ? 1 : 0];
+            const CromaHipTile *t = &b->tile;
             XIssue xi;
             GraphStats gst;
             long key[CH_GKEY];
             memset(key, 0, sizeof(key));
             memset(&gst, 0, sizeof(gst));
-            key[0] = protons;
+            key[0] = protons | (split << 1) | (c->coeff_fp32 << 2);
             key[1] = ntr;
             key[2] = t->rows_per_lane;
             key[3] = t->waves_per_simd;
             key[4] = (long)(size_t)d_ws;
+            key[5] = (long)(size_t)b->d_segrec;
+            key[6] = split ? b->segrows_cap : 0;
             xi.c = c;
             xi.protons = protons;
             xi.d_slot = d_slot;
             xi.d_tasks = d_tasks;
             xi.ntr = ntr;
+            xi.d_fqe = d_fqe;
+            xi.d_npmin = d_npm;
+            xi.d_rows = split ? d_npm + n : 0;
             if ((rc = graph_issue(c, c->stream, &c->x_graph, key, issue_tasks, &xi, &gst)) != 0) goto done;
             if (times) {
                 times->graph_launches += gst.launches;
@@ -2069,17 +2226,6 @@ static double at_normal(unsigned long long *s)
     return sqrt(-2.0 * log(u1)) * cos(2.0 * 3.14159265358979323846 * u2);
 }
 
-/* Whether every fused launch mode a tile runs has an FP32-coefficient
- * instance (electrons: mode 0; two species: the split passes 2 and 3, or the
- * in-kernel contraction 1, which the eta cap also selects). */
-static int tile_f32_ok(const CromaHipContext *c, int protons, int r, int w, int g)
-{
-    const int n = c->g.n;
-    if (!protons) return ck_fused_f32_supported(n, r, w, 0);
-    if (!g || c->prm.eta_dpp_cap > 0.0) return ck_fused_f32_supported(n, r, w, 1);
-    return ck_fused_f32_supported(n, r, w, 2) && ck_fused_f32_supported(n, r, w, 3);
-}
-
 /* Candidate tiles of the autotuners: rows per lane x waves per SIMD (x the
  * split secondary contraction for two species), one snapshot per task. */
 static int tile_candidates(const CromaHipContext *c, int protons, CromaHipTile *out)
@@ -2115,16 +2261,21 @@ int croma_hip_batch_autotune(CromaHipBatch *b, int s, int nsnap_total, const dou
     CromaHipTile cand[16], keep, bt;
     double best_ms = 1e300, *d_save = 0;
     size_t m;
-    int k, nc, rep, rc = 0;
+    int k, nc, rep, rc = 0, keep_set;
     if (!b || !z || !dt_snap || !best || s < 0 || s + 1 > b->nsnap_res || nsnap_total < s + 1)
         return CROMA_HIP_EINVAL;
     c = b->ctx;
     m = (size_t)b->ntr * c->g.n;
     keep = c->tile[b->protons ? 1 : 0];
+    keep_set = c->tile_set[b->protons ? 1 : 0];
+    c->tile_set[b->protons ? 1 : 0] = 1;
     bt = keep;
     /* every trial starts from the batch's current state */
     d_save = (double *)ck_malloc(m * sizeof(double) * (b->protons ? 2 : 1));
-    if (!d_save) return dev_fail("autotune state copy");
+    if (!d_save) {
+        c->tile_set[b->protons ? 1 : 0] = keep_set;
+        return dev_fail("autotune state copy");
+    }
     if (ck_d2d(d_save, b->d_cre, m * sizeof(double), c->stream) ||
         (b->protons && ck_d2d(d_save + m, b->d_crp, m * sizeof(double), c->stream))) {
         rc = dev_fail("autotune state copy");
@@ -2189,6 +2340,7 @@ out:
         ck_free(d_save);
     }
     c->tile[b->protons ? 1 : 0] = rc ? keep : bt;
+    if (rc) c->tile_set[b->protons ? 1 : 0] = keep_set;
     if (!rc) *best = bt;
     return rc;
 }
@@ -2202,9 +2354,11 @@ int croma_hip_autotune(CromaHipContext *c, int protons, int ntracer, CromaHipTil
     CromaHipTile keep, bt, cand[16];
     CromaHipBatch *b = 0;
     unsigned long long seed = 0x5EEDULL + (unsigned long long)n;
-    int i, s, f, k, nc, rc = 0;
+    int i, s, f, k, nc, rc = 0, keep_set;
     if (!c || ntracer <= 0 || !best) return CROMA_HIP_EINVAL;
     keep = c->tile[protons ? 1 : 0];
+    keep_set = c->tile_set[protons ? 1 : 0];
+    c->tile_set[protons ? 1 : 0] = 1;
     bt = keep;
     bg = (double *)malloc((size_t)(nsnap + 1) * CK_NBG * ntracer * sizeof(double));
     cre = (double *)malloc((size_t)ntracer * n * sizeof(double));
@@ -2272,6 +2426,7 @@ out:
     free(cre);
     free(crp);
     c->tile[protons ? 1 : 0] = rc ? keep : bt;
+    if (rc) c->tile_set[protons ? 1 : 0] = keep_set;
     if (!rc) *best = bt;
     return rc;
 }

@@ -40,6 +40,7 @@ void ch_ic_bounds(double z, double *e0min, double *e0max);
 /* IC cooling rate of the electron bins bins[0..count) at z (same arithmetic
  * as ch_ic_cooling_row, which fills every bin). */
 int ch_ic_cooling_bins(const ChGrid *g, double z, int count, const int *bins, double *out);
+void ch_ic_cooling_ends(const ChGrid *g, int nz, const double *z, double *out);
 
 /* croma_host.c */
 double ch_now_s(void);
@@ -52,7 +53,7 @@ const ChGrid *ch_ctx_grid(const CromaHipContext *c);
 const CkGrid *ch_ctx_dgrid(const CromaHipContext *c);
 const CkParams *ch_ctx_prm(const CromaHipContext *c);
 int ch_ctx_cu_count(const CromaHipContext *c);
-CromaHipTile ch_ctx_tile(const CromaHipContext *c, int protons);
+CromaHipTile ch_ctx_tile(const CromaHipContext *c, int protons, long ntr);
 int ch_ctx_coeff_fp32(const CromaHipContext *c); /* FP32 coefficient evaluation selected */
 int ch_ctx_fqe(CromaHipContext *c);              /* builds the secondary weights once */
 const double *ch_ctx_d_fqe(const CromaHipContext *c);
@@ -62,7 +63,7 @@ int ch_ctx_plain_ws(CromaHipContext *c, int count, CkPlainWs *out); /* plain-pat
 void *ch_ctx_stream(const CromaHipContext *c);
 int *ch_ctx_d_err(const CromaHipContext *c);
 int ch_ctx_take_err(CromaHipContext *c); /* reads and clears the error word: 0, EPIVOT or ENONFINITE */
-void ch_ctx_ic_ends(CromaHipContext *c, double z, double ends[2]); /* IC rate at bins 0, n-1 (cached) */
+void ch_ctx_ic_ends(CromaHipContext *c, int nz, const double *z, double *ends); /* IC rate at bins 0, n-1 (cached) */
 int ch_cost_bucket(double cost);                 /* log-scale bucket in [0, CH_HIST) */
 
 /* device-resident state of a batch (read by the file writers) */

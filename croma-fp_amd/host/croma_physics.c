@@ -456,6 +456,35 @@ int ch_ic_cooling_bins(const ChGrid *g, double z, int count, const int *bins, do
     return 0;
 }
 
+typedef struct {
+    const ChGrid *g;
+    const double *z;
+    double *out;
+} ChIcEndsJob;
+
+static void ch_ic_ends_range(void *arg, long i0, long i1)
+{
+    ChIcEndsJob *J = (ChIcEndsJob *)arg;
+    long i;
+    for (i = i0; i < i1; i++) {
+        const double p = J->g->ep[(i & 1) ? J->g->n - 1 : 0];
+        double lo, hi;
+        ch_cmb_bounds(J->z[i >> 1], &lo, &hi);
+        J->out[i] = ch_b_ic(sqrt(1.0 + p * p), lo, hi, J->z[i >> 1]);
+    }
+}
+
+/* IC cooling rates of the electron grid's first and last bins, out[2 q],
+ * out[2 q + 1], at z[q], q < nz. */
+void ch_ic_cooling_ends(const ChGrid *g, int nz, const double *z, double *out)
+{
+    ChIcEndsJob J;
+    J.g = g;
+    J.z = z;
+    J.out = out;
+    ch_parallel_for(2 * (long)nz, 1, ch_ic_ends_range, &J);
+}
+
 int ch_ic_cooling_row(const ChGrid *g, double z, double *row, double *m1, double *p1)
 {
     ChIcJob J;

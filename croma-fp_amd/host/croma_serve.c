@@ -299,15 +299,17 @@ static int sv_prepare(CromaHipServer *s, SvReq *r)
          * host estimate's integers, tracer_fp_nsub.c:94-282, with the IC
          * rate at the end bins from the host's exact rows), then to the
          * pinned host copy the task ordering reads */
+        double *const ends = (double *)malloc((size_t)r->nsnap * 2 * sizeof(double));
+        if (ends) ch_ctx_ic_ends(c, r->nsnap, r->z, ends);
+        else rc = 1;
         for (q = 0; q < r->nsnap && !rc; q++) {
             const double *db = r->d_bg + (size_t)q * CK_NBG * r->ntr;
-            double ends[2];
-            ch_ctx_ic_ends(c, r->z[q], ends);
-            rc |= ck_nsub_arrays(*ch_ctx_dgrid(c), r->prm, r->ntr, r->dt[q], ends[0], ends[1], db,
+            rc |= ck_nsub_arrays(*ch_ctx_dgrid(c), r->prm, r->ntr, r->dt[q], ends[2 * q], ends[2 * q + 1], db,
                                  db + (size_t)r->ntr, db + 2 * (size_t)r->ntr, db + 3 * (size_t)r->ntr,
                                  db + 4 * (size_t)r->ntr, db + 5 * (size_t)r->ntr, r->d_nsub + (size_t)q * r->ntr,
                                  r->d_non + (size_t)q * r->ntr, cs);
         }
+        free(ends);
         rc |= ck_d2h(r->h_sched, r->d_nsub, (size_t)r->nsnap * r->ntr * sizeof(int), cs);
         rc |= ck_d2h(r->h_sched + (size_t)r->nsnap * r->ntr, r->d_non, (size_t)r->nsnap * r->ntr * sizeof(int), cs);
         rc |= ck_h2d(r->d_zb, r->h_zb, (size_t)(r->nsnap + 1) * 3 * sizeof(double), cs);
@@ -453,7 +455,6 @@ static int sv_launch_class(CromaHipServer *s, int ci)
     int i, nslots = 0, ntasks = 0, nl = 0, q, split;
     long pos, segrows = 0, nsegoff = 0;
     if (!c) return 0;
-    tile = ch_ctx_tile(c, protons);
     for (i = 0; i < s->nactive; i++) {
         SvReq *r = s->active[i];
         if (r->cls != ci || r->state != SV_ACTIVE || r->snap_next >= r->nsnap || sv_cancelled(r)) continue;
@@ -464,12 +465,17 @@ static int sv_launch_class(CromaHipServer *s, int ci)
             r->ready = 1;
             sv_count_steps(r);
         }
-        r->inflight = r->nsnap - r->snap_next < tile.chain ? r->nsnap - r->snap_next : tile.chain;
-        nslots += r->inflight;
         ntasks += r->ntr;
         nl++;
     }
     if (nl == 0) return 0;
+    tile = ch_ctx_tile(c, protons, ntasks);
+    for (i = 0; i < s->nactive; i++) {
+        SvReq *r = s->active[i];
+        if (r->cls != ci || r->state != SV_ACTIVE || r->snap_next >= r->nsnap || sv_cancelled(r) || !r->ready) continue;
+        r->inflight = r->nsnap - r->snap_next < tile.chain ? r->nsnap - r->snap_next : tile.chain;
+        nslots += r->inflight;
+    }
     if (sv_grow_class(k, nslots, ntasks, nl)) return CROMA_HIP_ENOMEM;
     /* two species without the eta cap: proton pass, one GEMM, electron pass */
     split = protons && tile.secondary_gemm && !(ch_ctx_prm(c)->eta_dpp_cap > 0.0);

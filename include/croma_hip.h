@@ -123,7 +123,9 @@ typedef struct CromaHipContext CromaHipContext;
 CromaHipContext *croma_hip_context_create(const CromaHipGridSpec *grid, const CromaHipParams *prm);
 void croma_hip_context_destroy(CromaHipContext *ctx);
 int croma_hip_context_set_params(CromaHipContext *ctx, const CromaHipParams *prm);
-/* protons: 0 electron_only tile, 1 electron_proton tile, -1 both. */
+/* protons: 0 electron_only tile, 1 electron_proton tile, -1 both.  Until a tile
+ * is set here or by an autotuner, every run takes one by its grid, species,
+ * tracers and snapshots; get_tile then returns the grid's default. */
 int croma_hip_context_set_tile(CromaHipContext *ctx, int protons, const CromaHipTile *tile);
 int croma_hip_context_get_tile(const CromaHipContext *ctx, int protons, CromaHipTile *tile);
 /* 1 (default): a snapshot window whose launch shape repeats the previous
@@ -133,10 +135,11 @@ int croma_hip_context_get_tile(const CromaHipContext *ctx, int protons, CromaHip
 int croma_hip_context_set_graphs(CromaHipContext *ctx, int enable);
 /* 1: in batch runs with the split secondary contraction, the electron pass of each
  * snapshot window runs on a second stream beside the proton pass of the next
- * window, each on half the device; 0 (default): the passes of a window run
- * in turn on the full device.  The spectra are the same either way; which is
- * faster depends on the tile.  No reference counterpart (the reference runs
- * one species pass at a time). */
+ * window, each on half the device; 0: the passes of a window run in turn on
+ * the full device.  Until set, batches of up to 3 * 2^20 rows (tracers x bins)
+ * are pipelined: their passes wait for their costliest tracers and leave the
+ * device room for each other.  The spectra are the same either way.  No
+ * reference counterpart (the reference runs one species pass at a time). */
 int croma_hip_context_set_pipeline(CromaHipContext *ctx, int enable);
 /* 1 (default): batch runs estimate nsub (tracer_fp_nsub.c:94-282), order the
  * queue by cost and assign the split segment rows on the device, without a
