@@ -32,7 +32,7 @@ static float em_bf16f(uint16_t h)
 }
 
 /* kmat given as km(k, j) through a callback-free dense array [nbins][K]. */
-static int em_contract(int ntr, int K, int nbins, const double *spectra, const double *kmat_bk,
+static int em_contract(const CromaHipContext *ctx, int ntr, int K, int nbins, const double *spectra, const double *kmat_bk,
                        const double *row_scale, double *eps, int mode, double *elapsed_ms)
 {
     const int pad = (nbins + 63) / 64 * 64;
@@ -42,7 +42,9 @@ static int em_contract(int ntr, int K, int nbins, const double *spectra, const d
     uint16_t *khi = (uint16_t *)calloc(nk, sizeof(uint16_t)), *klo = (uint16_t *)calloc(nk, sizeof(uint16_t));
     int *csh = (int *)calloc((size_t)pad, sizeof(int));
     char *d = 0, *p;
-    void *st = 0, *e0 = 0, *e1 = 0;
+    ChWork w;
+    void *st, *e0, *e1;
+    const int dev = ch_ctx_device(ctx);
     int rc = 0, c, j;
     size_t bytes;
     if (!kt64 || !kt32 || !khi || !klo || !csh) {
@@ -70,11 +72,11 @@ static int em_contract(int ntr, int K, int nbins, const double *spectra, const d
         }
     }
     bytes = ns * 8 + nk * 8 + nk * 4 + nk * 4 + (size_t)pad * 4 + (size_t)ntr * 8 + no * 8 + 8 * 256;
-    d = (char *)ck_malloc(bytes);
-    st = ck_stream_create();
-    e0 = ck_event_create();
-    e1 = ck_event_create();
-    if (!d || !st || !e0 || !e1) {
+    d = ch_work_take(ctx, bytes, &w);
+    st = w.stream;
+    e0 = w.e0;
+    e1 = w.e1;
+    if (!d) {
         rc = CROMA_HIP_EDEVICE;
         ch_set_error("emission: device allocation: %s", ck_last_error());
         goto out;
@@ -99,12 +101,12 @@ static int em_contract(int ntr, int K, int nbins, const double *spectra, const d
         if (row_scale) EM_TAKE(d_rs, double, (size_t)ntr * 8);
         EM_TAKE(d_out, double, no * 8);
 #undef EM_TAKE
-        if (ck_h2d(d_s, spectra, ns * 8, st) || ck_h2d(d_k64, kt64, nk * 8, st) || ck_h2d(d_k32, kt32, nk * 4, st) ||
+        if (ch_stage_h2d(dev, d_s, spectra, ns * 8, st) || ck_h2d(d_k64, kt64, nk * 8, st) || ck_h2d(d_k32, kt32, nk * 4, st) ||
             ck_h2d(d_hi, khi, nk * 2, st) || ck_h2d(d_lo, klo, nk * 2, st) ||
             ck_h2d(d_cs, csh, (size_t)pad * 4, st) || (row_scale && ck_h2d(d_rs, row_scale, (size_t)ntr * 8, st)) ||
             ck_event_record(e0, st) ||
             ck_emission_contract(ntr, K, nbins, pad, d_s, d_hi, d_lo, d_k32, d_k64, d_cs, d_rs, d_out, mode, st) ||
-            ck_event_record(e1, st) || ck_d2h(eps, d_out, no * 8, st) || ck_stream_sync(st)) {
+            ck_event_record(e1, st) || ch_stage_d2h(dev, eps, d_out, no * 8, st) || ck_stream_sync(st)) {
             rc = CROMA_HIP_EDEVICE;
             ch_set_error("emission: %s", ck_last_error());
             goto out;
@@ -112,11 +114,10 @@ static int em_contract(int ntr, int K, int nbins, const double *spectra, const d
         if (elapsed_ms) *elapsed_ms = ck_event_elapsed_ms(e0, e1);
     }
 out:
-    if (st) ck_stream_sync(st);
-    ck_free(d);
-    ck_event_destroy(e0);
-    ck_event_destroy(e1);
-    if (st) ck_stream_destroy(st);
+    if (d) {
+        ck_stream_sync(st);
+        ch_work_give(ctx, &w);
+    }
     free(kt64);
     free(kt32);
     free(khi);
@@ -140,7 +141,7 @@ int croma_hip_emission_ic(const CromaHipContext *ctx, int ntracer, int nbins, co
     /* eps[i][k] = sum_j fic[k][j] cre[i][j] dp[j] (fp_shared_core.c:2131-2157) */
     for (k = 0; k < nbins; k++)
         for (j = 0; j < n; j++) km[(size_t)k * n + j] = fic_flat[(size_t)k * n + j] * g->edp[j];
-    rc = em_contract(ntracer, n, nbins, cre, km, 0, eps, mode, elapsed_ms);
+    rc = em_contract(ctx, ntracer, n, nbins, cre, km, 0, eps, mode, elapsed_ms);
     free(km);
     return rc;
 }
@@ -174,7 +175,7 @@ int croma_hip_emission_hadronic(const CromaHipContext *ctx, int ntracer, int nbi
         e = pow(10.0, a);
         for (j = 0; j < n; j++) km[(size_t)k * n + j] = e * 0.5 * g->beta_p[j] * tw[j] * f_flat[(size_t)k * n + j];
     }
-    rc = em_contract(ntracer, n, nbins, crp, km, n_gas, eps, mode, elapsed_ms);
+    rc = em_contract(ctx, ntracer, n, nbins, crp, km, n_gas, eps, mode, elapsed_ms);
     free(km);
     free(tw);
     return rc;
@@ -188,8 +189,9 @@ int croma_hip_synch_kernel_table(const CromaHipContext *ctx, int nfreq, int nthe
     const ChGrid *g;
     size_t ny, nt, bytes;
     double *d = 0;
-    void *st = 0, *e0 = 0, *e1 = 0;
-    int n, rc = 0;
+    ChWork w;
+    void *st, *e0, *e1;
+    int n, rc = 0, dev;
     if (!ctx || nfreq <= 0 || ntheta <= 0 || nlogb <= 0 || nx_tab < 1 || !logx_tab || !logfx_tab || !fx_tab ||
         !logy || !pitch_weight || !table || !(inv_dlogb > 0.0))
         return CROMA_HIP_EINVAL;
@@ -198,11 +200,12 @@ int croma_hip_synch_kernel_table(const CromaHipContext *ctx, int nfreq, int nthe
     ny = (size_t)nfreq * n * ntheta;
     nt = (size_t)nlogb * nfreq * n;
     bytes = (3 * (size_t)nx_tab + ny + (size_t)ntheta + nt) * sizeof(double);
-    d = (double *)ck_malloc(bytes);
-    st = ck_stream_create();
-    e0 = ck_event_create();
-    e1 = ck_event_create();
-    if (!d || !st || !e0 || !e1) {
+    dev = ch_ctx_device(ctx);
+    d = (double *)ch_work_take(ctx, bytes, &w);
+    st = w.stream;
+    e0 = w.e0;
+    e1 = w.e1;
+    if (!d) {
         rc = CROMA_HIP_EDEVICE;
         ch_set_error("synch table: device allocation: %s", ck_last_error());
         goto out;
@@ -211,11 +214,11 @@ int croma_hip_synch_kernel_table(const CromaHipContext *ctx, int nfreq, int nthe
         double *d_lx = d, *d_lfx = d + nx_tab, *d_fx = d + 2 * (size_t)nx_tab, *d_ly = d + 3 * (size_t)nx_tab;
         double *d_pw = d_ly + ny, *d_tab = d_pw + ntheta;
         if (ck_h2d(d_lx, logx_tab, (size_t)nx_tab * 8, st) || ck_h2d(d_lfx, logfx_tab, (size_t)nx_tab * 8, st) ||
-            ck_h2d(d_fx, fx_tab, (size_t)nx_tab * 8, st) || ck_h2d(d_ly, logy, ny * 8, st) ||
+            ck_h2d(d_fx, fx_tab, (size_t)nx_tab * 8, st) || ch_stage_h2d(dev, d_ly, logy, ny * 8, st) ||
             ck_h2d(d_pw, pitch_weight, (size_t)ntheta * 8, st) || ck_event_record(e0, st) ||
             ck_synch_table(n, nfreq, ntheta, nlogb, logb_min, inv_dlogb, nx_tab, xmin, d_lx, d_lfx, d_fx, d_ly,
                            d_pw, d_tab, st) ||
-            ck_event_record(e1, st) || ck_d2h(table, d_tab, nt * 8, st) || ck_stream_sync(st)) {
+            ck_event_record(e1, st) || ch_stage_d2h(dev, table, d_tab, nt * 8, st) || ck_stream_sync(st)) {
             rc = CROMA_HIP_EDEVICE;
             ch_set_error("synch table: %s", ck_last_error());
             goto out;
@@ -223,11 +226,10 @@ int croma_hip_synch_kernel_table(const CromaHipContext *ctx, int nfreq, int nthe
         if (elapsed_ms) *elapsed_ms = ck_event_elapsed_ms(e0, e1);
     }
 out:
-    if (st) ck_stream_sync(st);
-    ck_free(d);
-    ck_event_destroy(e0);
-    ck_event_destroy(e1);
-    if (st) ck_stream_destroy(st);
+    if (d) {
+        ck_stream_sync(st);
+        ch_work_give(ctx, &w);
+    }
     return rc;
 }
 
@@ -246,7 +248,7 @@ int croma_hip_emission_synch(const CromaHipContext *ctx, int ntracer, int nfreq,
  * grow to the largest call. */
 struct CromaHipSynchPlan {
     const CromaHipContext *ctx;
-    int n, nfreq, nlogb;
+    int device, n, nfreq, nlogb;
     double logb_min, inv_dlogb;
     char *d_const;
     double *d_tab, *d_dp;
@@ -271,6 +273,7 @@ void croma_hip_synch_plan_destroy(CromaHipSynchPlan *p)
     if (p->e0) ck_event_destroy(p->e0);
     if (p->e1) ck_event_destroy(p->e1);
     if (p->stream) ck_stream_destroy(p->stream);
+    ch_stage_unref(p->device);
     free(p);
 }
 
@@ -294,6 +297,8 @@ CromaHipSynchPlan *croma_hip_synch_plan_create(const CromaHipContext *ctx, int n
     p = (CromaHipSynchPlan *)calloc(1, sizeof(*p));
     if (!p) return 0;
     p->ctx = ctx;
+    p->device = ch_ctx_device(ctx);
+    ch_stage_ref(p->device);
     p->n = g->n;
     p->nfreq = nfreq;
     p->nlogb = nlogb;
@@ -324,7 +329,7 @@ CromaHipSynchPlan *croma_hip_synch_plan_create(const CromaHipContext *ctx, int n
     p->d_cs = (int *)q;
     q += SY_R(ncs * 4);
     p->d_lt = (float *)q;
-    if (ck_h2d(p->d_tab, table, ntab * 8, p->stream) || ck_h2d(p->d_dp, g->edp, (size_t)p->n * 8, p->stream) ||
+    if (ch_stage_h2d(p->device, p->d_tab, table, ntab * 8, p->stream) || ck_h2d(p->d_dp, g->edp, (size_t)p->n * 8, p->stream) ||
         ck_event_record(p->e0, p->stream) ||
         ck_synch_mfma_prepare(p->n, nfreq, nlogb, p->d_tab, p->d_dp, p->d_hi, p->d_lo, p->d_cs, p->d_lt, p->stream) ||
         ck_event_record(p->e1, p->stream) || ck_stream_sync(p->stream)) {
@@ -365,11 +370,12 @@ int croma_hip_synch_plan_run(CromaHipSynchPlan *p, int ntr, const double *cre, c
         p->d_fix = (int *)q;
         p->cap = ntr;
     }
-    if (ck_h2d(p->d_cre, cre, (size_t)ntr * n * 8, p->stream) ||
+    if (ch_stage_h2d(p->device, p->d_cre, cre, (size_t)ntr * n * 8, p->stream) ||
         ck_h2d(p->d_b, b_field, (size_t)ntr * 8, p->stream) || ck_event_record(p->e0, p->stream) ||
         ck_synch_mfma_run(ntr, n, p->nfreq, p->nlogb, p->logb_min, p->inv_dlogb, p->d_tab, p->d_hi, p->d_lo, p->d_cs,
                           p->d_lt, p->d_work, p->d_fix, p->d_cre, p->d_dp, p->d_b, p->d_eps, p->stream) ||
-        ck_event_record(p->e1, p->stream) || ck_d2h(eps, p->d_eps, (size_t)ntr * p->nfreq * 8, p->stream) ||
+        ck_event_record(p->e1, p->stream) ||
+        ch_stage_d2h(p->device, eps, p->d_eps, (size_t)ntr * p->nfreq * 8, p->stream) ||
         ck_stream_sync(p->stream)) {
         ch_set_error("synch MFMA: %s", ck_last_error());
         return CROMA_HIP_EDEVICE;
@@ -399,8 +405,9 @@ int croma_hip_emission_synch_mode(const CromaHipContext *ctx, int ntracer, int n
     const ChGrid *g;
     const size_t nt_tab = (size_t)nlogb * nfreq;
     char *d = 0, *p;
-    void *st = 0, *e0 = 0, *e1 = 0;
-    int n, rc = 0;
+    ChWork w;
+    void *st, *e0, *e1;
+    int n, rc = 0, dev;
     if (!ctx || ntracer <= 0 || nfreq <= 0 || nlogb < 2 || !table || !cre || !b_field || !eps ||
         (mode != CROMA_HIP_EMIS_FP64 && mode != CROMA_HIP_EMIS_FP32 && mode != CROMA_HIP_EMIS_MFMA_XF32))
         return CROMA_HIP_EINVAL;
@@ -408,12 +415,13 @@ int croma_hip_emission_synch_mode(const CromaHipContext *ctx, int ntracer, int n
     n = g->n;
     if (mode == CROMA_HIP_EMIS_MFMA_XF32) return synch_mfma(ctx, ntracer, nfreq, nlogb, logb_min, inv_dlogb, table,
                                                             cre, b_field, eps, elapsed_ms);
-    d = (char *)ck_malloc(2 * nt_tab * n * 8 + (size_t)ntracer * n * 8 + (size_t)n * 8 + (size_t)ntracer * 8 +
-                          (size_t)ntracer * nfreq * 8 + (3 * (size_t)ntracer + (size_t)nlogb) * 4 + 7 * 256);
-    st = ck_stream_create();
-    e0 = ck_event_create();
-    e1 = ck_event_create();
-    if (!d || !st || !e0 || !e1) {
+    dev = ch_ctx_device(ctx);
+    d = ch_work_take(ctx, 2 * nt_tab * n * 8 + (size_t)ntracer * n * 8 + (size_t)n * 8 + (size_t)ntracer * 8 +
+                          (size_t)ntracer * nfreq * 8 + (3 * (size_t)ntracer + (size_t)nlogb) * 4 + 7 * 256, &w);
+    st = w.stream;
+    e0 = w.e0;
+    e1 = w.e1;
+    if (!d) {
         rc = CROMA_HIP_EDEVICE;
         ch_set_error("synch emission: device allocation: %s", ck_last_error());
         goto out;
@@ -435,12 +443,14 @@ int croma_hip_emission_synch_mode(const CromaHipContext *ctx, int ntracer, int n
         d_eps = (double *)p;
         p += ((size_t)ntracer * nfreq * 8 + 255) & ~(size_t)255;
         d_work = (int *)p;
-        if (ck_h2d(d_tab, table, nt_tab * n * 8, st) || ck_h2d(d_cre, cre, (size_t)ntracer * n * 8, st) ||
+        if (ch_stage_h2d(dev, d_tab, table, nt_tab * n * 8, st) ||
+            ch_stage_h2d(dev, d_cre, cre, (size_t)ntracer * n * 8, st) ||
             ck_h2d(d_dp, g->edp, (size_t)n * 8, st) || ck_h2d(d_b, b_field, (size_t)ntracer * 8, st) ||
             ck_event_record(e0, st) ||
             ck_emission_synch(ntracer, n, nfreq, nlogb, logb_min, inv_dlogb, d_tab, d_logt, d_work, d_cre, d_dp, d_b,
                               d_eps, mode == CROMA_HIP_EMIS_FP64, st) ||
-            ck_event_record(e1, st) || ck_d2h(eps, d_eps, (size_t)ntracer * nfreq * 8, st) || ck_stream_sync(st)) {
+            ck_event_record(e1, st) || ch_stage_d2h(dev, eps, d_eps, (size_t)ntracer * nfreq * 8, st) ||
+            ck_stream_sync(st)) {
             rc = CROMA_HIP_EDEVICE;
             ch_set_error("synch emission: %s", ck_last_error());
             goto out;
@@ -448,10 +458,9 @@ int croma_hip_emission_synch_mode(const CromaHipContext *ctx, int ntracer, int n
         if (elapsed_ms) *elapsed_ms = ck_event_elapsed_ms(e0, e1);
     }
 out:
-    if (st) ck_stream_sync(st);
-    ck_free(d);
-    ck_event_destroy(e0);
-    ck_event_destroy(e1);
-    if (st) ck_stream_destroy(st);
+    if (d) {
+        ck_stream_sync(st);
+        ch_work_give(ctx, &w);
+    }
     return rc;
 }

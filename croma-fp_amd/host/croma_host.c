@@ -200,6 +200,11 @@ struct CromaHipContext {
     void *x_ws;
     size_t x_ws_bytes;
     ChGraph x_graph;
+    /* work of calls on host arrays (emission, tables) */
+    pthread_mutex_t work_lock;
+    int work_busy;
+    ChWork work;
+    int staged; /* holds a reference to the device's transfer ring */
 };
 
 /* Derived tables of the Chang-Cooper build for one species: face width
@@ -387,12 +392,16 @@ CromaHipContext *croma_hip_context_create(const CromaHipGridSpec *gs, const Crom
     c = (CromaHipContext *)calloc(1, sizeof(*c));
     if (!c) return 0;
     pthread_mutex_init(&c->ic_lock, 0);
+    pthread_mutex_init(&c->work_lock, 0);
     c->device = ck_get_device();
     if (c->device < 0) c->device = 0;
     c->cu_count = ck_device_cu_count(c->device);
     if (c->cu_count <= 0) c->cu_count = 256;
+    ch_stage_ref(c->device);
+    c->staged = 1;
     if (ch_grid_build(&c->g, gs->n, gs->pmin, gs->pmax, gs->pemin, gs->pemax) != 0) {
         ch_set_error("grid build failed");
+        ch_stage_unref(c->device);
         free(c);
         return 0;
     }
@@ -461,6 +470,12 @@ void croma_hip_context_destroy(CromaHipContext *c)
     free(c->h_npmin);
     if (c->stream_e) ck_stream_destroy(c->stream_e);
     if (c->stream) ck_stream_destroy(c->stream);
+    ck_free(c->work.dev);
+    if (c->work.e0) ck_event_destroy(c->work.e0);
+    if (c->work.e1) ck_event_destroy(c->work.e1);
+    if (c->work.stream) ck_stream_destroy(c->work.stream);
+    if (c->staged) ch_stage_unref(c->device);
+    pthread_mutex_destroy(&c->work_lock);
     pthread_mutex_destroy(&c->ic_lock);
     free(c);
 }
@@ -749,28 +764,75 @@ int croma_hip_emission_kernel_table(const CromaHipContext *cc, int kind, int nbi
     const int n = c ? c->g.n : 0;
     const double *mom;
     double *d_out;
-    void *e0 = 0, *e1 = 0;
+    ChWork w;
     int rc = 0;
     if (!c || !table || nbins <= 0 || nbins > 65535 || kind < CROMA_HIP_TABLE_GAMMA || kind > CROMA_HIP_TABLE_IC ||
         !(hi > lo) || !isfinite(lo) || !isfinite(hi) || !isfinite(z))
         return CROMA_HIP_EINVAL;
     mom = kind == CROMA_HIP_TABLE_IC ? c->dgrid.ep : c->dgrid.pp;
-    d_out = (double *)ck_malloc((size_t)nbins * n * sizeof(double));
+    d_out = (double *)ch_work_take(c, (size_t)nbins * n * sizeof(double), &w);
     if (!d_out) return dev_fail("kernel table alloc");
-    if (elapsed_ms) {
-        e0 = ck_event_create();
-        e1 = ck_event_create();
-    }
-    if ((e0 && ck_event_record(e0, c->stream)) ||
-        ck_emission_kernel_table(kind, n, nbins, lo, hi, z, mom, d_out, c->stream) ||
-        (e1 && ck_event_record(e1, c->stream)) ||
-        ck_d2h(table, d_out, (size_t)nbins * n * sizeof(double), c->stream) || ck_stream_sync(c->stream))
+    if (ck_event_record(w.e0, w.stream) ||
+        ck_emission_kernel_table(kind, n, nbins, lo, hi, z, mom, d_out, w.stream) ||
+        ck_event_record(w.e1, w.stream) ||
+        ck_d2h(table, d_out, (size_t)nbins * n * sizeof(double), w.stream) || ck_stream_sync(w.stream))
         rc = dev_fail("kernel table");
-    if (!rc && elapsed_ms) *elapsed_ms = (e0 && e1) ? (double)ck_event_elapsed_ms(e0, e1) : -1.0;
-    if (e0) ck_event_destroy(e0);
-    if (e1) ck_event_destroy(e1);
-    ck_free(d_out);
+    if (!rc && elapsed_ms) *elapsed_ms = (double)ck_event_elapsed_ms(w.e0, w.e1);
+    if (rc) ck_stream_sync(w.stream);
+    ch_work_give(c, &w);
     return rc;
+}
+
+int ch_ctx_device(const CromaHipContext *c) { return c->device; }
+
+char *ch_work_take(const CromaHipContext *cc, size_t bytes, ChWork *w)
+{
+    CromaHipContext *c = (CromaHipContext *)cc;
+    char *p;
+    memset(w, 0, sizeof(*w));
+    pthread_mutex_lock(&c->work_lock);
+    if (!c->work_busy) {
+        c->work_busy = 1;
+        *w = c->work;
+        w->kept = 1;
+    }
+    pthread_mutex_unlock(&c->work_lock);
+    w->device = c->device;
+    if (!w->stream) w->stream = ck_stream_create();
+    if (!w->e0) w->e0 = ck_event_create();
+    if (!w->e1) w->e1 = ck_event_create();
+    if (w->kept && bytes <= CH_WORK_KEEP) {
+        if (w->cap < bytes) {
+            ck_free(w->dev);
+            w->dev = (char *)ck_malloc(bytes);
+            w->cap = w->dev ? bytes : 0;
+        }
+        p = w->dev;
+    } else {
+        p = w->extra = (char *)ck_malloc(bytes);
+    }
+    if (p && w->stream && w->e0 && w->e1) return p;
+    ch_work_give(c, w);
+    return 0;
+}
+
+void ch_work_give(const CromaHipContext *cc, ChWork *w)
+{
+    CromaHipContext *c = (CromaHipContext *)cc;
+    ck_free(w->extra);
+    w->extra = 0;
+    if (w->kept) {
+        pthread_mutex_lock(&c->work_lock);
+        c->work = *w;
+        c->work_busy = 0;
+        pthread_mutex_unlock(&c->work_lock);
+    } else {
+        ck_free(w->dev);
+        if (w->e0) ck_event_destroy(w->e0);
+        if (w->e1) ck_event_destroy(w->e1);
+        if (w->stream) ck_stream_destroy(w->stream);
+    }
+    memset(w, 0, sizeof(*w));
 }
 
 /* Accessors for the serving loop (croma_serve.c). */
@@ -1082,12 +1144,12 @@ fail:
     return 0;
 }
 
-static int upload_opt(double **dst, const double *src, size_t bytes, void *stream)
+static int upload_opt(int dev, double **dst, const double *src, size_t bytes, void *stream)
 {
     if (!src) return 0;
     if (!*dst) *dst = (double *)ck_malloc(bytes);
     if (!*dst) return -1;
-    return ck_h2d(*dst, src, bytes, stream);
+    return ch_stage_h2d(dev, *dst, src, bytes, stream);
 }
 
 int croma_hip_batch_set_state(CromaHipBatch *b, const double *crp, const double *cre, const double *qpi,
@@ -1107,19 +1169,19 @@ int croma_hip_batch_set_state(CromaHipBatch *b, const double *crp, const double 
                 return CROMA_HIP_EINVAL;
             }
     }
-    if (ck_h2d(b->d_cre, cre, sn, c->stream)) return dev_fail("state upload");
+    if (ch_stage_h2d(c->device, b->d_cre, cre, sn, c->stream)) return dev_fail("state upload");
     if (b->protons) {
         if (crp) {
-            if (ck_h2d(b->d_crp, crp, sn, c->stream)) return dev_fail("state upload");
+            if (ch_stage_h2d(c->device, b->d_crp, crp, sn, c->stream)) return dev_fail("state upload");
         } else if (ck_fill_f64(b->d_crp, 0.0, (size_t)b->ntr * c->g.n, c->stream)) {
             return dev_fail("state clear");
         }
-        if (upload_opt(&b->d_qpi, qpi, sn, c->stream)) return dev_fail("qpi upload");
+        if (upload_opt(c->device, &b->d_qpi, qpi, sn, c->stream)) return dev_fail("qpi upload");
         b->has_qpi = qpi != 0;
     }
-    if (upload_opt(&b->d_qepri, qepri, sn, c->stream)) return dev_fail("qepri upload");
+    if (upload_opt(c->device, &b->d_qepri, qepri, sn, c->stream)) return dev_fail("qepri upload");
     b->has_qepri = qepri != 0;
-    if (upload_opt(&b->d_mass, mass, (size_t)b->ntr * sizeof(double), c->stream)) return dev_fail("mass upload");
+    if (upload_opt(c->device, &b->d_mass, mass, (size_t)b->ntr * sizeof(double), c->stream)) return dev_fail("mass upload");
     b->has_mass = mass != 0;
     if (dis) {
         if (!b->d_dis) b->d_dis = (unsigned char *)ck_malloc((size_t)b->ntr);
@@ -1148,10 +1210,10 @@ int croma_hip_batch_get_state(CromaHipBatch *b, double *crp, double *cre)
     if (!b) return CROMA_HIP_EINVAL;
     c = b->ctx;
     sn = (size_t)b->ntr * c->g.n * sizeof(double);
-    if (cre && ck_d2h(cre, b->d_cre, sn, c->stream)) return dev_fail("state download");
+    if (cre && ch_stage_d2h(c->device, cre, b->d_cre, sn, c->stream)) return dev_fail("state download");
     if (crp) {
         if (b->protons) {
-            if (ck_d2h(crp, b->d_crp, sn, c->stream)) return dev_fail("state download");
+            if (ch_stage_d2h(c->device, crp, b->d_crp, sn, c->stream)) return dev_fail("state download");
         } else {
             memset(crp, 0, sn);
         }
@@ -1196,12 +1258,12 @@ int croma_hip_batch_set_sources(CromaHipBatch *b, int isnap, const double *qpi, 
                         return CROMA_HIP_EINVAL;
                     }
             }
-            if (ck_h2d(dp, qpi, m * sizeof(double), b->ctx->stream)) return dev_fail("source upload");
+            if (ch_stage_h2d(b->ctx->device, dp, qpi, m * sizeof(double), b->ctx->stream)) return dev_fail("source upload");
         } else if (ck_fill_f64(dp, 0.0, m, b->ctx->stream)) {
             return dev_fail("source clear");
         }
         if (qepri) {
-            if (ck_h2d(dp + m, qepri, m * sizeof(double), b->ctx->stream)) return dev_fail("source upload");
+            if (ch_stage_h2d(b->ctx->device, dp + m, qepri, m * sizeof(double), b->ctx->stream)) return dev_fail("source upload");
         } else if (ck_fill_f64(dp + m, 0.0, m, b->ctx->stream)) {
             return dev_fail("source clear");
         }

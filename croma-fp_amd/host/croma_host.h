@@ -47,6 +47,29 @@ double ch_now_s(void);
 void ch_set_error(const char *fmt, ...);
 void ch_params_to_ck(const CromaHipParams *in, CkParams *out);
 
+/* croma_stage.c: transfers of pageable arrays of any size (4 MiB and more
+ * through the device's pinned ring), one reference per context */
+void ch_stage_ref(int dev);
+void ch_stage_unref(int dev);
+int ch_stage_h2d(int dev, void *dst, const void *src, size_t bytes, void *stream);
+int ch_stage_d2h(int dev, void *dst, const void *src, size_t bytes, void *stream);
+
+/* Stream, timing events and device memory of one call on host arrays: the
+ * context's own (memory up to CH_WORK_KEEP stays with it), or the call's own
+ * while another thread has those. */
+#define CH_WORK_KEEP ((size_t)512 << 20)
+typedef struct {
+    void *stream, *e0, *e1;
+    char *dev;
+    size_t cap;
+    int kept;     /* the context's */
+    char *extra;  /* memory of this call alone */
+    int device;
+} ChWork;
+char *ch_work_take(const CromaHipContext *c, size_t bytes, ChWork *w); /* device memory, or NULL */
+void ch_work_give(const CromaHipContext *c, ChWork *w);                /* after the stream drained */
+int ch_ctx_device(const CromaHipContext *c);
+
 /* context internals shared with the serving loop */
 #define CH_HIST 8192
 const ChGrid *ch_ctx_grid(const CromaHipContext *c);
