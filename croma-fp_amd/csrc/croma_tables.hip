@@ -1,10 +1,11 @@
 // Grid-constant kernel tables built on the device from the shared physics
-// header (croma_hadronic.h), one table entry per thread:
+// header (croma_hadronic.h), one table entry per thread (the IC table eight
+// lanes per entry):
 //   secondary-electron weights fqe_t[jp][je]   fp_shared_core.c:1453-1506 (QeKernel_BB05, HADRONIC.c:436-498)
 //   gamma / neutrino / IC kernel tables [k][j]  fp_shared_core.c:1724-1804 (prepare_*_kernel_flat),
 //                                              HADRONIC.c:139-289, FP_Coef.c:553-582
 // Every entry is an independent FP64 quadrature of 50..400 nodes (pow /
-// log10 / exp per node), so the tables are FP64-VALU bound and need no LDS;
+// log10 / exp per node), so the tables are FP64-VALU bound;
 // threads of a wave walk consecutive columns so each store is coalesced.
 #include <hip/hip_runtime.h>
 
@@ -58,11 +59,11 @@ __global__ void __launch_bounds__(kTabBlock) k_fqe_weights(int n, const double *
 
 // out[k][j] for k < nbins on the accumulated log grid a_k = lo + (k+1) d - d
 // summed term by term as the reference's loops do (so a_k is bit-identical
-// to theirs, fp_shared_core.c:1735-1741); kind 0 gamma(E_k, p_j), 1 neutrino(E_k, p_j), 2 IC
-// emissivity(nu_k, gamma_j = sqrt(1 + p_j^2), z).
+// to theirs, fp_shared_core.c:1735-1741); kind 0 gamma(E_k, p_j), 1 neutrino(E_k, p_j).
 __global__ void __launch_bounds__(kTabBlock) k_emis_table(int kind, int n, int nbins, double lo, double d, double z,
                                                            const double *__restrict__ mom, double *out)
 {
+    (void)z;
     const int j = blockIdx.x * kTabBlock + threadIdx.x;
     const int k = blockIdx.y;
     if (j >= n || k >= nbins) return;
@@ -72,9 +73,82 @@ __global__ void __launch_bounds__(kTabBlock) k_emis_table(int kind, int n, int n
     const double p = mom[j];
     double v;
     if (kind == 0) v = chk_gamma_kernel(e, p);
-    else if (kind == 1) v = chk_nu_kernel(e, p);
-    else v = chk_ic_emissivity_kernel(e, sqrt(1.0 + p * p), z);
+    else v = chk_nu_kernel(e, p);
     out[(size_t)k * n + j] = v;
+}
+
+// Inverse-Compton emissivity table: out[k][j] = chk_ic_emissivity_kernel(nu_k,
+// sqrt(1 + p_j^2), z), the 400-node quadrature of FP_Coef.c:553-582, a table
+// per snapshot's redshift.  Bound: FP64 VALU (a pow, a log and an exp per
+// node).  One thread per entry left one wave per CU with 400 nodes in a row
+// (635 us for 64 x 256 entries); here eight lanes share an entry, 50 nodes
+// each, leave their trapezoid terms in LDS and the first of them adds the 400
+// terms in the serial order (238 us, the same bits).  The integrand's squares
+// are products and its constants are formed once, where the shared header's
+// pow calls took half of the 720 instructions of a node (148 us).
+__device__ __forceinline__ double ict_kernel(double eps0, double gamma, double eps)
+{
+#pragma clang fp contract(off)
+    const double re = 2.82e-13;
+    const double kappa = eps / (4.0 * eps0 * gamma * (gamma - eps));
+    if (kappa <= 0.0) return 0.0;
+    const double q = 4.0 * eps0 * kappa * gamma;
+    const double C = 2.0 * kappa * log(kappa) + (1.0 + 2.0 * kappa) * (1.0 - kappa) +
+                     q * q / (2.0 * (1.0 + 4.0 * eps0 * gamma * kappa)) * (1.0 - kappa);
+    return 2.0 * CHK_PI * re * re * CHK_C / (gamma * gamma * eps0) * C;
+}
+
+// pre = 8 pi c^3 (m_e / h)^3, kt = k T_cmb
+__device__ __forceinline__ double ict_cmb_n(double eps, double pre, double kt)
+{
+#pragma clang fp contract(off)
+    const double meg = 9.11e-28, tiny = 1.0e-40;
+    const double x = eps * meg * CHK_C * CHK_C / kt;
+    if (x > 90.0 * log(10.0)) return 0.0;
+    const double em1 = exp(x) - 1.0;
+    if (em1 < tiny) return pre * eps / (meg * CHK_C * CHK_C * (1.0 + 0.5 * x + x / 6.0) / kt);
+    return pre * (eps * eps) / em1;
+}
+
+constexpr int kIcLanes = 8, kIcNodes = 400, kIcRun = kIcNodes / kIcLanes, kIcGroups = 64 / kIcLanes;
+
+__global__ void __launch_bounds__(64) k_ic_table(int n, int nbins, double lo, double d, double z,
+                                                 const double *__restrict__ mom, double *out)
+{
+    CHK_NOCONTRACT
+    __shared__ double s_t[kIcGroups][kIcNodes + 1];
+    const int g = threadIdx.x / kIcLanes, c = threadIdx.x % kIcLanes;
+    const int j = blockIdx.x * kIcGroups + g, k = blockIdx.y;
+    const double meg = 9.11e-28, cl = 3.0e+10;
+    const double r = meg / CHK_H, pre = 8.0 * CHK_PI * CHK_C * CHK_C * CHK_C * (r * r * r);
+    const double kt = 1.38e-16 * (2.757 * (1.0 + z));
+    double ak = lo - d;
+    for (int kk = 0; kk <= k; kk++) ak += d;
+    const double nu = pow(10.0, ak);
+    const double eps = CHK_H * nu / (meg * cl * cl);
+    if (j < n) {
+        const double p = mom[j], gamma = sqrt(1.0 + p * p);
+        double e0max = eps, e0min = eps / (4.0 * gamma * (gamma - eps));
+        if (e0min < 0) e0min = eps / (gamma * gamma);
+        const double da = (log10(e0max) - log10(e0min)) / (double)kIcNodes;
+        double a = log10(e0min);
+        for (int i = 0; i < c * kIcRun; i++) a = a + da;
+        double e0n = pow(10.0, a), Cn = ict_kernel(e0n, gamma, eps), nn = ict_cmb_n(e0n, pre, kt);
+        for (int i = c * kIcRun; i < (c + 1) * kIcRun; i++) {
+            const double e0 = e0n, C = Cn, n0 = nn;
+            a = a + da;
+            e0n = pow(10.0, a);
+            nn = ict_cmb_n(e0n, pre, kt);
+            Cn = ict_kernel(e0n, gamma, eps);
+            s_t[g][i] = 0.5 * (C * n0 + Cn * nn) * (e0n - e0);
+        }
+    }
+    __syncthreads();
+    if (j < n && c == 0) {
+        double sum = 0.0;
+        for (int i = 0; i < kIcNodes; i++) sum = sum + s_t[g][i];
+        out[(size_t)k * n + j] = CHK_H * eps * sum / (4.0 * CHK_PI);
+    }
 }
 
 }  // namespace
@@ -95,6 +169,11 @@ extern "C" int ck_emission_kernel_table(int kind, int n, int nbins, double lo, d
 {
     if (n <= 0 || nbins <= 0 || nbins > 65535 || kind < 0 || kind > 2) return 1;
     const unsigned gx = (unsigned)((n + kTabBlock - 1) / kTabBlock);
+    if (kind == 2) {
+        hipLaunchKernelGGL(k_ic_table, dim3((unsigned)((n + kIcGroups - 1) / kIcGroups), (unsigned)nbins), dim3(64), 0,
+                           (hipStream_t)stream, n, nbins, lo, (hi - lo) / (double)nbins, z, mom, out);
+        return hipGetLastError() != hipSuccess;
+    }
     hipLaunchKernelGGL(k_emis_table, dim3(gx, (unsigned)nbins), dim3(kTabBlock), 0, (hipStream_t)stream, kind, n,
                        nbins, lo, (hi - lo) / (double)nbins, z, mom, out);
     return hipGetLastError() != hipSuccess;
