@@ -229,10 +229,12 @@ int ck_plain_scatter(int n, int count, const int *idx_dev, const CkSlot *slot_ho
                      void *stream);
 
 /* Batched tridiagonal Chang-Cooper solve (solve_cc_cuda_batch semantics):
- * state_out = Thomas(a,b,c; dt*Q + state_in), cell-major, one system per thread. */
+ * state_out = Thomas(a,b,c; dt*Q + state_in), cell-major.  *err_dev becomes
+ * `mark` if a pivot vanishes and is left alone otherwise; cprime_ws is used
+ * for nrow > 1024 only. */
 int ck_solve_cc_batch(int nsys, int nrow, double dt, const double *a, const double *b,
                       const double *c, const double *q, const double *state_in, double *state_out,
-                      double *cprime_ws, int *err_dev, void *stream);
+                      double *cprime_ws, int *err_dev, int mark, void *stream);
 
 /* Emission contractions: out[i][k] = row_scale[i] * sum_j spectra[i][j] kmat[j][k].
  * spectra [ntr x K] FP64; the kernel matrix in bin-major layout [nbins_pad][K]

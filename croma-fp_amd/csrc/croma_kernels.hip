@@ -331,14 +331,14 @@ __global__ void k_plain_thomas(int n, int count, int nstep, double dt, int windo
 
 // Systems longer than the lane-group kernel below takes: one thread each.
 __global__ void k_solve_cc_batch(int nsys, int nrow, double dt, const double *a, const double *b, const double *c,
-                                 const double *q, const double *xin, double *xout, double *cp, int *err)
+                                 const double *q, const double *xin, double *xout, double *cp, int *err, int mark)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nsys) return;
     const size_t off = (size_t)i * nrow;
     for (int j = 0; j < nrow; ++j) xout[off + j] = xin[off + j];
     const int bad = d_thomas_cc(nrow, dt, a + off, b + off, c + off, q + off, xout + off, cp + off);
-    if (bad) atomicOr(err, bad);
+    if (bad) *err = mark;
 }
 
 // Batched Chang-Cooper solve, one lane group of G lanes per system, R rows per
@@ -366,7 +366,7 @@ template <int R, int G>
 __global__ __launch_bounds__(64) void k_solve_group(int nsys, int nrow, double dt, const double *__restrict__ a,
                                                      const double *__restrict__ b, const double *__restrict__ c,
                                                      const double *__restrict__ q, const double *xin, double *xout,
-                                                     int *__restrict__ err)
+                                                     int *__restrict__ err, int mark)
 {
     constexpr int S = 64 / G;
     __shared__ double buf[64 * (R + 1)];
@@ -482,7 +482,7 @@ __global__ __launch_bounds__(64) void k_solve_group(int nsys, int nrow, double d
 #pragma unroll
     for (int i = 0; i < R; ++i)
         if (pos[i] >= 0) xout[off + i * 64 + lane] = buf[pos[i]];
-    if (bad) atomicOr(err, bad);
+    if (bad) *err = mark;
 }
 
 static int grid1d(size_t work, int block)
@@ -555,7 +555,7 @@ extern "C" int ck_plain_thomas(int n, int count, int nstep, double dt, int windo
 
 extern "C" int ck_solve_cc_batch(int nsys, int nrow, double dt, const double *a, const double *b, const double *c,
                                  const double *q, const double *xin, double *xout, double *cp, int *err,
-                                 void *stream)
+                                 int mark, void *stream)
 {
     hipStream_t st = (hipStream_t)stream;
     // Fewest rows per lane that a wave's 64 lanes cover, at least 4: a lane's
@@ -566,7 +566,7 @@ extern "C" int ck_solve_cc_batch(int nsys, int nrow, double dt, const double *a,
     if (nrow <= (R_) * (G_)) {                                                                                         \
         const long nb = ((long)nsys + 64 / (G_) - 1) / (64 / (G_));                                                    \
         hipLaunchKernelGGL((k_solve_group<R_, G_>), dim3((unsigned)nb), dim3(64), 0, st, nsys, nrow, dt, a, b, c, q,   \
-                           xin, xout, err);                                                                            \
+                           xin, xout, err, mark);                                                                      \
         return hip_ok(hipGetLastError(), "k_solve_group");                                                             \
     }
     CK_SOLVE_CASE(4, 2)
@@ -579,7 +579,7 @@ extern "C" int ck_solve_cc_batch(int nsys, int nrow, double dt, const double *a,
     CK_SOLVE_CASE(16, 64)
 #undef CK_SOLVE_CASE
     hipLaunchKernelGGL(k_solve_cc_batch, dim3(grid1d((size_t)nsys, 64)), dim3(64), 0, st, nsys, nrow, dt, a, b, c, q,
-                       xin, xout, cp, err);
+                       xin, xout, cp, err, mark);
     return hip_ok(hipGetLastError(), "k_solve_cc_batch");
 }
 

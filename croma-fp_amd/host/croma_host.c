@@ -2250,7 +2250,7 @@ int croma_hip_solve_cc_batch(int nsys, int nrow, double dt, const double *a, con
     if (ck_fill_i32(derr, 0, 1, s) || ck_h2d(d, a, m * 8, s) || ck_h2d(d + m, bb, m * 8, s) ||
         ck_h2d(d + 2 * m, cc, m * 8, s) || ck_h2d(d + 3 * m, src, m * 8, s) || ck_h2d(d + 4 * m, st_in, m * 8, s) ||
         ck_event_record(e0, s) ||
-        ck_solve_cc_batch(nsys, nrow, dt, d, d + m, d + 2 * m, d + 3 * m, d + 4 * m, d + 5 * m, d + 6 * m, derr, s) ||
+        ck_solve_cc_batch(nsys, nrow, dt, d, d + m, d + 2 * m, d + 3 * m, d + 4 * m, d + 5 * m, d + 6 * m, derr, 1, s) ||
         ck_event_record(e1, s) || ck_d2h(st_out, d + 5 * m, m * 8, s) || ck_d2h(&err, derr, sizeof(int), s) ||
         ck_stream_sync(s)) {
         rc = dev_fail("solve");
