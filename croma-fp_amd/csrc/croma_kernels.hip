@@ -36,6 +36,9 @@ static int hip_ok(hipError_t e, const char *what)
 {
     if (e == hipSuccess) return 0;
     snprintf(g_errbuf, sizeof(g_errbuf), "%s: %s", what, hipGetErrorString(e));
+    // reported here: the check after the next launch, for a caller that goes
+    // on without what failed (memory, a capture), must not see it again
+    (void)hipGetLastError();
     return -1;
 }
 

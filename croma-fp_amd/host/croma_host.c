@@ -338,14 +338,16 @@ static int tile_f32_ok(const CromaHipContext *c, int protons, int r, int w, int 
  * 4083, 6,000 x 128 4104 / 5469, 16,000 x 128 2520 / 2860, 32,000 x 128 3245 /
  * 4619, 32,000 x 256 5770 / 6744, 60,000 x 64 3126 / 4183; both species,
  * split 2,000 x 256 5373 / 6599 (pipelined 3932), 300 x 512 7243 / 8300
- * (pipelined 5305). */
-static CromaHipTile run_tile(const CromaHipContext *c, int protons, long ntr, int run)
+ * (pipelined 5305).  in_kernel: both species without the split launch. */
+static CromaHipTile run_tile(const CromaHipContext *c, int protons, long ntr, int run, int in_kernel)
 {
     const int n = c->g.n, p = protons ? 1 : 0;
     const long rows = ntr * (long)n;
-    const int split = p && c->tile[1].secondary_gemm && !(c->prm.dpp_model != 3 && c->prm.eta_dpp_cap > 0.0);
+    const int split = p && !in_kernel && c->tile[1].secondary_gemm &&
+                      !(c->prm.dpp_model != 3 && c->prm.eta_dpp_cap > 0.0);
     CromaHipTile t = c->tile[p];
     if (c->tile_set[p]) return t;
+    if (in_kernel) t.secondary_gemm = 0;
     if (!p) {
         if (n == 64) t.rows_per_lane = rows <= CH_ROWS_LATENCY ? 4 : 8;
         else if (n <= 256) t.rows_per_lane = (n == 128 && rows <= CH_ROWS_LATENCY) ? 4 : rows <= CH_ROWS_MIDDLE ? 8 : 16;
@@ -840,7 +842,7 @@ const ChGrid *ch_ctx_grid(const CromaHipContext *c) { return &c->g; }
 const CkGrid *ch_ctx_dgrid(const CromaHipContext *c) { return &c->dgrid; }
 const CkParams *ch_ctx_prm(const CromaHipContext *c) { return &c->prm; }
 int ch_ctx_cu_count(const CromaHipContext *c) { return c->cu_count; }
-CromaHipTile ch_ctx_tile(const CromaHipContext *c, int protons, long ntr) { return run_tile(c, protons, ntr, 1); }
+CromaHipTile ch_ctx_tile(const CromaHipContext *c, int protons, long ntr) { return run_tile(c, protons, ntr, 1, 0); }
 const double *ch_ctx_d_fqe(const CromaHipContext *c) { return c->d_fqe; }
 /* np_min of the secondary weights on the device (after the weights and beta_p) */
 const int *ch_ctx_d_npmin(const CromaHipContext *c) { return c->d_fqe ? (const int *)(c->d_fqe + (size_t)c->g.n * c->g.n + c->g.n) : 0; }
@@ -1135,7 +1137,7 @@ CromaHipBatch *croma_hip_batch_create(CromaHipContext *c, int ntr, int species, 
         !b->ev_a || !b->ev_b || !b->d_cells)
         goto fail;
     for (k = 0; k < 2; k++)
-        if (win_reserve(c, &b->win[k], run_tile(c, b->protons, ntr, nsnap_res).chain, ntr, 0)) goto fail;
+        if (win_reserve(c, &b->win[k], run_tile(c, b->protons, ntr, nsnap_res, 0).chain, ntr, 0)) goto fail;
     if (b->protons && ch_ctx_fqe(c) != 0) goto fail;
     return b;
 fail:
@@ -1817,12 +1819,11 @@ int croma_hip_batch_sync(CromaHipBatch *b)
     return 0;
 }
 
-/* Segment rows of a window of wsz snapshots (split launches). */
-static int reserve_segrows(CromaHipBatch *b, int wsz)
+/* Segment rows of split launches: two arrays of at least `need` rows. */
+static int reserve_segrows(CromaHipBatch *b, long need)
 {
     CromaHipContext *c = b->ctx;
-    const long segmax = c->prm.coeff_interp_max_segments > 1 ? c->prm.coeff_interp_max_segments : 1;
-    long need = (long)wsz * b->ntr * segmax, q = 256;
+    long q = 256;
     while (q < need / 64) q <<= 1;
     need = (need + q - 1) / q * q;
     if (need > b->segrows_cap) {
@@ -1831,12 +1832,16 @@ static int reserve_segrows(CromaHipBatch *b, int wsz)
         ck_free(b->d_segrec);
         ck_free(b->d_seginje);
         b->d_segrec = (double *)ck_malloc(cnt * sizeof(double));
-        b->d_seginje = (double *)ck_malloc(cnt * sizeof(double));
-        b->segrows_cap = (b->d_segrec && b->d_seginje) ? need : 0;
-        if (!b->segrows_cap) return dev_fail("segment rows");
+        b->d_seginje = b->d_segrec ? (double *)ck_malloc(cnt * sizeof(double)) : 0;
+        b->segrows_cap = b->d_seginje ? need : 0;
+        if (!b->segrows_cap) {
+            ck_free(b->d_segrec);
+            b->d_segrec = 0;
+            return -1;
+        }
         /* rows past a window's segment count enter the rounded GEMM: keep them finite */
         if (ck_fill_f64(b->d_segrec, 0.0, cnt, c->stream) || ck_fill_f64(b->d_seginje, 0.0, cnt, c->stream))
-            return dev_fail("segment rows");
+            return -1;
     }
     b->seg_quantum = q;
     return 0;
@@ -1857,7 +1862,7 @@ int croma_hip_batch_run(CromaHipBatch *b, int s0, int s1, int nsnap_total, const
         return CROMA_HIP_EINVAL;
     if (s1 == s0) return 0;
     c = b->ctx;
-    b->tile = run_tile(c, b->protons, b->ntr, s1 - s0);
+    b->tile = run_tile(c, b->protons, b->ntr, s1 - s0, 0);
     b->pipe = c->pipeline < 0 ? (long)b->ntr * c->g.n <= CH_ROWS_PIPE : c->pipeline;
     wsz = (path == CROMA_HIP_PATH_FUSED) ? b->tile.chain : 1;
     if (wsz > s1 - s0) wsz = s1 - s0;
@@ -1866,7 +1871,10 @@ int croma_hip_batch_run(CromaHipBatch *b, int s0, int s1, int nsnap_total, const
             !(c->prm.dpp_model != 3 && c->prm.eta_dpp_cap > 0.0);
     /* the plain path keeps the reference's host-side buckets */
     dev_nsub = path == CROMA_HIP_PATH_FUSED && c->nsub_device;
-    if (split && (rc = reserve_segrows(b, wsz)) != 0) return rc;
+    if (split) {
+        const long segmax = c->prm.coeff_interp_max_segments > 1 ? c->prm.coeff_interp_max_segments : 1;
+        if (reserve_segrows(b, (long)wsz * b->ntr * segmax)) return dev_fail("segment rows");
+    }
     nwin = (s1 - s0 + wsz - 1) / wsz;
     for (k = 0; k < 2; k++)
         if ((rc = win_reserve(c, &b->win[k], wsz, b->ntr, !dev_nsub)) != 0) return rc;
@@ -1996,6 +2004,17 @@ static int snapshot_npmin(int n, int jp0, const double *fqe, int *first)
                 open--;
             }
     return 1;
+}
+
+/* Segment rows of one drop-in call: those the context holds, or new ones that
+ * leave at least as much device memory free as they take (the in-kernel
+ * contraction needs none, so a call that finds no room for them still runs). */
+static int snapshot_segrows(CromaHipBatch *b, long rows)
+{
+    size_t left = 0, total = 0;
+    if (rows <= b->segrows_cap) return 0;
+    if (ck_mem_info(&left, &total) || (size_t)rows * b->ctx->g.n * 2 * sizeof(double) > left / 2) return -1;
+    return reserve_segrows(b, rows);
 }
 
 /* ------------------------------------------------------------------ */
@@ -2153,22 +2172,27 @@ int croma_hip_execute_snapshot(
         S->elapsed = elapsed;
         S->prm = prm;
         /* two species without the eta cap: the split launch (a third to a half
-         * of the in-kernel contraction's time), when its instances exist */
-        b->tile = run_tile(c, protons, ntr, 1);
+         * of the in-kernel contraction's time), when its instances exist and
+         * there is room for the rows of the call's own substep counts (as
+         * many as int counts: more would not fit any device) */
+        b->tile = run_tile(c, protons, ntr, 1, 0);
         if (protons && b->tile.secondary_gemm && !(prm.dpp_model != 3 && prm.eta_dpp_cap > 0.0) &&
             (!c->coeff_fp32 || tile_f32_ok(c, 1, b->tile.rows_per_lane, b->tile.waves_per_simd, 1)) &&
             snapshot_npmin(n, jp0, fqe_flat, npm)) {
             long segrows = 0;
-            if ((rc = reserve_segrows(b, 1)) != 0) goto done;
             for (i = 0; i < ntr; i++) {
                 w->h_segoff[i] = (int)segrows;
                 segrows += ch_choose_segments(&prm, nsubsteps[i], allow);
             }
+            split = snapshot_segrows(b, segrows) == 0;
             npm[n] = (int)segrows;
+        }
+        if (split) {
             S->seg_off = w->d_segoff;
             S->seg_rec = b->d_segrec;
             S->seg_inje = b->d_seginje;
-            split = 1;
+        } else if (protons) {
+            b->tile = run_tile(c, 1, ntr, 1, 1);
         }
         if ((split && (ck_h2d(w->d_segoff, w->h_segoff, (size_t)ntr * sizeof(int), c->stream) ||
                        ck_h2d(d_npm, npm, ((size_t)n + 1) * sizeof(int), c->stream))) ||

@@ -3,12 +3,14 @@ several snapshots in one window equals the same snapshots run one at a time
 bit for bit, and a run at a fixed tile to rounding; the drop-in's split launch
 equals the in-kernel contraction that weights below the first proton row ask
 for."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import croma_hip as ch
 import synth
-from workloads import hip_params, small_workload
+from workloads import hip_params, run_hip, small_workload
 
 pytestmark = pytest.mark.gpu
 
@@ -90,3 +92,44 @@ def test_snapshot_split_equals_in_kernel_contraction(n):
     for a, b in zip(*out):
         m = np.abs(b) > 1e-30
         assert np.max(np.abs(a[m] - b[m]) / np.abs(b[m])) < 1e-11
+
+
+def test_snapshot_rows_follow_the_substep_counts():
+    """Two species, as many segments allowed as a call could ask for: the rows
+    reserved are those of the calls' own substep counts, and the result is that
+    of a limit no tracer reaches."""
+    n = 64
+    w = small_workload(n, 75, 1, 3, 1, seed=5)
+    out = []
+    for segs in (4096, 1 << 24):  # 75 x 2^24 rows of 64 bins: 1.3e12 bytes
+        ctx = ch.Context(n, hip_params(w, coeff_interp_max_segments=segs, coeff_interp_min_steps=2))
+        try:
+            row, m1, p1 = ctx.ic_cooling_row(float(w.z[0]))
+            f = w.bg[0]
+            ns, non = ctx.nsub(float(w.dt_snap[0]), f[0], f[1], f[2], f[3], row[0], row[-1], f[4], f[5])
+            assert ns.max() // 2 < 4096
+            fqe, npmin = ctx.secondary_weights()
+            crp, cre = w.crp0.copy(), w.cre0.copy()
+            zero = np.zeros(w.ntracer * n)
+            ctx.execute_snapshot(ns, non, True, 0.0, float(w.dt_snap[0]), f, row, m1, p1, w.bg[1], row, m1, p1, zero,
+                                 zero, fqe.ravel(), npmin, w.mass, None, crp, cre)
+            out.append((crp, cre))
+        finally:
+            ctx.close()
+    for a, b in zip(*out):
+        assert np.all(np.isfinite(a)) and np.array_equal(a, b)
+
+
+def test_failed_allocation_leaves_no_error_behind():
+    """A refused allocation is reported by its own call, not by the check after
+    the next launch (a call that does without what it could not get goes on)."""
+    ck_malloc = ch.lib().ck_malloc
+    ck_malloc.restype, ck_malloc.argtypes = C.c_void_p, [C.c_size_t]
+    w = small_workload(64, 20, 1, 1, 1)
+    ctx = ch.Context(64, hip_params(w))
+    try:
+        want = run_hip(w, ctx)[1]
+        assert not ck_malloc(1 << 50)
+        assert np.array_equal(run_hip(w, ctx)[1], want)
+    finally:
+        ctx.close()

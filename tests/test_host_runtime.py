@@ -1,0 +1,106 @@
+"""The C host runtime on a stand-in for the device layer (device_stub.c, host
+memory, kernels that compute nothing and are recorded): which launches a call
+takes, what it reserves and what it does when a reservation fails.  No GPU."""
+import ctypes as C
+import glob
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+import croma_hip as ch
+
+REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+PKG = os.path.join(REPO, "croma-fp_amd")
+
+
+@pytest.fixture(scope="module")
+def stub_path(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("stub") / "libcroma_stub.so")
+    subprocess.check_call(["gcc", "-shared", "-fPIC", "-O1", "-std=gnu11", "-ffp-contract=off", "-pthread", "-w",
+                           "-I", os.path.join(PKG, "csrc"), "-I", os.path.join(REPO, "include"), "-o", out,
+                           *sorted(glob.glob(os.path.join(PKG, "host", "*.c"))),
+                           os.path.join(REPO, "tests", "device_stub.c"), "-lm"])
+    return out
+
+
+@pytest.fixture
+def stub(stub_path, monkeypatch):
+    monkeypatch.setattr(ch, "LIB_PATH", stub_path)
+    monkeypatch.setattr(ch, "_lib", None)
+    L = ch.lib()
+    L.stub_peak.restype = L.stub_live.restype = C.c_size_t
+    L.stub_set_limit.argtypes = [C.c_size_t, C.c_size_t]
+    L.ck_set_device(0)
+    L.stub_reset()
+    yield L
+    L.ck_set_device(0)
+
+
+def _launches(L):
+    m, r, t = ((C.c_int * 4096)() for _ in range(3))
+    k = L.stub_launches(m, r, t, 4096)
+    return [(m[i], r[i], t[i]) for i in range(k)]
+
+
+def _snapshot(ctx, nt, nsub):
+    n = ctx.n
+    bg = np.ones((8, nt))
+    row = np.ones(n)
+    fqe = np.zeros((n, n))
+    fqe[n // 2:] = 1.0
+    x = np.ones(nt * n)
+    zero = np.zeros(nt * n)
+    crp, cre = x.copy(), x.copy()
+    nsub = np.asarray(nsub, np.int32)
+    ctx.execute_snapshot(nsub, nsub, True, 0.0, 0.01, bg, row, 1.0, 1.0, bg, row, 1.0, 1.0, zero, zero, fqe.ravel(),
+                         np.full(n, n // 2, np.int32), np.ones(nt), None, crp, cre)
+    return crp, cre
+
+
+# tracers, substeps, most segments: the rows that the calls' own substep
+# counts ask for, not tracers x most segments
+@pytest.mark.parametrize("nt,nsub,segs", [(500, 4, 16), (300, 37, 4096), (64, 4096, 1024)])
+def test_drop_in_reserves_the_rows_it_writes(stub, nt, nsub, segs):
+    n = 64
+    ctx = ch.Context(n, ch.default_params(coeff_interp_max_segments=segs, coeff_interp_min_steps=4))
+    try:
+        _snapshot(ctx, nt, np.full(nt, nsub))
+        assert [m for m, _, _ in _launches(stub)] == [2, 3]  # the split launch
+        most = 1
+        while most * 2 <= min(segs, nsub // 4):
+            most *= 2
+        rows = nt * most
+        # two arrays of rows, rounded up by at most 1/32 and 256 rows; the state,
+        # sources and backgrounds are below 8 arrays of the spectra and the weights
+        other = 8 * nt * n * 8 + 4 * n * n * 8 + (1 << 20)
+        assert stub.stub_peak() <= 2 * (rows * (1 + 1 / 32) + 256) * n * 8 + other
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+def test_drop_in_without_room_for_the_rows_runs_the_in_kernel_contraction(stub, fp32):
+    n, nt = 128, 400
+    ctx = ch.Context(n, ch.default_params(coeff_interp_max_segments=1024, coeff_interp_min_steps=1))
+    try:
+        ctx.set_coeff_precision(fp32)
+        state = nt * n * 8
+        for largest, free in ((4 * state, 1 << 38), (1 << 40, 100 * state)):
+            stub.stub_reset()
+            stub.stub_set_limit(largest, free)
+            before = stub.stub_live()
+            crp, cre = _snapshot(ctx, nt, np.full(nt, 1024))  # 1024 segments: 2048 x state
+            modes = [m & ~4 if fp32 else m for m, _, _ in _launches(stub)]
+            assert modes == [1]
+            assert np.all(crp == 1.0) and np.all(cre == 1.0)
+            # nothing of a failed reservation is left
+            assert stub.stub_live() - before < 12 * state + (4 << 20)
+        # fewer segments: room again
+        stub.stub_reset()
+        stub.stub_set_limit(1 << 40, 1 << 38)
+        _snapshot(ctx, nt, np.full(nt, 16))
+        assert [m & ~4 if fp32 else m for m, _, _ in _launches(stub)] == [2, 3]
+    finally:
+        ctx.close()
