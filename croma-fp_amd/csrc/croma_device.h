@@ -1389,8 +1389,10 @@ __device__ __forceinline__ void seg_radp_e(const SpGridT<T> &sg, const double *r
         const int j = base + k;
         const T pe = sg.x[sg.ix(j)];
         const T pe2 = sg.p2[sg.ix(j)];
-        // both rows loaded unconditionally (ric_n is always a valid row); alpha
-        // is 0 (exactly the current row) without interpolation, below 1 with it
+        // both rows loaded unconditionally; alpha is 0 (exactly the current row)
+        // without interpolation, below 1 with it.  ric_n holds finite values or
+        // is the current row: the host sees to it, since a select here or on
+        // the pointer costs 1% of a small launch
         const T ric = (T)(ric_c[j] + alpha * (ric_n[j] - ric_c[j]));
         const T coul = coul_coeff * ((T)1.0 + (sg.lnp[sg.ix(j)] + lning) * (T)(1.0 / 74.8)) * sg.ib2[sg.ix(j)];
         radp[k] = synch * pe2 + ric + coul + adia * pe;

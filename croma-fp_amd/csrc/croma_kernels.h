@@ -74,7 +74,7 @@ typedef struct {
     const double *bgc[CK_NBG];    /* current snapshot backgrounds [ntr] */
     const double *bgn[CK_NBG];    /* next snapshot backgrounds [ntr] */
     const double *ric_c;          /* IC cooling row at z_curr [n] */
-    const double *ric_n;          /* IC cooling row at z_next [n] */
+    const double *ric_n;          /* IC cooling row at z_next [n]; ric_c where no segment interpolates */
     const int *nsub;              /* [ntr] */
     const int *n_on;              /* [ntr] */
     const double *fqe_t;          /* [n * n] secondary weights (transposed) or NULL */

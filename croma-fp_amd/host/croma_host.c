@@ -2160,7 +2160,11 @@ int croma_hip_execute_snapshot(
             S->bgn[i] = b->d_bg + ((size_t)CK_NBG + i) * ntr;
         }
         S->ric_c = d_ric;
-        S->ric_n = d_ric + n;
+        /* the caller's next row may hold anything where no tracer interpolates
+         * (more substeps never mean fewer segments) */
+        for (i = 0, j = 1; i < ntr; i++)
+            if (nsubsteps[i] > j) j = nsubsteps[i];
+        S->ric_n = ch_choose_segments(&prm, j, allow) > 1 ? d_ric + n : d_ric;
         S->nsub = d_nsub;
         S->n_on = d_non;
         S->fqe_t = protons ? d_fqe : 0;

@@ -43,3 +43,34 @@ def test_segments_match_oracle(case):
     finally:
         ctx.close()
     assert np.all(np.isfinite(cre))
+
+
+@pytest.mark.parametrize("n,species", [(64, 1), (128, 3), (256, 3), (512, 1)])
+@pytest.mark.parametrize("fp32", [False, True])
+def test_uninterpolated_segments_ignore_the_next_row(n, species, fp32):
+    """Drop-in calls without interpolation, by the flag or because every tracer
+    has one segment: the next IC row and backgrounds may hold anything."""
+    w = small_workload(n, 21, 1, species, 1, seed=11)
+    nt = w.ntracer
+    crp0 = w.crp0 if w.protons else np.zeros(nt * n)
+    zero = np.zeros(nt * n)
+    for allow, extra in ((False, {}), (True, {"coeff_interp_max_segments": 1})):
+        ctx = ch.Context(n, hip_params(w, **extra))
+        try:
+            ctx.set_coeff_precision(fp32)
+            row, m1, p1 = ctx.ic_cooling_row(float(w.z[0]))
+            f = w.bg[0]
+            ns, non = ctx.nsub(float(w.dt_snap[0]), f[0], f[1], f[2], f[3], row[0], row[-1], f[4], f[5])
+            fqe, npmin = ctx.secondary_weights()
+            out = []
+            for nxt in (1.0, np.inf, -np.inf, np.nan):
+                crp, cre = crp0.copy(), w.cre0.copy()
+                ctx.execute_snapshot(ns, non, allow, 0.0, float(w.dt_snap[0]), f, row, m1, p1,
+                                     np.full((8, nt), nxt), np.full(n, nxt), nxt, nxt, zero, zero, fqe.ravel(), npmin,
+                                     w.mass, None, crp, cre)
+                out.append((crp, cre))
+        finally:
+            ctx.close()
+        assert np.all(np.isfinite(out[0][1]))
+        for crp, cre in out[1:]:
+            assert np.array_equal(cre, out[0][1]) and np.array_equal(crp, out[0][0])
