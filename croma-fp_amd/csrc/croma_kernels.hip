@@ -355,16 +355,25 @@ __global__ void k_solve_cc_batch(int nsys, int nrow, double dt, const double *a,
 // each lane runs the recurrences over its own rows from a value entering it,
 // first guessed from a scan across the lanes, and repeats them with the value
 // that the lane before (after, in the back substitution) came out with until
-// every entering value equals it.  The guesses are a few ulp off and the
+// every entering value has its bits.  The guesses are a few ulp off and the
 // recurrences of diagonally dominant systems contract, so two or three rounds
 // are the rule; whatever the system, lane l is exact after l + 1 rounds, which
-// bounds the loops and makes no assumption on signs or dominance.
+// bounds the loops and makes no assumption on signs, dominance or finite
+// values.  The rows past nrow take in whatever the last row comes out with, so
+// their results and the multipliers that would bring these back are set to 0,
+// and the sums that the sweep does not form (before the first row, after the
+// last) add -0, which changes no value.
 //
 // 8,192 x 512 rows: 760 -> 77 us (2.6 TB/s of 48 B per row; the rest is the division
 // chains, about 1,400 vector instructions per wave); 64 x 64: 91 -> 7.4 us.  One
 // wave per block, so that waves retire and start one by one (82 us with four).
 // The one-thread kernel read rows 8 nrow bytes apart across the lanes of a
 // wave and waited for HBM at every row.
+__device__ __forceinline__ bool bits_differ(double a, double b)
+{
+    return __double_as_longlong(a) != __double_as_longlong(b);
+}
+
 template <int R, int G>
 __global__ __launch_bounds__(64) void k_solve_group(int nsys, int nrow, double dt, const double *__restrict__ a,
                                                      const double *__restrict__ b, const double *__restrict__ c,
@@ -411,7 +420,7 @@ __global__ __launch_bounds__(64) void k_solve_group(int nsys, int nrow, double d
     take(vb, B, 1.0);
     take(vc, C, 0.0);
     take(vx, X, 0.0);
-    if (gl == 0) A[0] = 0.0;
+    if (gl == 0) A[0] = -0.0;
 #pragma unroll
     for (int k = 0; k < R; ++k)
         if (gl * R + k == nrow - 1) C[k] = 0.0;
@@ -428,13 +437,16 @@ __global__ __launch_bounds__(64) void k_solve_group(int nsys, int nrow, double d
             cp[k] = p;
         }
         const double prev = wave_up1(p);
-        if (it == G - 1 || !__any(gl > 0 && !(prev == in))) break;
+        if (it == G - 1 || !__any(gl > 0 && bits_differ(prev, in))) break;
         in = (gl == 0) ? 0.0 : prev;
     }
     int bad = 0;
 #pragma unroll
     for (int k = 0; k < R; ++k)
         if (fabs(den[k]) <= 1.0e-300) bad = ERR_PIVOT;
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+        if (gl * R + k >= nrow - 1) cp[k] = 0.0;
 
     // forward elimination, then back substitution; the scans only supply the
     // first entering values
@@ -459,9 +471,12 @@ __global__ __launch_bounds__(64) void k_solve_group(int nsys, int nrow, double d
             d[k] = p;
         }
         const double prev = wave_up1(p);
-        if (it == G - 1 || !__any(gl > 0 && !(prev == in))) break;
+        if (it == G - 1 || !__any(gl > 0 && bits_differ(prev, in))) break;
         in = (gl == 0) ? 0.0 : prev;
     }
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+        if (gl * R + k >= nrow) d[k] = 0.0;
     double M = d[R - 1];
 #pragma unroll
     for (int k = R - 2; k >= 0; --k) M = fma(-cp[k], M, d[k]);
@@ -475,7 +490,7 @@ __global__ __launch_bounds__(64) void k_solve_group(int nsys, int nrow, double d
             X[k] = p;
         }
         const double next = wave_dn1(p);
-        if (it == G - 1 || !__any(gl < G - 1 && !(next == in))) break;
+        if (it == G - 1 || !__any(gl < G - 1 && bits_differ(next, in))) break;
         in = (gl == G - 1) ? 0.0 : next;
     }
     wave_sync();
