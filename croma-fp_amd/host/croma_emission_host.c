@@ -266,7 +266,9 @@ struct CromaHipSynchPlan {
 
 void croma_hip_synch_plan_destroy(CromaHipSynchPlan *p)
 {
+    int prev;
     if (!p) return;
+    prev = ch_device_enter(p->device);
     if (p->stream) ck_stream_sync(p->stream);
     ck_free(p->d_const);
     ck_free(p->d_run);
@@ -274,16 +276,18 @@ void croma_hip_synch_plan_destroy(CromaHipSynchPlan *p)
     if (p->e1) ck_event_destroy(p->e1);
     if (p->stream) ck_stream_destroy(p->stream);
     ch_stage_unref(p->device);
+    ch_device_leave(prev);
     free(p);
 }
+
+static int plan_fill(CromaHipSynchPlan *p, const double *table, const ChGrid *g);
 
 CromaHipSynchPlan *croma_hip_synch_plan_create(const CromaHipContext *ctx, int nfreq, int nlogb, double logb_min,
                                                double inv_dlogb, const double *table, double *elapsed_ms)
 {
     CromaHipSynchPlan *p;
     const ChGrid *g;
-    size_t ntab, nkt, ncs;
-    char *q;
+    int prev, rc;
     if (!ctx || nfreq <= 0 || nlogb < 2 || !table || !isfinite(logb_min) || !isfinite(inv_dlogb)) {
         ch_set_error("synch plan: invalid arguments");
         return 0;
@@ -304,19 +308,32 @@ CromaHipSynchPlan *croma_hip_synch_plan_create(const CromaHipContext *ctx, int n
     p->nlogb = nlogb;
     p->logb_min = logb_min;
     p->inv_dlogb = inv_dlogb;
-    ntab = (size_t)nlogb * nfreq * p->n;
-    nkt = (size_t)(nlogb - 1) * 2 * ((nfreq + 15) / 16) * 64 * p->n;
-    ncs = (size_t)(nlogb - 1) * nfreq;
+    prev = ch_device_enter(p->device);
+    rc = prev < 0 || plan_fill(p, table, g);
+    ch_device_leave(prev);
+    if (rc) {
+        ch_set_error("synch plan: %s", ck_last_error());
+        croma_hip_synch_plan_destroy(p);
+        return 0;
+    }
+    if (elapsed_ms) *elapsed_ms = ck_event_elapsed_ms(p->e0, p->e1);
+    return p;
+}
+
+/* The plan's stream, events and memory, and its table's MFMA form. */
+static int plan_fill(CromaHipSynchPlan *p, const double *table, const ChGrid *g)
+{
+    const int nfreq = p->nfreq, nlogb = p->nlogb;
+    const size_t ntab = (size_t)nlogb * nfreq * p->n;
+    const size_t nkt = (size_t)(nlogb - 1) * 2 * ((nfreq + 15) / 16) * 64 * p->n;
+    const size_t ncs = (size_t)(nlogb - 1) * nfreq;
+    char *q;
     p->d_const = (char *)ck_malloc(SY_R(ntab * 8) + SY_R((size_t)p->n * 8) + 2 * SY_R(nkt * 2) + SY_R(ncs * 4) +
                                    SY_R(ntab * 4));
     p->stream = ck_stream_create();
     p->e0 = ck_event_create();
     p->e1 = ck_event_create();
-    if (!p->d_const || !p->stream || !p->e0 || !p->e1) {
-        ch_set_error("synch plan: device allocation: %s", ck_last_error());
-        croma_hip_synch_plan_destroy(p);
-        return 0;
-    }
+    if (!p->d_const || !p->stream || !p->e0 || !p->e1) return -1;
     q = p->d_const;
     p->d_tab = (double *)q;
     q += SY_R(ntab * 8);
@@ -329,23 +346,16 @@ CromaHipSynchPlan *croma_hip_synch_plan_create(const CromaHipContext *ctx, int n
     p->d_cs = (int *)q;
     q += SY_R(ncs * 4);
     p->d_lt = (float *)q;
-    if (ch_stage_h2d(p->device, p->d_tab, table, ntab * 8, p->stream) || ck_h2d(p->d_dp, g->edp, (size_t)p->n * 8, p->stream) ||
-        ck_event_record(p->e0, p->stream) ||
-        ck_synch_mfma_prepare(p->n, nfreq, nlogb, p->d_tab, p->d_dp, p->d_hi, p->d_lo, p->d_cs, p->d_lt, p->stream) ||
-        ck_event_record(p->e1, p->stream) || ck_stream_sync(p->stream)) {
-        ch_set_error("synch plan: %s", ck_last_error());
-        croma_hip_synch_plan_destroy(p);
-        return 0;
-    }
-    if (elapsed_ms) *elapsed_ms = ck_event_elapsed_ms(p->e0, p->e1);
-    return p;
+    return ch_stage_h2d(p->device, p->d_tab, table, ntab * 8, p->stream) ||
+           ck_h2d(p->d_dp, g->edp, (size_t)p->n * 8, p->stream) || ck_event_record(p->e0, p->stream) ||
+           ck_synch_mfma_prepare(p->n, nfreq, nlogb, p->d_tab, p->d_dp, p->d_hi, p->d_lo, p->d_cs, p->d_lt,
+                                 p->stream) ||
+           ck_event_record(p->e1, p->stream) || ck_stream_sync(p->stream);
 }
 
-int croma_hip_synch_plan_run(CromaHipSynchPlan *p, int ntr, const double *cre, const double *b_field, double *eps,
-                             double *elapsed_ms)
+static int plan_run(CromaHipSynchPlan *p, int ntr, const double *cre, const double *b_field, double *eps)
 {
-    const int n = p ? p->n : 0;
-    if (!p || ntr <= 0 || !cre || !b_field || !eps) return CROMA_HIP_EINVAL;
+    const int n = p->n;
     if (ntr > p->cap) {
         const size_t nt = (size_t)ntr;
         char *q;
@@ -380,10 +390,21 @@ int croma_hip_synch_plan_run(CromaHipSynchPlan *p, int ntr, const double *cre, c
         ch_set_error("synch MFMA: %s", ck_last_error());
         return CROMA_HIP_EDEVICE;
     }
-    if (elapsed_ms) *elapsed_ms = ck_event_elapsed_ms(p->e0, p->e1);
     return 0;
 }
 #undef SY_R
+
+int croma_hip_synch_plan_run(CromaHipSynchPlan *p, int ntr, const double *cre, const double *b_field, double *eps,
+                             double *elapsed_ms)
+{
+    int prev, rc;
+    if (!p || ntr <= 0 || !cre || !b_field || !eps) return CROMA_HIP_EINVAL;
+    if ((prev = ch_device_enter(p->device)) < 0) return CROMA_HIP_EDEVICE;
+    rc = plan_run(p, ntr, cre, b_field, eps);
+    if (!rc && elapsed_ms) *elapsed_ms = ck_event_elapsed_ms(p->e0, p->e1);
+    ch_device_leave(prev);
+    return rc;
+}
 
 static int synch_mfma(const CromaHipContext *ctx, int ntr, int nfreq, int nlogb, double logb_min, double inv_dlogb,
                       const double *table, const double *cre, const double *b_field, double *eps, double *elapsed_ms)

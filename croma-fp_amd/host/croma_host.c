@@ -787,19 +787,31 @@ int croma_hip_emission_kernel_table(const CromaHipContext *cc, int kind, int nbi
 
 int ch_ctx_device(const CromaHipContext *c) { return c->device; }
 
+int ch_device_enter(int dev)
+{
+    const int prev = ck_get_device();
+    return prev == dev || (prev >= 0 && ck_set_device(dev) == 0) ? prev : -1;
+}
+
+void ch_device_leave(int prev)
+{
+    if (prev >= 0 && prev != ck_get_device()) ck_set_device(prev);
+}
+
 char *ch_work_take(const CromaHipContext *cc, size_t bytes, ChWork *w)
 {
     CromaHipContext *c = (CromaHipContext *)cc;
     char *p;
     memset(w, 0, sizeof(*w));
+    if ((w->prev = ch_device_enter(c->device)) < 0) return 0;
     pthread_mutex_lock(&c->work_lock);
     if (!c->work_busy) {
         c->work_busy = 1;
+        c->work.prev = w->prev;
         *w = c->work;
         w->kept = 1;
     }
     pthread_mutex_unlock(&c->work_lock);
-    w->device = c->device;
     if (!w->stream) w->stream = ck_stream_create();
     if (!w->e0) w->e0 = ck_event_create();
     if (!w->e1) w->e1 = ck_event_create();
@@ -821,6 +833,7 @@ char *ch_work_take(const CromaHipContext *cc, size_t bytes, ChWork *w)
 void ch_work_give(const CromaHipContext *cc, ChWork *w)
 {
     CromaHipContext *c = (CromaHipContext *)cc;
+    const int prev = w->prev;
     ck_free(w->extra);
     w->extra = 0;
     if (w->kept) {
@@ -835,6 +848,7 @@ void ch_work_give(const CromaHipContext *cc, ChWork *w)
         if (w->stream) ck_stream_destroy(w->stream);
     }
     memset(w, 0, sizeof(*w));
+    ch_device_leave(prev);
 }
 
 /* Accessors for the serving loop (croma_serve.c). */

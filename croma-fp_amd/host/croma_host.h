@@ -48,15 +48,22 @@ void ch_set_error(const char *fmt, ...);
 void ch_params_to_ck(const CromaHipParams *in, CkParams *out);
 
 /* croma_stage.c: transfers of pageable arrays of any size (4 MiB and more
- * through the device's pinned ring), one reference per context */
+ * through the device's pinned ring), one reference per context.  The device
+ * current in the calling thread may be another one. */
 void ch_stage_ref(int dev);
 void ch_stage_unref(int dev);
 int ch_stage_h2d(int dev, void *dst, const void *src, size_t bytes, void *stream);
 int ch_stage_d2h(int dev, void *dst, const void *src, size_t bytes, void *stream);
 
+/* Makes dev the calling thread's device: the device to go back to with
+ * ch_device_leave, or -1 if dev cannot be made current. */
+int ch_device_enter(int dev);
+void ch_device_leave(int prev);
+
 /* Stream, timing events and device memory of one call on host arrays: the
  * context's own (memory up to CH_WORK_KEEP stays with it), or the call's own
- * while another thread has those. */
+ * while another thread has those.  From take to give the context's device is
+ * the thread's. */
 #define CH_WORK_KEEP ((size_t)512 << 20)
 typedef struct {
     void *stream, *e0, *e1;
@@ -64,7 +71,7 @@ typedef struct {
     size_t cap;
     int kept;     /* the context's */
     char *extra;  /* memory of this call alone */
-    int device;
+    int prev;     /* the thread's device before the call */
 } ChWork;
 char *ch_work_take(const CromaHipContext *c, size_t bytes, ChWork *w); /* device memory, or NULL */
 void ch_work_give(const CromaHipContext *c, ChWork *w);                /* after the stream drained */

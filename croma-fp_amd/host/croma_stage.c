@@ -16,7 +16,8 @@
  * One ring per device, made at the first large transfer and shared by the
  * device's contexts (8 MiB of pinned memory, a millisecond to allocate); it is
  * freed with the last of them.  Its lock is held for a whole transfer; a slot
- * is reused after the event behind its last transfer.
+ * is reused after the event behind its last transfer.  The ring is made and
+ * used with its device current, which the calling thread's need not be.
  */
 #include "croma_host.h"
 
@@ -122,14 +123,13 @@ static size_t piece_bytes(const StJob *j, size_t k)
 }
 
 /* Pieces t, t + nthr, ... of one transfer. */
-static void *stage_run(void *arg)
+static void stage_run(StJob *j)
 {
-    StJob *j = (StJob *)arg;
     const size_t n = (j->bytes + ST_PIECE - 1) / ST_PIECE;
     size_t k, back = (size_t)j->t;
     int s = 0, sb = 0, rc = 0;
     void *const st = j->r->st[j->t];
-    if ((j->t && ck_set_device(j->dev)) || ck_stream_wait_event(st, j->r->ev_go)) rc = -1;
+    if (ck_stream_wait_event(st, j->r->ev_go)) rc = -1;
     for (k = (size_t)j->t; k < n && !rc; k += (size_t)j->nthr, s ^= 1) {
         char *slot = j->r->pin + (size_t)(j->t * ST_SLOTS + s) * ST_PIECE;
         void *ev = j->r->ev[j->t][s];
@@ -159,6 +159,14 @@ static void *stage_run(void *arg)
         else memcpy(j->dst + back * ST_PIECE, j->r->pin + (size_t)(j->t * ST_SLOTS + sb) * ST_PIECE, piece_bytes(j, back));
     }
     j->rc = rc || ck_event_record(j->r->ev_done[j->t], st);
+}
+
+/* a new thread starts on device 0 */
+static void *stage_thread(void *arg)
+{
+    StJob *j = (StJob *)arg;
+    if (ck_set_device(j->dev)) j->rc = -1;
+    else stage_run(j);
     return 0;
 }
 
@@ -167,19 +175,24 @@ static int stage(int dev, int up, void *dst, const void *src, size_t bytes, void
     StJob jobs[ST_THREADS];
     pthread_t th[ST_THREADS];
     int started[ST_THREADS] = {0}, t, nthr = ch_host_threads(), rc = 0;
-    StRing *r = bytes >= ST_MIN ? ring_take(dev) : 0;
-    if (!r) return up ? ck_h2d(dst, src, bytes, stream) : ck_d2h(dst, src, bytes, stream);
+    const int prev = bytes >= ST_MIN ? ch_device_enter(dev) : -1;
+    StRing *r = prev >= 0 ? ring_take(dev) : 0;
+    if (!r) {
+        ch_device_leave(prev);
+        return up ? ck_h2d(dst, src, bytes, stream) : ck_d2h(dst, src, bytes, stream);
+    }
     if (nthr > ST_THREADS) nthr = ST_THREADS;
     if (nthr < 1) nthr = 1;
     if (ck_event_record(r->ev_go, stream)) {
         pthread_mutex_unlock(&r->lock);
+        ch_device_leave(prev);
         return -1;
     }
     for (t = 0; t < nthr; t++) {
         const StJob j = {r, dev, t, nthr, up, 0, (char *)dst, (const char *)src, bytes};
         jobs[t] = j;
     }
-    for (t = 1; t < nthr; t++) started[t] = pthread_create(&th[t], 0, stage_run, &jobs[t]) == 0;
+    for (t = 1; t < nthr; t++) started[t] = pthread_create(&th[t], 0, stage_thread, &jobs[t]) == 0;
     stage_run(&jobs[0]);
     for (t = 1; t < nthr; t++) {
         if (started[t]) pthread_join(th[t], 0);
@@ -187,6 +200,7 @@ static int stage(int dev, int up, void *dst, const void *src, size_t bytes, void
     }
     for (t = 0; t < nthr; t++) rc |= jobs[t].rc || ck_stream_wait_event(stream, r->ev_done[t]);
     pthread_mutex_unlock(&r->lock);
+    ch_device_leave(prev);
     return rc;
 }
 

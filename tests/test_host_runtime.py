@@ -5,6 +5,7 @@ import ctypes as C
 import glob
 import os
 import subprocess
+import threading
 
 import numpy as np
 import pytest
@@ -103,4 +104,68 @@ def test_drop_in_without_room_for_the_rows_runs_the_in_kernel_contraction(stub, 
         _snapshot(ctx, nt, np.full(nt, 16))
         assert [m & ~4 if fp32 else m for m, _, _ in _launches(stub)] == [2, 3]
     finally:
+        ctx.close()
+
+
+def _made(L, d):
+    out = (C.c_int * 3)()
+    L.stub_made(d, out)
+    return list(out)
+
+
+def _in_new_thread(L, fn):
+    """fn in a thread that has chosen no device; its device afterwards."""
+    out = {}
+
+    def run():
+        try:
+            out["value"] = fn()
+        except Exception as e:  # pragma: no cover
+            out["error"] = e
+        out["device"] = L.ck_get_device()
+
+    t = threading.Thread(target=run)
+    t.start()
+    t.join()
+    assert "error" not in out, out["error"]
+    assert out["device"] == 0
+    return out["value"]
+
+
+@pytest.mark.parametrize("first", ["own", "thread"])
+def test_calls_from_another_threads_device(stub, first):
+    """A context of device 3 used by a thread whose device is 0: transfers and
+    the emission calls make what they need on device 3 and leave the thread's
+    device as it was."""
+    stub.ck_set_device(3)
+    n, nt, nb = 64, 9000, 8  # 4.6 MB: through the pinned ring
+    ctx = ch.Context(n, ch.default_params())
+    b = ch.Batch(ctx, nt, ch.SPECIES_ELECTRON, 1)
+    x = np.random.default_rng(1).uniform(size=nt * n)
+    fic = np.ones(nb * n)
+    table = np.ones(200 * 16 * n)
+
+    def transfer():
+        b.set_state(None, x)
+        return np.array_equal(b.get_state()[1], x)
+
+    def emission():
+        ctx.emission_ic(x, fic, nb, ch.EMIS_FP64)
+        ctx.emission_kernel_table(ch.TABLE_IC, nb, 8.0, 20.0, 0.1)
+        p = ch.SynchPlan(ctx, table, 16, 200, -8.0, 100.0)
+        p.run(x, np.full(nt, 1e-6))
+        p.run(np.tile(x, 2), np.full(2 * nt, 1e-6))
+        p.close()
+        return True
+
+    try:
+        stub.stub_reset()
+        if first == "own":
+            assert transfer() and emission()
+        assert _in_new_thread(stub, transfer) and _in_new_thread(stub, emission)
+        assert transfer() and emission()
+        assert _made(stub, 0) == [0, 0, 0]
+        assert _made(stub, 3)[0] >= 4  # the ring's streams
+    finally:
+        b.close()
         ctx.close()
