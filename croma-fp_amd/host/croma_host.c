@@ -624,18 +624,17 @@ static int ic_ends_find(CromaHipContext *c, double z, double ends[2])
 void ch_ctx_ic_ends(CromaHipContext *c, int nz, const double *z, double *ends)
 {
     double zn[CH_IC_ENDS], v[2 * CH_IC_ENDS];
-    int q, k, first = 0;
+    int at[CH_IC_ENDS], q, k, first = 0;
     while (first < nz) {
         int m = 0, last;
         pthread_mutex_lock(&c->ic_lock);
         for (last = first; last < nz && m < CH_IC_ENDS; last++)
-            if (!ic_ends_find(c, z[last], ends + 2 * last)) zn[m++] = z[last];
+            if (!ic_ends_find(c, z[last], ends + 2 * last)) at[m] = last, zn[m++] = z[last];
         pthread_mutex_unlock(&c->ic_lock);
         if (m) ch_ic_cooling_ends(&c->g, m, zn, v);
         pthread_mutex_lock(&c->ic_lock);
         for (k = 0; k < m; k++) {
-            for (q = first; q < last; q++)
-                if (z[q] == zn[k]) memcpy(ends + 2 * q, v + 2 * k, 2 * sizeof(double));
+            memcpy(ends + 2 * at[k], v + 2 * k, 2 * sizeof(double));
             if (ic_ends_find(c, zn[k], 0)) continue;
             q = c->ic_end_next;
             c->ic_end_next = (q + 1) % CH_IC_ENDS;

@@ -169,3 +169,34 @@ def test_calls_from_another_threads_device(stub, first):
     finally:
         b.close()
         ctx.close()
+
+
+def test_ic_end_rates_of_many_redshifts(stub):
+    """The nsub estimate's IC rates at the first and last bin, batched and
+    cached: the row's own values bit for bit, in the order asked for, over more
+    redshifts than the cache holds, with repeats; also for a redshift that is
+    not a number (equal to none in the cache)."""
+    ctx = ch.Context(64, ch.default_params())
+    try:
+        stub.ch_ctx_ic_ends.argtypes = [C.c_void_p, C.c_int, C.POINTER(C.c_double), C.POINTER(C.c_double)]
+        stub.ch_ctx_ic_ends.restype = None
+        dp = C.POINTER(C.c_double)
+
+        def ends(z):
+            z = np.ascontiguousarray(z, np.float64)
+            out = np.full((len(z), 2), 12345.0)
+            stub.ch_ctx_ic_ends(C.c_void_p(ctx.h), len(z), z.ctypes.data_as(dp), out.ctypes.data_as(dp))
+            return out
+
+        few = np.array([0.0, 0.3, 0.1, 0.3, 6.0])
+        want = np.array([[ctx.ic_cooling_row(v)[0][i] for i in (0, -1)] for v in few])
+        assert np.array_equal(ends(few), want) and np.array_equal(ends(few), want)
+        many = np.linspace(0.0, 2.0, 700)
+        got = ends(many)
+        assert np.array_equal(got[::-1], ends(many[::-1])) and np.array_equal(ends(few), want)
+        assert np.array_equal(got[350], [ctx.ic_cooling_row(many[350])[0][i] for i in (0, -1)])
+        got, row = ends([0.1, np.nan, 0.3]), ctx.ic_cooling_row(np.nan)[0]
+        assert np.array_equal(got[[0, 2]], want[[2, 1]])
+        assert np.array_equal(got[1], row[[0, -1]], equal_nan=True)
+    finally:
+        ctx.close()
