@@ -52,6 +52,7 @@ typedef struct {
     int *d_nsub, *d_non;
     void *ev_ready, *ev_done;
     int snap_next, inflight, ready;
+    int picked; /* part of the launch being put together */
     double elapsed;
     double t_submit, t_admit, t_done;
     long long cell_steps;
@@ -457,7 +458,11 @@ static int sv_launch_class(CromaHipServer *s, int ci)
     if (!c) return 0;
     for (i = 0; i < s->nactive; i++) {
         SvReq *r = s->active[i];
-        if (r->cls != ci || r->state != SV_ACTIVE || r->snap_next >= r->nsnap || sv_cancelled(r)) continue;
+        if (r->cls != ci) continue;
+        /* decided once: a request that is cancelled from here on is launched
+         * and dropped when the launch is done, like one cancelled later */
+        r->picked = 0;
+        if (r->state != SV_ACTIVE || r->snap_next >= r->nsnap || sv_cancelled(r)) continue;
         if (!r->ready) {
             const int e = ck_event_query(r->ev_ready);
             if (e == 0) continue;
@@ -465,6 +470,7 @@ static int sv_launch_class(CromaHipServer *s, int ci)
             r->ready = 1;
             sv_count_steps(r);
         }
+        r->picked = 1;
         ntasks += r->ntr;
         nl++;
     }
@@ -472,7 +478,7 @@ static int sv_launch_class(CromaHipServer *s, int ci)
     tile = ch_ctx_tile(c, protons, ntasks);
     for (i = 0; i < s->nactive; i++) {
         SvReq *r = s->active[i];
-        if (r->cls != ci || r->state != SV_ACTIVE || r->snap_next >= r->nsnap || sv_cancelled(r) || !r->ready) continue;
+        if (r->cls != ci || !r->picked) continue;
         r->inflight = r->nsnap - r->snap_next < tile.chain ? r->nsnap - r->snap_next : tile.chain;
         nslots += r->inflight;
     }
@@ -483,8 +489,7 @@ static int sv_launch_class(CromaHipServer *s, int ci)
         long need_off = 0, need_rows = 0;
         for (i = 0; i < s->nactive; i++) {
             SvReq *r = s->active[i];
-            if (r->cls != ci || r->state != SV_ACTIVE || r->snap_next >= r->nsnap || sv_cancelled(r) || !r->ready)
-                continue;
+            if (r->cls != ci || !r->picked) continue;
             need_off += (long)r->inflight * r->ntr;
             for (q = 0; q < r->inflight; q++) {
                 const int *ns = r->h_sched + (size_t)(r->snap_next + q) * r->ntr;
@@ -526,8 +531,7 @@ static int sv_launch_class(CromaHipServer *s, int ci)
     for (i = 0; i < s->nactive; i++) {
         SvReq *r = s->active[i];
         int first, t;
-        if (r->cls != ci || r->state != SV_ACTIVE || r->snap_next >= r->nsnap || sv_cancelled(r) || !r->ready)
-            continue;
+        if (r->cls != ci || !r->picked) continue;
         first = nslots;
         for (q = 0; q < r->inflight; q++) {
             const int sn = r->snap_next + q;

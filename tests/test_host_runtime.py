@@ -6,6 +6,7 @@ import glob
 import os
 import subprocess
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -33,6 +34,7 @@ def stub(stub_path, monkeypatch):
     L = ch.lib()
     L.stub_peak.restype = L.stub_live.restype = C.c_size_t
     L.stub_set_limit.argtypes = [C.c_size_t, C.c_size_t]
+    L.stub_set_host_alloc_hook.argtypes = [C.c_void_p]
     L.ck_set_device(0)
     L.stub_reset()
     yield L
@@ -200,3 +202,34 @@ def test_ic_end_rates_of_many_redshifts(stub):
         assert np.array_equal(got[1], row[[0, -1]], equal_nan=True)
     finally:
         ctx.close()
+
+
+def test_cancel_while_a_launch_is_put_together(stub):
+    """A request cancelled after the scheduler has counted it for a launch (the
+    growing task list's allocation is such a moment) still comes to an end."""
+    def chunk(nt, nsnap):
+        return srv.submit(64, ch.SPECIES_ELECTRON, 1, 0.01 * np.arange(nsnap + 1)[::-1], np.full(nsnap, 0.01),
+                          np.ones((nsnap + 1, 8, nt)), cre=np.ones(nt * 64))
+
+    srv = ch.Server(64 << 20)
+    me, ids, hits = threading.get_ident(), [], []
+
+    @C.CFUNCTYPE(None)
+    def hook():  # the submitting thread allocates too
+        if threading.get_ident() != me and not hits:
+            hits.append(1)
+            srv.cancel(ids[0])
+
+    try:
+        srv.wait(chunk(4, 1))  # the class's first, small task list
+        ids.append(2)          # the next request's number
+        stub.stub_set_host_alloc_hook(C.cast(hook, C.c_void_p))
+        assert chunk(500, 50) == ids[0]
+        end = time.time() + 5.0
+        while srv.poll(ids[0]) == 0 and time.time() < end:
+            time.sleep(0.01)
+        assert hits and srv.poll(ids[0]) == ch.ECANCELED
+        assert srv.stats()["in_use_bytes"] == 0
+    finally:
+        stub.stub_set_host_alloc_hook(None)
+        srv.close()
