@@ -82,6 +82,7 @@ typedef struct {
 
 struct CromaHipServer {
     CromaHipParams uprm;
+    int device; /* the creating thread's: the pool's and the streams' */
     double pmin, pmax, pemin, pemax;
     CromaHipContext *ctx[4];
     SvClass cls[SV_NCLASS];
@@ -673,6 +674,9 @@ static int sv_complete_class(CromaHipServer *s, int ci)
 static void *sv_main(void *arg)
 {
     CromaHipServer *s = (CromaHipServer *)arg;
+    /* a new thread starts on device 0; where this fails, so do its launches,
+     * and with them the requests */
+    if (s->device >= 0) ck_set_device(s->device);
     for (;;) {
         int i, any = 0, ci;
         pthread_mutex_lock(&s->mu);
@@ -779,6 +783,7 @@ CromaHipServer *croma_hip_serve_create(const CromaHipParams *prm, size_t budget,
     s = (CromaHipServer *)calloc(1, sizeof(*s));
     if (!s) return 0;
     s->uprm = *prm;
+    s->device = ck_get_device();
     s->pmin = pmin;
     s->pmax = pmax;
     s->pemin = pemin;

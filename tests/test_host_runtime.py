@@ -233,3 +233,16 @@ def test_cancel_while_a_launch_is_put_together(stub):
     finally:
         stub.stub_set_host_alloc_hook(None)
         srv.close()
+
+
+def test_server_works_on_the_device_it_was_made_on(stub):
+    stub.ck_set_device(5)
+    srv = ch.Server(64 << 20)
+    try:
+        stub.stub_reset()
+        rid = srv.submit(64, ch.SPECIES_ELECTRON, 1, np.array([0.01, 0.0]), np.array([0.01]), np.ones((2, 8, 30)),
+                         cre=np.ones(30 * 64))
+        assert np.all(srv.wait(rid)[1] == 1.0)
+        assert _made(stub, 0) == [0, 0, 0] and _made(stub, 5)[2] > 0
+    finally:
+        srv.close()
