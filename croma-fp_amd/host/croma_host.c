@@ -158,6 +158,8 @@ struct CromaHipContext {
     int *d_err;
     CromaHipTile tile[2]; /* [protons]; used once set (set_tile, autotuners), else by size (run_tile) */
     int tile_set[2];
+    CromaHipTile ran[2]; /* of the latest fused run, if ran_ok */
+    int ran_ok[2];
     pthread_mutex_t ic_lock;
     struct {
         int valid;
@@ -506,10 +508,22 @@ int croma_hip_context_set_tile(CromaHipContext *c, int protons, const CromaHipTi
     return 0;
 }
 
+/* What a fused run took: its tile, the snapshots of its windows, and whether
+ * its secondaries went through the split launch. */
+static void note_run(CromaHipContext *c, int protons, const CromaHipTile *t, int window, int split)
+{
+    const int p = protons ? 1 : 0;
+    c->ran[p] = *t;
+    c->ran[p].chain = window;
+    c->ran[p].secondary_gemm = split;
+    c->ran_ok[p] = 1;
+}
+
 int croma_hip_context_get_tile(const CromaHipContext *c, int protons, CromaHipTile *t)
 {
     if (!c || !t) return CROMA_HIP_EINVAL;
-    *t = c->tile[protons ? 1 : 0];
+    protons = protons ? 1 : 0;
+    *t = !c->tile_set[protons] && c->ran_ok[protons] ? c->ran[protons] : c->tile[protons];
     return 0;
 }
 
@@ -1888,6 +1902,7 @@ int croma_hip_batch_run(CromaHipBatch *b, int s0, int s1, int nsnap_total, const
         const long segmax = c->prm.coeff_interp_max_segments > 1 ? c->prm.coeff_interp_max_segments : 1;
         if (reserve_segrows(b, (long)wsz * b->ntr * segmax)) return dev_fail("segment rows");
     }
+    if (path == CROMA_HIP_PATH_FUSED) note_run(c, b->protons, &b->tile, wsz, split);
     nwin = (s1 - s0 + wsz - 1) / wsz;
     for (k = 0; k < 2; k++)
         if ((rc = win_reserve(c, &b->win[k], wsz, b->ntr, !dev_nsub)) != 0) return rc;
@@ -2211,6 +2226,7 @@ int croma_hip_execute_snapshot(
         } else if (protons) {
             b->tile = run_tile(c, 1, ntr, 1, 1);
         }
+        note_run(c, protons, &b->tile, 1, split);
         if ((split && (ck_h2d(w->d_segoff, w->h_segoff, (size_t)ntr * sizeof(int), c->stream) ||
                        ck_h2d(d_npm, npm, ((size_t)n + 1) * sizeof(int), c->stream))) ||
             ck_h2d(d_nsub, w->h_nsub, (size_t)ntr * sizeof(int), c->stream) ||

@@ -125,7 +125,10 @@ void croma_hip_context_destroy(CromaHipContext *ctx);
 int croma_hip_context_set_params(CromaHipContext *ctx, const CromaHipParams *prm);
 /* protons: 0 electron_only tile, 1 electron_proton tile, -1 both.  Until a tile
  * is set here or by an autotuner, every run takes one by its grid, species,
- * tracers and snapshots; get_tile then returns the grid's default. */
+ * tracers and snapshots; get_tile then returns what the context's latest run or
+ * snapshot call of the species took (chain: the snapshots of its windows,
+ * secondary_gemm: whether it took the split launch), and before the first one
+ * the grid's default. */
 int croma_hip_context_set_tile(CromaHipContext *ctx, int protons, const CromaHipTile *tile);
 int croma_hip_context_get_tile(const CromaHipContext *ctx, int protons, CromaHipTile *tile);
 /* 1 (default): a snapshot window whose launch shape repeats the previous

@@ -65,7 +65,7 @@ def test_windows_and_tiles_by_size(case):
         assert not m.any() or np.max(np.abs(a[m] - f[m]) / np.abs(f[m])) < 1e-11
 
 
-@pytest.mark.parametrize("n", [64, 128, 256])
+@pytest.mark.parametrize("n", [64, 128, 256, 512])
 def test_snapshot_split_equals_in_kernel_contraction(n):
     w = small_workload(n, 75, 1, 3, 1, seed=5)
     out = []
@@ -86,6 +86,7 @@ def test_snapshot_split_equals_in_kernel_contraction(n):
             for _ in range(4):  # eager, captured, replayed
                 ctx.execute_snapshot(ns, non, True, 0.0, float(w.dt_snap[0]), w.bg[0], row, m1, p1, w.bg[1], row, m1,
                                      p1, zero, zero, fqe.ravel(), npmin, w.mass, None, crp, cre)
+            assert ctx.get_tile(True)[3] == (0 if below else 1)  # the launch it took
             out.append((crp, cre))
         finally:
             ctx.close()

@@ -246,3 +246,38 @@ def test_server_works_on_the_device_it_was_made_on(stub):
         assert _made(stub, 0) == [0, 0, 0] and _made(stub, 5)[2] > 0
     finally:
         srv.close()
+
+
+def test_get_tile_tells_what_a_run_took(stub):
+    def run(ctx, species, nt, ns):
+        b = ch.Batch(ctx, nt, species, ns)
+        for s in range(ns):
+            b.set_background(s, np.ones((8, nt)))
+        b.set_state(None, np.ones(nt * ctx.n))
+        stub.stub_reset()
+        b.run(0, ns, ns, np.linspace(0.1, 0.0, ns + 1), np.full(ns, 0.01))
+        b.close()
+        return ctx.get_tile(species != ch.SPECIES_ELECTRON), _launches(stub)
+
+    ctx = ch.Context(128, ch.default_params())
+    try:
+        e, p = ctx.get_tile(False), ctx.get_tile(True)
+        tile, log = run(ctx, ch.SPECIES_ELECTRON, 100, 5)
+        assert tile[2:] == (5, 0) and [(r, t) for _, r, t in log] == [(tile[0], 100)]  # one window
+        assert ctx.get_tile(True) == p
+        tile, log = run(ctx, ch.SPECIES_ELECTRON, 70000, 2)
+        assert tile[2] == 1 and len(log) == 2 and log[0][1] == tile[0] != 4
+        tile, log = run(ctx, ch.SPECIES_ELECTRON_PROTON, 100, 3)
+        assert tile[2:] == (1, 1) and [m for m, _, _ in log] == [2, 3] * 3
+        _snapshot(ctx, 50, np.full(50, 8))
+        assert ctx.get_tile(True)[3] == 1
+        ctx.set_tile(8, 2, 1, protons=0, secondary_gemm=0)
+        assert ctx.get_tile(False) == (8, 2, 1, 0) and e[3] == 0
+    finally:
+        ctx.close()
+    ctx = ch.Context(128, ch.default_params(dpp_model=1, eta_dpp_cap=0.1))
+    try:
+        tile, log = run(ctx, ch.SPECIES_ELECTRON_PROTON, 100, 3)
+        assert tile[2:] == (3, 0) and [m for m, _, _ in log] == [1]
+    finally:
+        ctx.close()
