@@ -144,6 +144,10 @@ typedef struct {
     int state; /* 0 empty, 1 key seen once, 2 captured, -1 capture refused */
 } ChGraph;
 
+/* A species' tile: by size; as set; rows, waves and contraction as an
+ * autotuner left them, window lengths by size. */
+enum { TILE_BY_SIZE = 0, TILE_SET, TILE_TUNED };
+
 struct CromaHipContext {
     int device;
     int cu_count;
@@ -157,7 +161,7 @@ struct CromaHipContext {
     int *d_counter;
     int *d_err;
     CromaHipTile tile[2]; /* [protons]; used once set (set_tile, autotuners), else by size (run_tile) */
-    int tile_set[2];
+    int tile_set[2]; /* TILE_* */
     CromaHipTile ran[2]; /* of the latest fused run, if ran_ok */
     int ran_ok[2];
     pthread_mutex_t ic_lock;
@@ -295,20 +299,22 @@ static int ctx_upload_grid(CromaHipContext *c)
     return 0;
 }
 
-static void default_tiles(CromaHipContext *c)
+static CromaHipTile default_tile(int n, int protons)
 {
-    const int n = c->g.n;
     /* rows per lane: the spectrum and one factor set stay in registers;
      * two waves per SIMD hide the cross-lane latency of the substep scans */
     /* measured defaults (the autotuner refines them per workload) */
-    c->tile[0].rows_per_lane = (n == 64) ? 4 : (n == 128) ? 8 : (n == 256) ? 8 : 16;
-    c->tile[0].waves_per_simd = (n <= 128) ? 1 : 2;
-    c->tile[0].chain = 1;
-    c->tile[0].secondary_gemm = 0;
-    c->tile[1].rows_per_lane = (n <= 256) ? 4 : 8;
-    c->tile[1].waves_per_simd = (n == 64) ? 1 : 2;
-    c->tile[1].chain = 1;
-    c->tile[1].secondary_gemm = 1;
+    CromaHipTile t;
+    t.chain = 1;
+    t.secondary_gemm = protons;
+    if (protons) {
+        t.rows_per_lane = (n <= 256) ? 4 : 8;
+        t.waves_per_simd = (n == 64) ? 1 : 2;
+    } else {
+        t.rows_per_lane = (n == 64) ? 4 : (n <= 256) ? 8 : 16;
+        t.waves_per_simd = (n <= 128) ? 1 : 2;
+    }
+    return t;
 }
 
 /* Whether every fused launch mode a tile runs has an FP32-coefficient
@@ -348,9 +354,11 @@ static CromaHipTile run_tile(const CromaHipContext *c, int protons, long ntr, in
     const int split = p && !in_kernel && c->tile[1].secondary_gemm &&
                       !(c->prm.dpp_model != 3 && c->prm.eta_dpp_cap > 0.0);
     CromaHipTile t = c->tile[p];
-    if (c->tile_set[p]) return t;
+    if (c->tile_set[p] == TILE_SET) return t;
     if (in_kernel) t.secondary_gemm = 0;
-    if (!p) {
+    if (c->tile_set[p] == TILE_TUNED) {
+        /* as found */
+    } else if (!p) {
         if (n == 64) t.rows_per_lane = rows <= CH_ROWS_LATENCY ? 4 : 8;
         else if (n <= 256) t.rows_per_lane = (n == 128 && rows <= CH_ROWS_LATENCY) ? 4 : rows <= CH_ROWS_MIDDLE ? 8 : 16;
         t.waves_per_simd = (n <= 128 && rows <= CH_ROWS_LATENCY) ? 1 : 2;
@@ -363,7 +371,7 @@ static CromaHipTile run_tile(const CromaHipContext *c, int protons, long ntr, in
     }
     if (c->coeff_fp32 && !tile_f32_ok(c, p, t.rows_per_lane, t.waves_per_simd, t.secondary_gemm)) t = c->tile[p];
     /* a window's schedule buffers are bounded by 16 snapshots of 65,536 tracers */
-    if (!split && ntr <= 65536) t.chain = run < 16 ? run : 16;
+    if (!split && ntr <= 65536 && t.chain < (run < 16 ? run : 16)) t.chain = run < 16 ? run : 16;
     return t;
 }
 
@@ -423,7 +431,8 @@ CromaHipContext *croma_hip_context_create(const CromaHipGridSpec *gs, const Crom
         croma_hip_context_destroy(c);
         return 0;
     }
-    default_tiles(c);
+    c->tile[0] = default_tile(c->g.n, 0);
+    c->tile[1] = default_tile(c->g.n, 1);
     c->use_graphs = 1;
     c->pipeline = -1;
     c->nsub_device = 1;
@@ -503,8 +512,8 @@ int croma_hip_context_set_tile(CromaHipContext *c, int protons, const CromaHipTi
 {
     if (!c || !t || protons < -1 || protons > 1) return CROMA_HIP_EINVAL;
     if (!tile_ok(c->g.n, t)) return CROMA_HIP_EUNSUPPORTED;
-    if (protons != 1) c->tile[0] = *t, c->tile_set[0] = 1;
-    if (protons != 0) c->tile[1] = *t, c->tile_set[1] = 1;
+    if (protons != 1) c->tile[0] = *t, c->tile_set[0] = TILE_SET;
+    if (protons != 0) c->tile[1] = *t, c->tile_set[1] = TILE_SET;
     return 0;
 }
 
@@ -523,7 +532,7 @@ int croma_hip_context_get_tile(const CromaHipContext *c, int protons, CromaHipTi
 {
     if (!c || !t) return CROMA_HIP_EINVAL;
     protons = protons ? 1 : 0;
-    *t = !c->tile_set[protons] && c->ran_ok[protons] ? c->ran[protons] : c->tile[protons];
+    *t = c->tile_set[protons] != TILE_SET && c->ran_ok[protons] ? c->ran[protons] : c->tile[protons];
     return 0;
 }
 
@@ -2373,6 +2382,55 @@ static int tile_better(double ms, const CromaHipTile *t, double best_ms, const C
     return ms < best_ms * 0.98 || (ms < best_ms * 1.02 && t->rows_per_lane > bt->rows_per_lane);
 }
 
+/* State of the batch back from its copy. */
+static int tune_restore(CromaHipBatch *b, const double *d_save)
+{
+    CromaHipContext *c = b->ctx;
+    const size_t m = (size_t)b->ntr * c->g.n;
+    if (ck_d2d(b->d_cre, d_save, m * sizeof(double), c->stream) ||
+        (b->protons && ck_d2d(b->d_crp, d_save + m, m * sizeof(double), c->stream)))
+        return dev_fail("autotune state restore");
+    return 0;
+}
+
+/* Replaces *bt by the tile chosen by size if runs of up to four snapshots from
+ * s are more than 1% faster with it. */
+static int tune_against_size(CromaHipBatch *b, int s, int nsnap_total, const double *z, const double *dt_snap,
+                             double elapsed, const double *d_save, CromaHipTile *bt)
+{
+    CromaHipContext *c = b->ctx;
+    const int p = b->protons ? 1 : 0;
+    CromaHipTile t[2];
+    double ms[2] = {0.0, 0.0};
+    int run = 4, k, rep, rc;
+    /* a snapshot needs its successor resident unless it is the last */
+    while (run > 1 && !(s + run <= b->nsnap_res && (s + run == nsnap_total || s + run < b->nsnap_res))) run--;
+    t[0] = *bt;
+    c->tile[p] = default_tile(c->g.n, p);
+    c->tile_set[p] = TILE_BY_SIZE;
+    t[1] = run_tile(c, p, b->ntr, run, 0);
+    t[1].chain = 1;
+    c->tile_set[p] = TILE_TUNED;
+    if (run < 2 || (t[0].rows_per_lane == t[1].rows_per_lane && t[0].waves_per_simd == t[1].waves_per_simd &&
+                    (!p || t[0].secondary_gemm == t[1].secondary_gemm)))
+        return 0;
+    for (k = 0; k < 2; k++) {
+        c->tile[p] = t[k];
+        for (rep = 0; rep < 2; rep++) {
+            CromaHipTimes tm;
+            memset(&tm, 0, sizeof(tm));
+            if ((rc = tune_restore(b, d_save)) != 0 ||
+                (rc = croma_hip_batch_run(b, s, s + run, nsnap_total, z, dt_snap, elapsed, CROMA_HIP_PATH_FUSED,
+                                          &tm)) != 0)
+                return rc;
+            ms[k] = tm.kernel_ms;
+            if (ms[k] > 100.0) break;
+        }
+    }
+    if (ms[1] < 0.99 * ms[0]) *bt = t[1];
+    return 0;
+}
+
 int croma_hip_batch_autotune(CromaHipBatch *b, int s, int nsnap_total, const double *z, const double *dt_snap,
                              double elapsed, CromaHipTile *best)
 {
@@ -2387,7 +2445,7 @@ int croma_hip_batch_autotune(CromaHipBatch *b, int s, int nsnap_total, const dou
     m = (size_t)b->ntr * c->g.n;
     keep = c->tile[b->protons ? 1 : 0];
     keep_set = c->tile_set[b->protons ? 1 : 0];
-    c->tile_set[b->protons ? 1 : 0] = 1;
+    c->tile_set[b->protons ? 1 : 0] = TILE_SET;
     bt = keep;
     /* every trial starts from the batch's current state */
     d_save = (double *)ck_malloc(m * sizeof(double) * (b->protons ? 2 : 1));
@@ -2409,11 +2467,7 @@ int croma_hip_batch_autotune(CromaHipBatch *b, int s, int nsnap_total, const dou
         for (rep = 0; rep < 2; rep++) {
             CromaHipTimes tm;
             memset(&tm, 0, sizeof(tm));
-            if (ck_d2d(b->d_cre, d_save, m * sizeof(double), c->stream) ||
-                (b->protons && ck_d2d(b->d_crp, d_save + m, m * sizeof(double), c->stream))) {
-                rc = dev_fail("autotune state restore");
-                goto out;
-            }
+            if ((rc = tune_restore(b, d_save)) != 0) goto out;
             if ((rc = croma_hip_batch_run(b, s, s + 1, nsnap_total, z, dt_snap, elapsed, CROMA_HIP_PATH_FUSED, &tm)) !=
                 0)
                 goto out;
@@ -2437,11 +2491,7 @@ int croma_hip_batch_autotune(CromaHipBatch *b, int s, int nsnap_total, const dou
             for (rep = 0; rep < 2; rep++) {
                 CromaHipTimes tm;
                 memset(&tm, 0, sizeof(tm));
-                if (ck_d2d(b->d_cre, d_save, m * sizeof(double), c->stream) ||
-                    (b->protons && ck_d2d(b->d_crp, d_save + m, m * sizeof(double), c->stream))) {
-                    rc = dev_fail("autotune state restore");
-                    goto out;
-                }
+                if ((rc = tune_restore(b, d_save)) != 0) goto out;
                 if ((rc = croma_hip_batch_run(b, s, s + 2, nsnap_total, z, dt_snap, elapsed, CROMA_HIP_PATH_FUSED,
                                               &tm)) != 0)
                     goto out;
@@ -2451,6 +2501,10 @@ int croma_hip_batch_autotune(CromaHipBatch *b, int s, int nsnap_total, const dou
         }
         bt.chain = (cms[1] < 0.99 * cms[0]) ? 2 : 1;
     }
+    /* the trials ran one snapshot each; runs take longer windows or pipelined
+     * passes by size.  The winner against the tile that the size alone would
+     * choose, in that form over the snapshots at hand */
+    if ((rc = tune_against_size(b, s, nsnap_total, z, dt_snap, elapsed, d_save, &bt)) != 0) goto out;
 out:
     if (d_save) {
         if (ck_d2d(b->d_cre, d_save, m * sizeof(double), c->stream) ||
@@ -2459,7 +2513,8 @@ out:
         ck_free(d_save);
     }
     c->tile[b->protons ? 1 : 0] = rc ? keep : bt;
-    if (rc) c->tile_set[b->protons ? 1 : 0] = keep_set;
+    c->tile_set[b->protons ? 1 : 0] = rc ? keep_set : TILE_TUNED;
+    c->ran_ok[b->protons ? 1 : 0] = 0;
     if (!rc) *best = bt;
     return rc;
 }
@@ -2477,7 +2532,7 @@ int croma_hip_autotune(CromaHipContext *c, int protons, int ntracer, CromaHipTil
     if (!c || ntracer <= 0 || !best) return CROMA_HIP_EINVAL;
     keep = c->tile[protons ? 1 : 0];
     keep_set = c->tile_set[protons ? 1 : 0];
-    c->tile_set[protons ? 1 : 0] = 1;
+    c->tile_set[protons ? 1 : 0] = TILE_TUNED;
     bt = keep;
     bg = (double *)malloc((size_t)(nsnap + 1) * CK_NBG * ntracer * sizeof(double));
     cre = (double *)malloc((size_t)ntracer * n * sizeof(double));
@@ -2546,6 +2601,7 @@ out:
     free(crp);
     c->tile[protons ? 1 : 0] = rc ? keep : bt;
     if (rc) c->tile_set[protons ? 1 : 0] = keep_set;
+    c->ran_ok[protons ? 1 : 0] = 0;
     if (!rc) *best = bt;
     return rc;
 }

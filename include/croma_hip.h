@@ -125,10 +125,12 @@ void croma_hip_context_destroy(CromaHipContext *ctx);
 int croma_hip_context_set_params(CromaHipContext *ctx, const CromaHipParams *prm);
 /* protons: 0 electron_only tile, 1 electron_proton tile, -1 both.  Until a tile
  * is set here or by an autotuner, every run takes one by its grid, species,
- * tracers and snapshots; get_tile then returns what the context's latest run or
- * snapshot call of the species took (chain: the snapshots of its windows,
- * secondary_gemm: whether it took the split launch), and before the first one
- * the grid's default. */
+ * tracers and snapshots; an autotuner leaves the window lengths (chain) of runs
+ * of up to 65,536 tracers to that rule.  Until a tile is set here, get_tile
+ * returns what the context's latest run or snapshot call of the species took
+ * (chain: the snapshots of its windows, secondary_gemm: whether it took the
+ * split launch), before the first one the autotuner's tile or the grid's
+ * default. */
 int croma_hip_context_set_tile(CromaHipContext *ctx, int protons, const CromaHipTile *tile);
 int croma_hip_context_get_tile(const CromaHipContext *ctx, int protons, CromaHipTile *tile);
 /* 1 (default): a snapshot window whose launch shape repeats the previous
@@ -267,7 +269,9 @@ int croma_hip_batch_sync(CromaHipBatch *b);
  * after each trial and at the end.  Then, where snapshot s + 1 is resident
  * with its successor, the winner advances snapshots s and s + 1 with one
  * and with two snapshots per queue task, and keeps two if that is more than
- * 1% faster.  Stores the fastest tile in the context and returns it.  No
+ * 1% faster.  Where the tile that the size alone would choose is another one,
+ * both then advance up to four of the resident snapshots as runs do (windows
+ * and pipelined passes by size), and it wins if more than 1% faster.  Stores the fastest tile in the context and returns it.  No
  * reference counterpart (the reference has no tiles). */
 int croma_hip_batch_autotune(CromaHipBatch *b, int isnap, int nsnap_total, const double *z,
                              const double *dt_snap, double elapsed_gyr, CromaHipTile *best);

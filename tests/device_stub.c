@@ -16,6 +16,7 @@
 
 typedef struct {
     int dev;
+    double at; /* events: the clock when recorded */
 } Obj;
 
 typedef struct {
@@ -30,6 +31,9 @@ static size_t live, peak, limit = (size_t)1 << 40, free_mem = (size_t)1 << 38;
 static int log_mode[STUB_LOG], log_rows[STUB_LOG], log_tasks[STUB_LOG], nlog;
 static int dev_streams[8], dev_events[8], dev_allocs[8];
 static void (*hook_host_alloc)(void);
+/* the clock advances with each fused launch of tasks over k snapshots at r
+ * rows per lane by launch_ms[r] + k slot_ms[r] */
+static double now_ms, launch_ms[17], slot_ms[17];
 
 void stub_reset(void)
 {
@@ -38,6 +42,7 @@ void stub_reset(void)
     free_mem = (size_t)1 << 38;
     nlog = 0;
     hook_host_alloc = 0;
+    for (int r = 0; r <= 16; r++) launch_ms[r] = 1.0, slot_ms[r] = 0.0;
     memset(dev_streams, 0, sizeof(dev_streams));
     memset(dev_events, 0, sizeof(dev_events));
     memset(dev_allocs, 0, sizeof(dev_allocs));
@@ -46,6 +51,11 @@ void stub_set_limit(size_t largest, size_t free_bytes)
 {
     limit = largest;
     free_mem = free_bytes;
+}
+void stub_set_cost(int r, double launch, double slot)
+{
+    launch_ms[r] = launch;
+    slot_ms[r] = slot;
 }
 void stub_set_host_alloc_hook(void (*f)(void)) { hook_host_alloc = f; }
 size_t stub_peak(void) { return peak; }
@@ -147,11 +157,12 @@ int ck_event_destroy(void *e)
 }
 int ck_event_record(void *e, void *s)
 {
+    ((Obj *)e)->at = now_ms;
     return !s || ((Obj *)e)->dev == ((Obj *)s)->dev ? 0 : fail("event of another device");
 }
 int ck_event_query(void *e) { return e ? 1 : -1; }
 int ck_event_sync(void *e) { return e ? 0 : -1; }
-float ck_event_elapsed_ms(void *a, void *b) { return a && b ? 1.0f : -1.0f; }
+float ck_event_elapsed_ms(void *a, void *b) { return a && b ? (float)(((Obj *)b)->at - ((Obj *)a)->at) : -1.0f; }
 int ck_stream_wait_event(void *s, void *e) { return s && e ? 0 : -1; }
 int ck_h2d(void *dst, const void *src, size_t bytes, void *s)
 {
@@ -201,6 +212,7 @@ int ck_launch_fused(int n, int r, int occ, int nblocks, int mode, CkGrid g, cons
     (void)n, (void)occ, (void)nblocks, (void)g, (void)slots, (void)tasks, (void)counter, (void)e;
     if (on_current(s)) return -1;
     pthread_mutex_lock(&mu);
+    now_ms += launch_ms[r] + (ntasks > 0 ? tasks[0].nslot : 0) * slot_ms[r];
     if (nlog < STUB_LOG) log_mode[nlog] = mode, log_rows[nlog] = r, log_tasks[nlog] = ntasks, nlog++;
     pthread_mutex_unlock(&mu);
     return 0;
@@ -217,6 +229,17 @@ int ck_nsub_arrays(CkGrid g, CkParams prm, int ntr, double dt, double lo, double
     return 0;
 }
 
+/* the tasks in the tracers' order */
+int ck_nsub_order(CkGrid g, const CkSlot *slots, int count, int ntr, int protons, int split, CkTask *tasks, int *key,
+                  int *segloc, int *blk, int *hist, unsigned long long *cells, void *s)
+{
+    int i;
+    (void)g, (void)slots, (void)protons, (void)split, (void)key, (void)segloc, (void)blk, (void)hist, (void)cells;
+    if (on_current(s)) return -1;
+    for (i = 0; i < ntr; i++) tasks[i].slot = 0, tasks[i].tracer = i, tasks[i].nslot = count;
+    return 0;
+}
+
 /* the remaining launches do nothing but look at their stream, the last argument */
 int ck_sec_contract(int n, const double *a, const int *b, const double *c, double *d, long e, const int *f, int g,
                     void *s)
@@ -227,12 +250,6 @@ int ck_sec_contract(int n, const double *a, const int *b, const double *c, doubl
 int ck_ic_rows(int n, const double *a, double b, double c, int d, const double *e, double *f, double *g, int *h, void *s)
 {
     (void)n, (void)a, (void)b, (void)c, (void)d, (void)e, (void)f, (void)g, (void)h;
-    return on_current(s);
-}
-int ck_nsub_order(CkGrid g, const CkSlot *a, int b, int c, int d, int e, CkTask *f, int *h, int *i, int *j, int *k,
-                  unsigned long long *l, void *s)
-{
-    (void)g, (void)a, (void)b, (void)c, (void)d, (void)e, (void)f, (void)h, (void)i, (void)j, (void)k, (void)l;
     return on_current(s);
 }
 int ck_grid_loss_tables(CkGrid g, double epmax, void *s)

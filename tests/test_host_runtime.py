@@ -34,6 +34,7 @@ def stub(stub_path, monkeypatch):
     L = ch.lib()
     L.stub_peak.restype = L.stub_live.restype = C.c_size_t
     L.stub_set_limit.argtypes = [C.c_size_t, C.c_size_t]
+    L.stub_set_cost.argtypes = [C.c_int, C.c_double, C.c_double]
     L.stub_set_host_alloc_hook.argtypes = [C.c_void_p]
     L.ck_set_device(0)
     L.stub_reset()
@@ -279,5 +280,50 @@ def test_get_tile_tells_what_a_run_took(stub):
     try:
         tile, log = run(ctx, ch.SPECIES_ELECTRON_PROTON, 100, 3)
         assert tile[2:] == (3, 0) and [m for m, _, _ in log] == [1]
+    finally:
+        ctx.close()
+
+
+def test_tuned_runs_keep_the_windows_by_size(stub):
+    """An autotuner times rows, waves and the contraction; the snapshots of a
+    window stay a matter of size, and a tile that wins one snapshot at a time
+    does not displace the rule's where runs are slower with it."""
+    n, nt, ns = 128, 100, 6
+    z, dt = np.linspace(0.1, 0.0, ns + 1), np.full(ns, 0.01)
+    for costs, rows in (({4: (1.5, 0.1), 8: (2.0, 0.1), 16: (0.0, 1.0)}, 4),   # 16 rows win one snapshot alone
+                        ({4: (2.0, 0.5), 8: (2.0, 0.1), 16: (0.5, 0.3)}, 16)):  # and here runs too
+        ctx = ch.Context(n, ch.default_params())
+        ctx.set_graphs(False)  # every launch on the record
+        b = ch.Batch(ctx, nt, ch.SPECIES_ELECTRON, ns)
+        try:
+            for s in range(ns):
+                b.set_background(s, np.ones((8, nt)))
+            b.set_state(None, np.ones(nt * n))
+            for r, c in costs.items():
+                stub.stub_set_cost(r, *c)
+            tile = b.autotune(0, ns, z, dt)
+            assert tile[0] == rows and tile == ctx.get_tile(False)
+            stub.stub_reset()
+            b.run(0, ns, ns, z, dt)
+            assert [(r, t) for _, r, t in _launches(stub)] == [(rows, nt)]  # one window
+            assert ctx.get_tile(False) == (rows, tile[1], ns, 0)
+            ctx.set_tile(8, 2, 1, protons=0)
+            stub.stub_reset()
+            b.run(0, ns, ns, z, dt)
+            assert [r for _, r, _ in _launches(stub)] == [8] * ns  # as set
+        finally:
+            b.close()
+            ctx.close()
+    ctx = ch.Context(n, ch.default_params())
+    try:
+        ctx.autotune(False, 64)
+        b = ch.Batch(ctx, nt, ch.SPECIES_ELECTRON, ns)
+        for s in range(ns):
+            b.set_background(s, np.ones((8, nt)))
+        b.set_state(None, np.ones(nt * n))
+        stub.stub_reset()
+        b.run(0, ns, ns, z, dt)
+        b.close()
+        assert len(_launches(stub)) == 1
     finally:
         ctx.close()
