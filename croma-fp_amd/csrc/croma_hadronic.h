@@ -1,14 +1,16 @@
 /*
- * croma_hadronic.h -- the emission and secondary-source kernels' physics,
- * compiled both by the host C runtime (gcc, -ffp-contract=off) and by the
- * device tables (hipcc, contraction off inside every function), so the host
- * and device tables follow one arithmetic:
+ * croma_hadronic.h -- the hadronic emission and secondary-source kernels'
+ * physics, compiled both by the host C runtime (gcc, -ffp-contract=off) and by
+ * the device tables (hipcc, contraction off inside every function), so the
+ * host and device tables follow one arithmetic:
  *   pp cross section (Kamae 2006 fit, Blattnig 2000 charged ratios)  HADRONIC.c:342-431
  *   pion spectra, muon decay, Qe kernel                             HADRONIC.c:433-533
  *   gamma kernel                                                    HADRONIC.c:139-174
  *   electron / muon neutrino kernels                                HADRONIC.c:179-322
  *   IC scattering kernel, CMB photon density                        FP_Coef.c:378-405
- *   IC emissivity kernel (N = 400 trapezoid)                        FP_Coef.c:553-582
+ * The last line is the host's (exact IC cooling rates); the device's IC cooling
+ * rows and emissivity table write these two functions for their own lanes
+ * (croma_ic.hip, k_ic_table in croma_tables.hip).
  */
 #ifndef CROMA_HADRONIC_H
 #define CROMA_HADRONIC_H
@@ -286,31 +288,6 @@ CHK_FN double chk_nu_kernel(double E, double p)
 {
     CHK_NOCONTRACT
     return chk_ekernel(2, E, p) + chk_ekernel(1, E, p) + chk_numu1(E, p);
-}
-
-CHK_FN double chk_ic_emissivity_kernel(double nu, double gamma, double z)
-{
-    CHK_NOCONTRACT
-    const int N = 400;
-    const double meg = 9.11e-28, c = 3.0e+10;
-    const double eps = CHK_H * nu / (meg * c * c);
-    double e0max = eps, e0min = eps / (4.0 * gamma * (gamma - eps)), a, da, Cn, nn, e0n, sum = 0.0;
-    int i;
-    if (e0min < 0) e0min = eps / (gamma * gamma);
-    da = (log10(e0max) - log10(e0min)) / (double)N;
-    a = log10(e0min);
-    e0n = pow(10.0, a);
-    Cn = chk_ic_kernel(e0n, gamma, eps);
-    nn = chk_cmb_n(e0n, z);
-    for (i = 0; i < N; i++) {
-        const double e0 = e0n, C = Cn, n0 = nn;
-        a = a + da;
-        e0n = pow(10.0, a);
-        nn = chk_cmb_n(e0n, z);
-        Cn = chk_ic_kernel(e0n, gamma, eps);
-        sum = sum + 0.5 * (C * n0 + Cn * nn) * (e0n - e0);
-    }
-    return CHK_H * eps * sum / (4.0 * CHK_PI);
 }
 
 #endif

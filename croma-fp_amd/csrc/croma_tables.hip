@@ -1,6 +1,7 @@
-// Grid-constant kernel tables built on the device from the shared physics
-// header (croma_hadronic.h), one table entry per thread (the IC table eight
-// lanes per entry):
+// Grid-constant kernel tables built on the device: the secondary weights and
+// the gamma and neutrino rows from the shared physics header
+// (croma_hadronic.h), one table entry per thread; the IC rows from this file's
+// own form of the integrand (k_ic_table), eight lanes per entry:
 //   secondary-electron weights fqe_t[jp][je]   fp_shared_core.c:1453-1506 (QeKernel_BB05, HADRONIC.c:436-498)
 //   gamma / neutrino / IC kernel tables [k][j]  fp_shared_core.c:1724-1804 (prepare_*_kernel_flat),
 //                                              HADRONIC.c:139-289, FP_Coef.c:553-582
@@ -60,10 +61,9 @@ __global__ void __launch_bounds__(kTabBlock) k_fqe_weights(int n, const double *
 // out[k][j] for k < nbins on the accumulated log grid a_k = lo + (k+1) d - d
 // summed term by term as the reference's loops do (so a_k is bit-identical
 // to theirs, fp_shared_core.c:1735-1741); kind 0 gamma(E_k, p_j), 1 neutrino(E_k, p_j).
-__global__ void __launch_bounds__(kTabBlock) k_emis_table(int kind, int n, int nbins, double lo, double d, double z,
+__global__ void __launch_bounds__(kTabBlock) k_emis_table(int kind, int n, int nbins, double lo, double d,
                                                            const double *__restrict__ mom, double *out)
 {
-    (void)z;
     const int j = blockIdx.x * kTabBlock + threadIdx.x;
     const int k = blockIdx.y;
     if (j >= n || k >= nbins) return;
@@ -77,15 +77,16 @@ __global__ void __launch_bounds__(kTabBlock) k_emis_table(int kind, int n, int n
     out[(size_t)k * n + j] = v;
 }
 
-// Inverse-Compton emissivity table: out[k][j] = chk_ic_emissivity_kernel(nu_k,
-// sqrt(1 + p_j^2), z), the 400-node quadrature of FP_Coef.c:553-582, a table
+// Inverse-Compton emissivity table: out[k][j], the emissivity at nu_k of an
+// electron of gamma = sqrt(1 + p_j^2) in the CMB at z, by the 400-node
+// trapezoid rule over log10 of the photon energy (FP_Coef.c:553-582), a table
 // per snapshot's redshift.  Bound: FP64 VALU (a pow, a log and an exp per
 // node).  One thread per entry left one wave per CU with 400 nodes in a row
 // (635 us for 64 x 256 entries); here eight lanes share an entry, 50 nodes
 // each, leave their trapezoid terms in LDS and the first of them adds the 400
 // terms in the serial order (238 us, the same bits).  The integrand's squares
-// are products and its constants are formed once, where the shared header's
-// pow calls took half of the 720 instructions of a node (148 us).
+// are products and its constants are formed once, where pow calls took half of
+// the 720 instructions of a node (148 us).
 __device__ __forceinline__ double ict_kernel(double eps0, double gamma, double eps)
 {
 #pragma clang fp contract(off)
@@ -175,6 +176,6 @@ extern "C" int ck_emission_kernel_table(int kind, int n, int nbins, double lo, d
         return hipGetLastError() != hipSuccess;
     }
     hipLaunchKernelGGL(k_emis_table, dim3(gx, (unsigned)nbins), dim3(kTabBlock), 0, (hipStream_t)stream, kind, n,
-                       nbins, lo, (hi - lo) / (double)nbins, z, mom, out);
+                       nbins, lo, (hi - lo) / (double)nbins, mom, out);
     return hipGetLastError() != hipSuccess;
 }

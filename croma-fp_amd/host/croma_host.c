@@ -1935,7 +1935,8 @@ int croma_hip_batch_run(CromaHipBatch *b, int s0, int s1, int nsnap_total, const
     if (ck_event_record(b->ev_a, c->stream)) return dev_fail("event");
     if (dev_nsub && ck_fill_i32((int *)b->d_cells, 0, 2, c->stream)) return dev_fail("cell counter");
     if ((rc = run_ic_rows(b, s0, s1, nsnap_total, z)) != 0) return rc;
-    /* the first window's, and in its shadow the others': a run's redshifts at once */
+    /* the IC end rates of the run's redshifts side by side on the host threads,
+     * before the first window asks for its own */
     if (s1 - s0 > 1 && dev_nsub) {
         double *ends = (double *)malloc((size_t)(s1 - s0) * 2 * sizeof(double));
         const double t0 = ch_now_s();

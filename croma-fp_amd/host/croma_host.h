@@ -37,9 +37,7 @@ int ch_choose_segments(const CkParams *prm, int nsub, int allow);
 int ch_ic_cooling_row(const ChGrid *g, double z, double *row, double *m1, double *p1);
 /* CMB photon-energy bounds of the IC integral at z (FP_Coef.c:413-436). */
 void ch_ic_bounds(double z, double *e0min, double *e0max);
-/* IC cooling rate of the electron bins bins[0..count) at z (same arithmetic
- * as ch_ic_cooling_row, which fills every bin). */
-int ch_ic_cooling_bins(const ChGrid *g, double z, int count, const int *bins, double *out);
+/* IC cooling rates at the first and last electron bin at nz redshifts. */
 void ch_ic_cooling_ends(const ChGrid *g, int nz, const double *z, double *out);
 
 /* croma_host.c */

@@ -425,39 +425,6 @@ void ch_ic_bounds(double z, double *e0min, double *e0max) { ch_cmb_bounds(z, e0m
 
 typedef struct {
     const ChGrid *g;
-    double z, lo, hi;
-    const int *bins;
-    double *out;
-} ChIcBinsJob;
-
-static void ch_ic_bins_range(void *arg, long i0, long i1)
-{
-    ChIcBinsJob *J = (ChIcBinsJob *)arg;
-    long i;
-    for (i = i0; i < i1; i++) {
-        const double p = J->g->ep[J->bins[i]];
-        J->out[i] = ch_b_ic(sqrt(1.0 + p * p), J->lo, J->hi, J->z);
-    }
-}
-
-int ch_ic_cooling_bins(const ChGrid *g, double z, int count, const int *bins, double *out)
-{
-    ChIcBinsJob J;
-    int i;
-    if (!g || count < 0 || !bins || !out) return -1;
-    for (i = 0; i < count; i++)
-        if (bins[i] < 0 || bins[i] >= g->n) return -1;
-    J.g = g;
-    J.z = z;
-    J.bins = bins;
-    J.out = out;
-    ch_cmb_bounds(z, &J.lo, &J.hi);
-    ch_parallel_for(count, 1, ch_ic_bins_range, &J);
-    return 0;
-}
-
-typedef struct {
-    const ChGrid *g;
     const double *z;
     double *out;
 } ChIcEndsJob;
@@ -475,7 +442,8 @@ static void ch_ic_ends_range(void *arg, long i0, long i1)
 }
 
 /* IC cooling rates of the electron grid's first and last bins, out[2 q],
- * out[2 q + 1], at z[q], q < nz. */
+ * out[2 q + 1], at z[q], q < nz (same arithmetic as ch_ic_cooling_row, which
+ * fills every bin). */
 void ch_ic_cooling_ends(const ChGrid *g, int nz, const double *z, double *out)
 {
     ChIcEndsJob J;

@@ -75,13 +75,13 @@ def test_host_grid_and_ic_end_bins_match_reference(lib, n):
     assert lib.ch_grid_build(C.byref(g), n, pmin, pmax, pemin, pemax) == 0
     for key in ("pp", "pdp", "pE", "ep", "edp", "eE"):
         assert np.array_equal(np.ctypeslib.as_array(getattr(g, key))[:n], d[key]), key
-    bins = (C.c_int * 2)(0, n - 1)
-    out = (C.c_double * 2)()
-    lib.ch_ic_cooling_bins.argtypes = [C.c_void_p, C.c_double, C.c_int, C.POINTER(C.c_int),
-                                       C.POINTER(C.c_double)]
-    for iz, z in enumerate(d["ic_z"]):
-        assert lib.ch_ic_cooling_bins(C.byref(g), C.c_double(z), 2, bins, out) == 0
-        assert out[0] == d["ic_rows"][iz][0] and out[1] == d["ic_rows"][iz][n - 1]
+    z = np.ascontiguousarray(d["ic_z"], np.float64)
+    out = np.zeros((len(z), 2))
+    dp = C.POINTER(C.c_double)
+    lib.ch_ic_cooling_ends.argtypes = [C.c_void_p, C.c_int, dp, dp]
+    lib.ch_ic_cooling_ends.restype = None
+    lib.ch_ic_cooling_ends(C.byref(g), len(z), z.ctypes.data_as(dp), out.ctypes.data_as(dp))
+    assert np.array_equal(out, d["ic_rows"][:, [0, n - 1]])
 
 
 def test_host_nsub_matches_oracle(lib):
