@@ -518,11 +518,13 @@ __device__ __forceinline__ double wave_dn1(double v) { return dpp64<0x130>(v); }
 // multiplier); or HS = 2, seven broadcasts that do not wait for each other
 // (11 instructions, seven multipliers, a third less latency), for up to 4 rows
 // per lane, where the chain through the scans is what a substep waits for.
-// With this, the overlap below and the wave priorities of k_fused_body: 256
-// electrons x 64 bins, 10 snapshots, 2.72 -> 2.51 ms (a launch waits for its
-// longest chain); 10,000 of both species x 256 bins 17.6 -> 16.9 ms; 65,536 x
-// 512 bins 153.7 -> 152.1 ms (8% fewer vector instructions, but the FP64
-// operations, which stay, hold the clock at 2.13 GHz).
+// With this and the overlap below: 256 electrons x 64 bins, 10 snapshots, 2.72
+// -> 2.51 ms (a launch waits for its longest chain); 10,000 of both species x
+// 256 bins 17.6 -> 16.9 ms; 65,536 x 512 bins 153.7 -> 152.1 ms (8% fewer
+// vector instructions, but the FP64 operations, which stay, hold the clock at
+// 2.13 GHz).  Measured together with wave priorities by task cost, which alone
+// turned out to cost (1,024 x 128 1.5%, served chunks 1.5%, others -0.7 to
+// 1.6%) and are gone.
 template <int R, int G>
 struct Factor {
     static constexpr bool ROW = G >= 16;           // the group covers whole 16-lane rows
@@ -1750,12 +1752,6 @@ __device__ __forceinline__ void k_fused_body(const CkGrid &g, const CkSlot *__re
         // zero, so every lane must hold finite values of a real tracer, not
         // registers that were never written in this launch
         const bool idle = tid >= ntasks;
-        // the costliest tasks (taken first) issue ahead of the wave they share
-        // a SIMD with: the launch ends with the longest of them
-        if (tbase < ntasks / 8) __builtin_amdgcn_s_setprio(3);
-        else if (tbase < ntasks / 4) __builtin_amdgcn_s_setprio(2);
-        else if (tbase < ntasks / 2) __builtin_amdgcn_s_setprio(1);
-        else __builtin_amdgcn_s_setprio(0);
         {
             const CkTask task = tasks[idle ? tbase : tid];
             const CkSlot &S0 = slots[task.slot];
