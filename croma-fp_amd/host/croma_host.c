@@ -1864,7 +1864,15 @@ static int reserve_segrows(CromaHipBatch *b, long need)
     need = (need + q - 1) / q * q;
     if (need > b->segrows_cap) {
         const size_t cnt = (size_t)need * c->g.n;
+        int k;
         ck_stream_sync(c->stream);
+        /* graphs hold both addresses, their keys one: none outlives the rows */
+        for (k = 0; k < 2; k++) {
+            graph_reset(c, &b->win[k].graph);
+            graph_reset(c, &b->win[k].graph_g);
+            graph_reset(c, &b->win[k].graph_e);
+        }
+        if (b == c->xb) graph_reset(c, &c->x_graph);
         ck_free(b->d_segrec);
         ck_free(b->d_seginje);
         b->d_segrec = (double *)ck_malloc(cnt * sizeof(double));

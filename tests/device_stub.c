@@ -4,7 +4,9 @@
  * are immediate, events are always complete, kernels compute nothing and are
  * recorded.  A stream or event belongs to the device current at its creation;
  * recording an event on another device's stream, and a launch on a stream of
- * a device that is not current, fail as they do in the HIP runtime. */
+ * a device that is not current, fail as they do in the HIP runtime.  So does
+ * the replay of a graph whose contraction writes to memory since freed, which
+ * on a device would be a write out of range. */
 #include "croma_kernels.h"
 
 #include <pthread.h>
@@ -19,10 +21,16 @@ typedef struct {
     double at; /* events: the clock when recorded */
 } Obj;
 
-typedef struct {
+typedef struct Head {
     size_t bytes;
-    int dev;
+    int dev, fixed, serial;
+    struct Head *next;
 } Head; /* before every device allocation */
+
+typedef struct {
+    const void *inje; /* what the captured contraction writes, */
+    int serial;       /* and the allocation it lay in */
+} Graph;
 
 static pthread_mutex_t mu = PTHREAD_MUTEX_INITIALIZER;
 static __thread int cur;
@@ -30,6 +38,13 @@ static char err[128] = "stub";
 static size_t live, peak, limit = (size_t)1 << 40, free_mem = (size_t)1 << 38;
 static int log_mode[STUB_LOG], log_rows[STUB_LOG], log_tasks[STUB_LOG], nlog;
 static int dev_streams[8], dev_events[8], dev_allocs[8];
+static Head *allocs;
+static char fixed_mem[16 << 20];
+static size_t fixed_next;
+static int fixed_used;
+static __thread int capturing;
+static __thread const void *captured;
+static int nalloc;
 static void (*hook_host_alloc)(void);
 /* the clock advances with each fused launch of tasks over k snapshots at r
  * rows per lane by launch_ms[r] + k slot_ms[r] */
@@ -57,6 +72,9 @@ void stub_set_cost(int r, double launch, double slot)
     launch_ms[r] = launch;
     slot_ms[r] = slot;
 }
+/* the next device allocation of this size takes the one fixed address, if that
+ * is free */
+void stub_fix_next(size_t bytes) { fixed_next = bytes; }
 void stub_set_host_alloc_hook(void (*f)(void)) { hook_host_alloc = f; }
 size_t stub_peak(void) { return peak; }
 size_t stub_live(void) { return live; }
@@ -101,13 +119,19 @@ int ck_mem_info(size_t *f, size_t *t)
 void *ck_malloc(size_t bytes)
 {
     Head *h;
-    if (bytes > limit || !(h = (Head *)calloc(1, 256 + bytes))) {
+    const int fix = fixed_next == bytes && !fixed_used && 256 + bytes <= sizeof(fixed_mem);
+    if (bytes > limit || !(h = fix ? (Head *)fixed_mem : (Head *)calloc(1, 256 + bytes))) {
         fail("out of memory");
         return 0;
     }
+    if (fix) memset(h, 0, 256 + bytes), fixed_next = 0, fixed_used = 1;
     h->bytes = bytes;
     h->dev = cur;
+    h->fixed = fix;
     pthread_mutex_lock(&mu);
+    h->serial = ++nalloc;
+    h->next = allocs;
+    allocs = h;
     live += bytes;
     if (live > peak) peak = live;
     dev_allocs[cur]++;
@@ -116,11 +140,15 @@ void *ck_malloc(size_t bytes)
 }
 int ck_free(void *p)
 {
+    Head *h = (Head *)((char *)p - 256), **q;
     if (!p) return 0;
     pthread_mutex_lock(&mu);
-    live -= ((Head *)((char *)p - 256))->bytes;
+    live -= h->bytes;
+    for (q = &allocs; *q != h; q = &(*q)->next) {}
+    *q = h->next;
     pthread_mutex_unlock(&mu);
-    free((char *)p - 256);
+    if (h->fixed) fixed_used = 0;
+    else free(h);
     return 0;
 }
 void *ck_host_alloc(size_t bytes)
@@ -173,9 +201,32 @@ int ck_h2d(void *dst, const void *src, size_t bytes, void *s)
 int ck_d2h(void *dst, const void *src, size_t bytes, void *s) { return ck_h2d(dst, src, bytes, s); }
 int ck_d2d(void *dst, const void *src, size_t bytes, void *s) { return ck_h2d(dst, src, bytes, s); }
 int ck_device_sync(void) { return 0; }
-int ck_graph_begin(void *s) { return s ? 0 : -1; }
-void *ck_graph_end(void *s) { return s ? calloc(1, 8) : 0; }
-int ck_graph_launch(void *g, void *s) { return g && s ? 0 : -1; }
+static int serial_at(const void *p)
+{
+    Head *h;
+    pthread_mutex_lock(&mu);
+    for (h = allocs; h && (char *)h + 256 != (const char *)p; h = h->next) {}
+    pthread_mutex_unlock(&mu);
+    return h ? h->serial : 0;
+}
+int ck_graph_begin(void *s)
+{
+    capturing = 1;
+    captured = 0;
+    return s ? 0 : -1;
+}
+void *ck_graph_end(void *s)
+{
+    Graph *g = (Graph *)calloc(1, sizeof(*g));
+    g->inje = captured;
+    g->serial = serial_at(captured);
+    capturing = 0;
+    return s ? g : 0;
+}
+int ck_graph_launch(void *g, void *s)
+{
+    return !s || serial_at(((Graph *)g)->inje) != ((Graph *)g)->serial ? fail("graph writes to freed memory") : 0;
+}
 int ck_graph_destroy(void *g)
 {
     free(g);
@@ -244,7 +295,8 @@ int ck_nsub_order(CkGrid g, const CkSlot *slots, int count, int ntr, int protons
 int ck_sec_contract(int n, const double *a, const int *b, const double *c, double *d, long e, const int *f, int g,
                     void *s)
 {
-    (void)n, (void)a, (void)b, (void)c, (void)d, (void)e, (void)f, (void)g;
+    (void)n, (void)a, (void)b, (void)c, (void)e, (void)f, (void)g;
+    if (capturing) captured = d;
     return on_current(s);
 }
 int ck_ic_rows(int n, const double *a, double b, double c, int d, const double *e, double *f, double *g, int *h, void *s)

@@ -34,6 +34,7 @@ def stub(stub_path, monkeypatch):
     L = ch.lib()
     L.stub_peak.restype = L.stub_live.restype = C.c_size_t
     L.stub_set_limit.argtypes = [C.c_size_t, C.c_size_t]
+    L.stub_fix_next.argtypes = [C.c_size_t]
     L.stub_set_cost.argtypes = [C.c_int, C.c_double, C.c_double]
     L.stub_set_host_alloc_hook.argtypes = [C.c_void_p]
     L.ck_set_device(0)
@@ -325,5 +326,50 @@ def test_tuned_runs_keep_the_windows_by_size(stub):
         b.run(0, ns, ns, z, dt)
         b.close()
         assert len(_launches(stub)) == 1
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("pipelined", [False, True])
+def test_graphs_do_not_outlive_the_segment_rows(stub, pipelined):
+    """Growing the segment rows replaces both arrays; a window whose launch key
+    repeats (the first array back at its old address, the same row count) must
+    not replay a graph that writes to the second one's old address."""
+    n, nt, ns = 64, 40, 6
+    z, dt = np.linspace(0.06, 0.0, ns + 1), np.full(ns, 0.01)
+    ctx = ch.Context(n, ch.default_params(coeff_interp_max_segments=1))
+    ctx.set_nsub_device(False)
+    ctx.set_pipeline(pipelined)
+    b = ch.Batch(ctx, nt, ch.SPECIES_ELECTRON_PROTON, ns)
+    try:
+        for s in range(ns):
+            b.set_background(s, np.ones((8, nt)))
+        b.set_state(np.ones(nt * n), np.ones(nt * n))
+        stub.stub_fix_next(256 * n * 8)  # rows in steps of 256
+        assert b.run(0, ns, ns, z, dt).graph_launches > 0
+        # more segments allowed, none taken: the same row counts
+        ctx.set_params(ch.default_params(coeff_interp_max_segments=64, coeff_interp_min_steps=1 << 20))
+        stub.stub_fix_next(nt * 64 * n * 8)
+        b.run(0, ns, ns, z, dt)
+    finally:
+        b.close()
+        ctx.close()
+
+
+def test_drop_in_graph_does_not_outlive_its_batch(stub):
+    """A call of another shape that fails after the old batch is gone leaves no
+    graph of that batch for the next call of the old shape."""
+    n, nt = 64, 40
+    ctx = ch.Context(n, ch.default_params())
+    try:
+        for failing in (True, False):
+            stub.stub_fix_next(256 * n * 8)
+            for _ in range(4):  # eager, captured, replayed
+                _snapshot(ctx, nt, np.full(nt, 4))
+            if failing:
+                stub.stub_set_limit(1 << 10, 1 << 38)
+                with pytest.raises(ch.CromaHipError):
+                    _snapshot(ctx, 2 * nt, np.full(2 * nt, 4))
+                stub.stub_set_limit(1 << 40, 1 << 38)
     finally:
         ctx.close()
