@@ -717,7 +717,11 @@ __device__ __forceinline__ double d_exp_nonpos(double x)
 // correction squares the quotient's): the division sequence without the
 // operand scaling and fix-up for denormal, infinite or zero divisors, which
 // the build's divisors (face diffusion averages above 1e-200, Bernoulli
-// denominators in (0, 1], pivots above 1e-300 in magnitude) never are.
+// denominators in (0, 1], pivots above 1e-300 in magnitude, and pivot_in's
+// renormalised v of a diagonally dominant system) never are.  The batched
+// solve, whose systems are the caller's, uses pivot_in's quotient only as a
+// first guess and repeats its rounds until none is left: there any value will
+// do, also from a zero, infinite or NaN divisor.
 // Within an ulp of the IEEE quotient.
 __device__ __forceinline__ double d_div_normal(double a, double b)
 {

@@ -16,7 +16,8 @@
 // looks for its own number, so nothing clears the word between calls: a call
 // is one kernel and one 4-byte download (31.2 -> 28.7 us at 64 x 64 rows).
 // Calls that overlap on one GPU (two host threads, or two streams) share the
-// array and race.
+// array and race: in c', and in the word, where of two failing calls the later
+// writer's number stands and the other call reports success.
 #include <hip/hip_runtime.h>
 
 #include <pthread.h>

@@ -294,8 +294,10 @@ int croma_hip_solve_cc_batch(int nsys, int nrow, double dt, const double *a, con
  * pivot-failure word) is a static device array of the library, one per GPU,
  * held until the process ends: nsys * nrow may not exceed
  * CROMA_HIP_NOALLOC_MAX_CELLS (32 MiB of c'), else CROMA_HIP_EINVAL.  Calls
- * that overlap on one GPU share that array and race.  Returns 0,
- * CROMA_HIP_EPIVOT, CROMA_HIP_EINVAL or CROMA_HIP_EDEVICE. */
+ * that overlap on one GPU share that array and race: systems of more than
+ * 1,024 rows come out wrong, and of two failing calls one may return 0 (the
+ * other's number stands in the word).  Returns 0, CROMA_HIP_EPIVOT,
+ * CROMA_HIP_EINVAL or CROMA_HIP_EDEVICE. */
 #define CROMA_HIP_NOALLOC_MAX_CELLS (4 * 1024 * 1024)
 int croma_hip_solve_cc_batch_noalloc(int nsys, int nrow, double dt, const double *a, const double *b,
                                      const double *c, const double *source, const double *state_init,

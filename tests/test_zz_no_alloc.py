@@ -2,8 +2,9 @@
 against the allocating entry point (croma_hip_solve_cc_batch) on the same
 systems: bit-identical states on two calls in a row, the second smaller than
 the first, plus the oracle's Thomas sweep (fp_shared_core.c:226-257) on a
-sample of systems within 1e-12, the size limit and the pivot-failure word
-being cleared between calls.  The caller's device arrays come from the HIP
+sample of systems within 1e-12, the size limit, and a call after one whose
+pivot vanished (the failing call's number stays in the failure word; the next
+call looks for its own).  The caller's device arrays come from the HIP
 runtime the library itself links (hipMalloc / hipMemcpy through ctypes)."""
 import ctypes as C
 
@@ -104,6 +105,6 @@ def test_noalloc_limits_and_pivot_word():
     b_bad[5, 0] = 0.0
     with pytest.raises(ch.CromaHipError):
         _noalloc(a, b_bad, c, q, x, 0.1)
-    # ... and the failure word starts at zero again on the next call
+    # ... and the next call does not take that failure for its own
     ref, _ = ch.solve_cc_batch(a, b, c, q, x, 0.1)
     assert np.array_equal(_noalloc(a, b, c, q, x, 0.1), ref)
